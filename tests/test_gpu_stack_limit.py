@@ -150,3 +150,38 @@ def test_chain_beyond_the_limit_reports_overflow_and_recovers():
         assert np.all(hits["prim_id"] == 100)
         img = r.render(hs_ok.camera(), 1, 4)
         assert np.all(np.isfinite(img))
+
+
+@pytest.mark.parametrize("lds_stack", [1, 2, 16, 17, 128])
+@pytest.mark.parametrize("depth", [1, 15, 16, 17, 63, 128])
+def test_chain_at_the_edges_of_the_lds_part(depth, lds_stack):
+    """Chains whose deepest stack is one entry, around the LDS part's last
+    slot and at the limit (depth 128), with LDS
+    parts of one entry up to all of them, in ray batches and in a render: the
+    bottom triangle is found and a ray from the other side is occluded, and
+    the image equals the one with the default LDS part."""
+    from xenon_amd import HipRenderer
+    hs, flat, keep = _chain_scene(depth)
+    images = []
+    for lds in (lds_stack, 0):
+        with HipRenderer(8, 8, 4, 3, spp_per_launch=4, lds_stack=lds) as r:
+            _upload(r, flat)
+            print(f"[stack] chain depth {depth}, LDS part {lds or 16}", flush=True)
+            hits = r.trace_closest(_rays(130, (-1.0, 0.1, 0.2), (1.0, 0.0, 0.0), np.inf))
+            assert np.all(hits["prim_id"] == depth)
+            assert np.all(r.trace_any(_rays(130, (12.0, 0.1, 0.2), (-1.0, 0.0, 0.0), 100.0)) == 1)
+            images.append(r.render(hs.camera(8, 8), 1, 4))
+    assert np.array_equal(images[0].view(np.uint32), images[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("lds_stack", [1, 16, 128])
+def test_one_entry_past_the_limit_is_refused(lds_stack):
+    from xenon_amd import HipRenderer, native as N
+    hs, flat, keep = _chain_scene(129)
+    with HipRenderer(8, 8, 4, 3, spp_per_launch=4, lds_stack=lds_stack) as r:
+        _upload(r, flat)
+        print(f"[stack] chain depth 129, LDS part {lds_stack}", flush=True)
+        with pytest.raises(N.XnhError) as e:
+            r.trace_closest(_rays(130, (-1.0, 0.1, 0.2), (1.0, 0.0, 0.0), np.inf))
+        assert e.value.code == OVERFLOW
+        assert r.stats()["stack_overflows"] == 130

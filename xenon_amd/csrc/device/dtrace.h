@@ -20,10 +20,12 @@
 // 15 = a leaf of 15 or more: low bits = its first slot, whose bigcnt word
 // holds the count). Node and slot indices are < 2^28.
 //
-// Stack: the top `lds_depth` entries of each lane live in LDS, laid out
-// entry-major ([entry][lane]) so lanes at equal depth hit distinct banks;
-// deeper entries spill, in order, to a per-lane HBM region. The BLAS walk of
-// an instance runs on top of the TLAS entries, so both share kMaxStack.
+// Stack: the entry on top is held in a register (TravStack::tos). Of those
+// below it the deepest `lds_depth` live in LDS, laid out entry-major
+// ([entry][lane]) so lanes at equal depth hit distinct banks; the others
+// spill, in order, to a per-lane HBM region. The BLAS walk of an instance
+// runs on top of the TLAS entries, so both share kMaxStack; a marker entry
+// (kEntEnd) under each BLAS walk ends it when it is popped.
 #pragma once
 #include "../common/dev_types.h"
 #include "dmath.h"
@@ -33,36 +35,70 @@ namespace xnh {
 // The kernels' dynamic LDS: lds_depth x blockDim.x stack entries.
 extern __shared__ uint32_t trav_lds[];
 
+constexpr uint32_t kEntEnd = kNoRoot;            // no entry: the lane is not in a BLAS walk
+constexpr uint32_t kStackBottom = 0xFFFFFFFEu;   // the top of an empty stack (equals no entry)
+
 struct TravStack {
-  int lds_col;          // this lane's column: trav_lds[e * lds_stride + lds_col]
-  int lds_off;          // sp * lds_stride + lds_col (kept as a running index)
-  uint32_t* spill;      // this lane's spill column: spill[(e - lds_depth) * spill_stride]
-  int lds_stride, spill_stride, lds_depth, sp;   // lds_depth >= 1
+  // LDS slots are byte addresses: an LDS pointer is 32 bits, and the walk
+  // steps and compares them. They are signed: the row below a lane's first
+  // slot lies below address 0 in a kernel whose LDS holds nothing else.
+  typedef __attribute__((address_space(3))) uint32_t LdsWord;
+  uint32_t tos;         // the entry on top (kStackBottom: the stack is empty)
+  int32_t top;          // slot of the entry below it: bottom + row * (entries held)
+  int32_t bottom;       // one row below this lane's first slot
+  int32_t last;         // this lane's last slot (entries from lds_depth on are in the spill)
+  uint32_t* spill;      // this lane's spill column: entry e is spill[(e - lds_depth) * spill_stride]
+  int32_t row;          // bytes from one entry's slot to the next
+  int spill_stride, lds_depth;   // lds_depth >= 1
   bool overflow;
+  __device__ __forceinline__ void clear() {
+    tos = kStackBottom;
+    top = bottom;
+  }
   __device__ __forceinline__ void reset() {
-    sp = 0;
-    lds_off = lds_col;
+    clear();
     overflow = false;
   }
-  __device__ __forceinline__ void push(uint32_t v) {
-    if (sp >= kMaxStack) {
+  __device__ __forceinline__ bool empty() const { return tos == kStackBottom; }
+  __device__ __forceinline__ static LdsWord* word(int32_t slot) {
+    return (LdsWord*)static_cast<uint32_t>(slot);
+  }
+  // Entries held (rarely needed: the walk compares slots instead).
+  __device__ __forceinline__ int size() const { return static_cast<int>(static_cast<uint32_t>(top - bottom) / static_cast<uint32_t>(row)); }
+  // The entry below the top, for a pop. The LDS read is issued for every
+  // lane, at its last slot when the entry is in the spill, so that the walk
+  // can issue it with its node loads; in_spill() lanes replace the value.
+  __device__ __forceinline__ uint32_t below() const { return *word(min(top, last)); }
+  __device__ __forceinline__ bool in_spill() const { return top > last; }
+  __device__ __forceinline__ uint32_t spilled() const {
+    return gld1(spill, static_cast<size_t>(size() - 1 - lds_depth) * static_cast<size_t>(spill_stride));
+  }
+  // Stores v, the former top, in the spill slot the stack has just grown
+  // into (top was advanced). False past `limit` entries.
+  __device__ __forceinline__ bool keep_spilled(uint32_t v, int limit) {
+    const int n = size();
+    if (n > limit) return false;
+    gst1(spill, static_cast<size_t>(n - 1 - lds_depth) * static_cast<size_t>(spill_stride), v);
+    return true;
+  }
+  // Entries beyond kMaxStack are not stored: the flag ends the ray. The
+  // marker under a BLAS walk takes a place of its own (`extra`).
+  __device__ __forceinline__ void push(uint32_t v, int extra = 0) {
+    top += row;
+    if (top <= last) {
+      *word(top) = tos;
+    } else if (!keep_spilled(tos, kMaxStack + extra)) {
+      top -= row;
       overflow = true;
       return;
     }
-    if (sp < lds_depth) trav_lds[lds_off] = v;
-    else gst1(spill, static_cast<size_t>(sp - lds_depth) * spill_stride, v);
-    ++sp;
-    lds_off += lds_stride;
+    tos = v;
   }
-  // The LDS read is issued unconditionally (at this lane's entry 0 when the
-  // entry lies in the spill) so that the common case compiles to a plain
-  // LDS access rather than a generic-address load.
   __device__ __forceinline__ uint32_t pop() {
-    --sp;
-    lds_off -= lds_stride;
-    const bool in_lds = sp < lds_depth;
-    uint32_t v = trav_lds[in_lds ? lds_off : lds_col];
-    if (!in_lds) v = gld1(spill, static_cast<size_t>(sp - lds_depth) * spill_stride);
+    const uint32_t v = tos;
+    tos = below();
+    if (in_spill()) tos = spilled();
+    top -= row;
     return v;
   }
 };
@@ -77,9 +113,20 @@ struct TravCount {
   uint32_t int_iters, leaf_iters, leaf_steps, round_iters, round_lanes;
 };
 
+// The lanes where p holds (as a lane mask, without the detour over an
+// integer that HIP's __ballot takes), and how many.
+__device__ __forceinline__ unsigned long long ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+// (The empty asm keeps the count a 32-bit scalar; left to itself the compiler
+// compares two such counts as 64-bit values on the vector unit.)
+__device__ __forceinline__ int lanes_of(bool p) {
+  int n = __builtin_popcountll(__builtin_amdgcn_ballot_w64(p));
+  asm("" : "+s"(n));
+  return n;
+}
+
 // True on the lowest active lane of the wave.
 __device__ __forceinline__ bool first_active_lane() {
-  return static_cast<int>(threadIdx.x & 63u) == __ffsll(static_cast<long long>(__ballot(1))) - 1;
+  return static_cast<int>(threadIdx.x & 63u) == __ffsll(static_cast<long long>(ballot(1))) - 1;
 }
 
 struct HitRef {
@@ -88,28 +135,34 @@ struct HitRef {
   int32_t inst;    // instance index, -1 = none
 };
 
+struct TriRec {
+  float4 a, b, c;
+};
+__device__ __forceinline__ TriRec load_tri(const float4* __restrict__ tris, uint32_t slot) {
+  const size_t k = 3 * static_cast<size_t>(slot);
+  return TriRec{gld4(tris, k), gld4(tris, k + 1), gld4(tris, k + 2)};
+}
+
 // Moller-Trumbore on a pre-gathered triangle (geometry/primitives.h:25-49).
-__device__ __forceinline__ bool tri_test(const float4* __restrict__ tris, uint32_t slot, f3 o, f3 d, float tmin,
-                                         float tmax, float& t, float& u, float& v) {
-  const float4 a = gld4(tris, 3 * slot), b = gld4(tris, 3 * slot + 1), c = gld4(tris, 3 * slot + 2);
-  const f3 v0{a.x, a.y, a.z}, e1{a.w, b.x, b.y}, e2{b.z, b.w, c.x};
+// The reference's early returns are one conjunction here: lanes of a wave
+// seldom fail together, so a branch per condition cost more than it skipped.
+__device__ __forceinline__ bool tri_test(const TriRec& r, f3 o, f3 d, float tmin, float tmax, float& t, float& u,
+                                         float& v) {
+  const f3 v0{r.a.x, r.a.y, r.a.z}, e1{r.a.w, r.b.x, r.b.y}, e2{r.b.z, r.b.w, r.c.x};
   const f3 h = cross(d, e2);
   const float det = dot(e1, h);
-  if (fabsf(det) < 1e-7f) return false;
   const float ia = 1.f / det;
   const f3 s = o - v0;
   u = ia * dot(s, h);
-  if (u < 0.f || u > 1.f) return false;
   const f3 q = cross(s, e1);
   v = ia * dot(d, q);
-  if (v < 0.f || u + v > 1.f) return false;
   t = ia * dot(e2, q);
-  return t >= tmin && t <= tmax;
+  return !(fabsf(det) < 1e-7f) & !(u < 0.f) & !(u > 1.f) & !(v < 0.f) & !(u + v > 1.f) & (t >= tmin) & (t <= tmax);
 }
 
-// Two-child slab test; returns the hit mask, near distances in tn0/tn1.
-__device__ __forceinline__ int pair_test(float4 la, float4 lb, float4 ra, float4 rb, f3 inv, f3 o, float tmin,
-                                         float tmax, float& tn0, float& tn1) {
+// Two-child slab test: hits in hl/hr, near distances in tn0/tn1.
+__device__ __forceinline__ void pair_test(float4 la, float4 lb, float4 ra, float4 rb, f3 inv, f3 o, float tmin,
+                                          float tmax, float& tn0, float& tn1, bool& hl, bool& hr) {
   const float lx0 = (la.x - o.x) * inv.x, lx1 = (la.w - o.x) * inv.x;
   const float ly0 = (la.y - o.y) * inv.y, ly1 = (lb.x - o.y) * inv.y;
   const float lz0 = (la.z - o.z) * inv.z, lz1 = (lb.y - o.z) * inv.z;
@@ -122,7 +175,8 @@ __device__ __forceinline__ int pair_test(float4 la, float4 lb, float4 ra, float4
   const float rf = xmin(xmin(xmin(xmax(rx0, rx1), xmax(ry0, ry1)), xmax(rz0, rz1)), tmax);
   tn0 = ln;
   tn1 = rn;
-  return (ln <= lf ? 1 : 0) | (rn <= rf ? 2 : 0);
+  hl = ln <= lf;
+  hr = rn <= rf;
 }
 
 // pair_test with the hardware min/max (v_min3/v_max3 chains instead of
@@ -131,8 +185,8 @@ __device__ __forceinline__ int pair_test(float4 la, float4 lb, float4 ra, float4
 // direction and inverse direction are finite in every component (box
 // coordinates are finite). Without NaNs the two differ at
 // most in the sign of a zero distance, which no comparison distinguishes.
-__device__ __forceinline__ int pair_test_fast(float4 la, float4 lb, float4 ra, float4 rb, f3 inv, f3 o, float tmin,
-                                              float tmax, float& tn0, float& tn1) {
+__device__ __forceinline__ void pair_test_fast(float4 la, float4 lb, float4 ra, float4 rb, f3 inv, f3 o, float tmin,
+                                               float tmax, float& tn0, float& tn1, bool& hl, bool& hr) {
   const float lx0 = (la.x - o.x) * inv.x, lx1 = (la.w - o.x) * inv.x;
   const float ly0 = (la.y - o.y) * inv.y, ly1 = (lb.x - o.y) * inv.y;
   const float lz0 = (la.z - o.z) * inv.z, lz1 = (lb.y - o.z) * inv.z;
@@ -145,7 +199,8 @@ __device__ __forceinline__ int pair_test_fast(float4 la, float4 lb, float4 ra, f
   const float rf = fminf(fminf(fminf(fmaxf(rx0, rx1), fmaxf(ry0, ry1)), fmaxf(rz0, rz1)), tmax);
   tn0 = ln;
   tn1 = rn;
-  return (ln <= lf ? 1 : 0) | (rn <= rf ? 2 : 0);
+  hl = ln <= lf;
+  hr = rn <= rf;
 }
 
 __device__ __forceinline__ bool all_finite(f3 v) {
@@ -370,15 +425,26 @@ __device__ __forceinline__ f3 prim_normal(const PrimRec& p, f3 o, f3 d, float tm
 // a persistent kernel can retire a finished ray and start the next in the
 // same lane while the rest of the wave keeps walking.
 //
-// A round runs the lane's TLAS steps until it enters a BLAS walk, then two
-// wave-wide phases over the lanes inside BLAS walks (the while-while loop of
-// Aila and Laine): an interior phase that walks node pairs, continuing with
-// the nearer hit child in registers and pushing only the farther, until the
-// lane reaches a leaf (held in a slot), and a leaf phase that tests the held
-// leaves, continuing through consecutive leaves. Each phase runs one kind
-// of step for all its lanes instead of both kinds every iteration.
+// A lane needs one of three kinds of step next: a TLAS step (no BLAS entry
+// at hand), an interior step (test a node's two children, continue with the
+// nearer hit one, push the farther) or a leaf step (test its triangles,
+// continue with the entry on top of the stack). wave_step runs one kind at a
+// time for the whole wave.
 //
-// No step is taken early: a lane holding a leaf walks no further interior
+// What bounds it: instruction issue in large launches, the latency of a
+// step's loads in small ones. The step loops therefore keep everything they
+// decide on in a few registers: the entry at hand alone names the kind of
+// step, the stack's top is a register and its slot a byte address, the entry
+// below it is read with the node (a pop waits for nothing), a marker under
+// each BLAS walk replaces the test for its end, and stack entries beyond the
+// LDS part are handled in a branch that a wave takes only when one of its
+// lanes needs it. Against a walk that held a reached leaf and its successor
+// apart and branched on push, pop and spill per lane (about 90 vector and 80
+// scalar instructions an interior step; 70 and 25 here): 1.3M-triangle mesh
+// 1920x1080x256 302.5 -> 267.2 ms, 4096 instances 389.6 -> 364.5 ms, Cornell
+// 512x512x64 15.1 -> 14.2 ms a pass.
+//
+// No step is taken early: a lane at a leaf walks no further interior
 // nodes until the leaf is tested, since a node box tested against a t_best
 // not yet lowered by the leaf's hits may let through a subtree the reference
 // culls, and box and triangle rounding differ enough for such a subtree to
@@ -394,10 +460,9 @@ __device__ __forceinline__ f3 prim_normal(const PrimRec& p, f3 o, f3 d, float tm
 // ignores tmax, as Scene::intersect does with a default HitRecord; any hit
 // uses [tmin, tmax]. A stack overflow ends the ray with what it has found.
 constexpr uint32_t kInstTag = 0x80000000u;
-constexpr uint32_t kEntEnd = kNoRoot;   // no entry left in the BLAS walk
 
-__device__ __forceinline__ bool ent_interior(uint32_t e) { return e != kEntEnd && (e >> kEntShift) == 0u; }
-__device__ __forceinline__ bool ent_leaf(uint32_t e) { return e != kEntEnd && (e >> kEntShift) != 0u; }
+__device__ __forceinline__ bool ent_interior(uint32_t e) { return e < (1u << kEntShift); }
+__device__ __forceinline__ bool ent_leaf(uint32_t e) { return e - (1u << kEntShift) < kEntEnd - (1u << kEntShift); }
 
 // kPrims: the scene may hold analytic primitives (a variant, because their
 // walk raises the register count of the whole kernel).
@@ -407,14 +472,16 @@ struct Walker {
   f3 lo, ld, linv;    // instance-space ray of the BLAS walk in progress
   float tmin, tbest;
   float rtmax;        // the ray's tmax (bounds the primitives' box tests, aabb.h:43)
-  int blas_base;      // stack depth under the current BLAS walk; -1 in the TLAS
   int inst;           // instance of the BLAS walk
-  uint32_t e;         // next BLAS entry to process, or kEntEnd; a leaf only while `leaf` is held
-  uint32_t leaf;      // held leaf entry (tested before e), 0 = none
-  bool inst_found, found;
+  uint32_t e;         // BLAS entry to process next (interior or leaf), kEntEnd outside a BLAS walk
+  bool occluded;      // any hit: an occluder was found
   bool fast;          // lo, ld, linv finite: pair_test_fast is exact
-  bool stuck;         // the step bound was reached (the walk was abandoned)
   HitRef hit;         // u, v, slot, inst of the closest hit; its t is tbest
+
+  __device__ __forceinline__ void idle(TravStack& st) {
+    e = kEntEnd;
+    st.reset();
+  }
 
   __device__ __forceinline__ void begin(const DevScene& S, f3 o_, f3 d_, float tmin_, float tmax_, TravStack& st) {
     o = o_;
@@ -423,28 +490,24 @@ struct Walker {
     tmin = tmin_;
     rtmax = tmax_;
     tbest = kAny ? tmax_ : __builtin_huge_valf();
-    blas_base = -1;
     inst = -1;
     e = kEntEnd;
-    leaf = 0u;
-    inst_found = false;
-    found = false;
+    occluded = false;
     fast = false;
-    stuck = false;
     hit = HitRef{0.f, 0.f, 0.f, 0u, -1};
     st.reset();
     if (S.num_tnodes > 0) st.push(0u);
   }
 
-  __device__ __forceinline__ void end_instance() {
-    if (!kAny && inst_found) {
-      hit.inst = inst;
-      found = true;
-    }
-    blas_base = -1;
-  }
+  __device__ __forceinline__ bool found() const { return kAny ? occluded : hit.inst >= 0; }
 
-  __device__ __forceinline__ uint32_t pop_blas(TravStack& st) { return st.sp > blas_base ? st.pop() : kEntEnd; }
+  // The walk is over: nothing on the stack, no BLAS entry at hand.
+  __device__ __forceinline__ bool finished(const TravStack& st) const { return e == kEntEnd && st.empty(); }
+
+  __device__ __forceinline__ void stop(TravStack& st) {
+    e = kEntEnd;
+    st.clear();
+  }
 
   // The scene's primitives, walked to the end at once in the instance-space
   // ray lo/ld (PrimBLAS::intersect / ::intersects, prim_blas.cpp:165-229):
@@ -452,9 +515,9 @@ struct Walker {
   // nearer last; true when an any-hit walk found an occluder.
   __device__ __forceinline__ bool prim_walk(const DevScene& S, TravStack& st, TravCount& c) {
     if (S.num_pnodes <= 0) return false;
-    const int base = st.sp;
+    const int32_t base = st.top;
     st.push(0u);
-    while (st.sp > base && !st.overflow) {
+    while (st.top > base && !st.overflow) {
       const uint32_t idx = st.pop();
       const float4 na = gld4(S.pnodes, 2 * static_cast<size_t>(idx)), nb = gld4(S.pnodes, 2 * static_cast<size_t>(idx) + 1);
       float tn;
@@ -469,12 +532,12 @@ struct Walker {
           float t;
           if (kCount) ++c.tri_tests;
           if (prim_hit(pr, lo, ld, tmin, kAny ? rtmax : tbest, t)) {
-            if (kAny) return true;   // the ray is finished; its stack is reset by the next begin()
+            if (kAny) return true;   // the ray is finished
             tbest = t;
             hit.u = 0.f;
             hit.v = 0.f;
             hit.slot = pi | kPrimHit;
-            inst_found = true;
+            hit.inst = inst;
           }
         }
         continue;
@@ -514,9 +577,8 @@ struct Walker {
 
   // One TLAS step: pops one TLAS entry, a node (tested on pop, its children
   // or instances pushed) or an instance to enter (its BLAS walk starts, or
-  // the primitives are walked to the end). True once the ray is finished.
-  __device__ __forceinline__ bool tlas_step(const DevScene& S, TravStack& st, TravCount& c) {
-    if (st.sp == 0) return true;
+  // the primitives are walked to the end). The stack is not empty.
+  __device__ __forceinline__ void tlas_step(const DevScene& S, TravStack& st, TravCount& c) {
     const uint32_t te = st.pop();
     if (te & kInstTag) {
       const int ii = static_cast<int>(te & ~kInstTag);
@@ -527,31 +589,18 @@ struct Walker {
       linv = f3{1.f / ld.x, 1.f / ld.y, 1.f / ld.z};
       fast = all_finite(linv) && all_finite(ld) && all_finite(lo);
       inst = ii;
-      inst_found = false;
       if (in.root == kPrimRoot) {   // the primitives: walked here, to the end
-        if (kPrims) {
-          if (prim_walk(S, st, c)) {
-            found = true;
-            return true;
-          }
-          if (!kAny && inst_found) {
-            hit.inst = ii;
-            found = true;
-          }
-          if (st.overflow) return true;
+        if (kPrims && prim_walk(S, st, c)) {
+          occluded = true;
+          stop(st);
         }
-        return false;
+      } else if (in.root != kNoRoot) {   // (kNoRoot: an empty mesh)
+        // the marker that ends the walk; at kMaxStack it is always taken
+        st.push(kEntEnd, 1);
+        e = in.root;
       }
-      blas_base = st.sp;
-      // e never holds a leaf unless one is already held: a root that is a
-      // leaf is held at once (kNoRoot, an empty mesh, is kEntEnd)
-      e = in.root;
-      leaf = 0u;
-      if (ent_leaf(e)) {
-        leaf = e;
-        e = kEntEnd;
-      }
-      return false;
+      if (st.overflow) stop(st);
+      return;
     }
     const uint32_t ni = te;
     const float4 na = gld4(S.tnodes, 3 * ni), nb = gld4(S.tnodes, 3 * ni + 1);
@@ -566,7 +615,7 @@ struct Walker {
     const float tzn = (bz0 - o.z) * inv.z, tzf = (bz1 - o.z) * inv.z;
     const float lo_t = smax(smax(smax(tmin, txn), tyn), tzn);
     const float hi_t = smin(smin(smin(tbest, txf), tyf), tzf);
-    if (!(lo_t <= hi_t)) return false;
+    if (!(lo_t <= hi_t)) return;
     const uint32_t child = __float_as_uint(nb.z), count = __float_as_uint(nb.w);
     if (count > 0) {
       for (uint32_t k = count; k-- > 0;) st.push(kInstTag | gld1(S.torder, child + k));
@@ -588,87 +637,116 @@ struct Walker {
         st.push(child + 1);
       }
     }
-    return st.overflow;
+    if (st.overflow) stop(st);
   }
 
-  // The kind of step the lane needs next: 0 a TLAS step, 1 the held leaf,
-  // 2 an interior step. A finished BLAS walk (no entry left, no leaf held)
-  // first returns the lane to the TLAS.
-  __device__ __forceinline__ int next_kind() {
-    if (blas_base >= 0 && leaf == 0u && !ent_interior(e)) end_instance();
-    return blas_base < 0 ? 0 : (leaf != 0u ? 1 : 2);
-  }
-
-  // One interior step on e (an interior entry, no leaf held): pair-test its
-  // children, continue with the nearer hit one, push the farther; a leaf
-  // reached is held and the next entry popped (walked after the leaf).
+  // One interior step on e (an interior entry): pair-test its children,
+  // continue with the nearer hit one, push the farther; with no child hit,
+  // continue with the entry on top of the stack.
   template <bool kFast>
   __device__ __forceinline__ void interior_step(const DevScene& S, TravStack& st, TravCount& c) {
-    const uint32_t child = e;
-    const float4 la = gld4(S.bnodes, 2 * child), lb = gld4(S.bnodes, 2 * child + 1);
-    const float4 ra = gld4(S.bnodes, 2 * child + 2), rb = gld4(S.bnodes, 2 * child + 3);
+    const float4* pair = S.bnodes + 2 * static_cast<size_t>(e);
+    const float4 la = gld4(pair, 0), lb = gld4(pair, 1), ra = gld4(pair, 2), rb = gld4(pair, 3);
+    const uint32_t below = st.below();
     float tn0, tn1;
+    bool hl, hr;
     if (kCount) {
       ++c.interior;
       c.node_tests += 2;
     }
-    const int m = kFast ? pair_test_fast(la, lb, ra, rb, linv, lo, tmin, tbest, tn0, tn1)
-                        : pair_test(la, lb, ra, rb, linv, lo, tmin, tbest, tn0, tn1);
+    if (kFast) pair_test_fast(la, lb, ra, rb, linv, lo, tmin, tbest, tn0, tn1, hl, hr);
+    else pair_test(la, lb, ra, rb, linv, lo, tmin, tbest, tn0, tn1, hl, hr);
     const uint32_t el = __float_as_uint(lb.w), er = __float_as_uint(rb.w);
-    uint32_t next;
-    if (m == 3) {
-      // closest: nearer first, ties right first (blas.cpp:252-258). Any
-      // hit: farther first. Occlusion does not depend on the order (every
-      // box is tested against the fixed tmax); a shadow ray's nearer child
-      // is mostly the box around its own origin, whose triangles it cannot
-      // hit, so the farther child meets occluders sooner.
-      const bool left_first = kAny ? !(tn0 < tn1) : tn0 < tn1;
-      st.push(left_first ? er : el);
-      next = left_first ? el : er;
-    } else if (m) {
-      next = (m & 1) ? el : er;
-    } else {
-      next = pop_blas(st);
-    }
-    if (ent_leaf(next)) {
-      leaf = next;
-      next = pop_blas(st);
-    }
-    e = next;
-  }
-
-  // Tests the held leaf; true when an any-hit walk found an occluder.
-  __device__ __forceinline__ bool leaf_step(const DevScene& S, TravStack& st, TravCount& c) {
-    uint32_t count = leaf >> kEntShift;
-    const uint32_t first = leaf & kEntIndexMask;
-    if (count == kEntBigLeaf) count = gld1(S.bigcnt, first);
-    for (uint32_t k = 0; k < count; ++k) {
-      float t, u, v;
-      if (kCount) ++c.tri_tests;
-      if (tri_test(S.tris, first + k, lo, ld, tmin, tbest, t, u, v)) {
-        if (kAny) {
-          found = true;
-          return true;
+    // closest: nearer first, ties right first (blas.cpp:252-258). Any hit:
+    // farther first. Occlusion does not depend on the order (every box is
+    // tested against the fixed tmax); a shadow ray's nearer child is mostly
+    // the box around its own origin, whose triangles it cannot hit, so the
+    // farther child meets occluders sooner.
+    const bool left_first = kAny ? !(tn0 < tn1) : tn0 < tn1;
+    const bool both = hl && hr, none = !(hl || hr);
+    const bool left = hl && (!hr || left_first);
+    const uint32_t next = left ? el : er, other = left ? er : el;
+    const uint32_t was = st.tos;
+    const int32_t at = st.top, up = at + st.row;
+    e = none ? was : next;
+    st.tos = both ? other : (none ? below : was);
+    st.top = both ? up : (none ? at - st.row : at);
+    const bool fits = up <= st.last;
+    if (both && fits) *TravStack::word(up) = was;
+    // rare: lanes whose entry lies in the spill
+    if ((ballot(both && !fits) | ballot(none && at > st.last)) != 0ull) {
+      if (both && !fits) {
+        if (!st.keep_spilled(was, kMaxStack + 1)) {
+          st.overflow = true;
+          stop(st);
         }
-        tbest = t;   // the hit distance (hit.t is not kept during the walk)
-        hit.u = u;
-        hit.v = v;
-        hit.slot = first + k;
-        inst_found = true;
+      } else if (none && at > st.last) {
+        st.top = at;
+        st.tos = st.spilled();
+        st.top = at - st.row;
       }
     }
-    leaf = 0u;
-    if (ent_leaf(e)) {
-      leaf = e;
-      e = pop_blas(st);
-    }
-    return false;
   }
 
+  // Tests the leaf e and continues with the entry on top of the stack. The
+  // first two triangles (a leaf of the reference's builder holds at most
+  // two) are fetched together.
+  __device__ __forceinline__ void leaf_step(const DevScene& S, TravStack& st, TravCount& c) {
+    uint32_t count = e >> kEntShift;
+    const uint32_t first = e & kEntIndexMask;
+    const TriRec r0 = load_tri(S.tris, first);
+    const TriRec r1 = load_tri(S.tris, count > 1u ? first + 1u : first);
+    const uint32_t below = st.below();
+    bool ended = test_tri(r0, first, true, c);
+    if (!kAny || !ended) ended = test_tri(r1, first + 1u, count > 1u, c);
+    if (ballot(count > 2u) != 0ull) {   // larger leaves (equal centres, other builders)
+      if (count == kEntBigLeaf) count = gld1(S.bigcnt, first);
+      for (uint32_t k = 2; k < count && !(kAny && ended); ++k) ended = test_tri(load_tri(S.tris, first + k), first + k, true, c);
+    }
+    if (kAny && ended) {
+      occluded = true;
+      stop(st);
+    } else {
+      e = st.tos;
+      st.tos = below;
+      if (st.in_spill()) st.tos = st.spilled();
+      st.top -= st.row;
+    }
+  }
+
+  // Tests one triangle of the leaf (if `there`); a closest hit takes it, true
+  // when an any-hit walk is done.
+  __device__ __forceinline__ bool test_tri(const TriRec& r, uint32_t slot, bool there, TravCount& c) {
+    float t, u, v;
+    if (kCount && there) ++c.tri_tests;
+    const bool yes = tri_test(r, lo, ld, tmin, tbest, t, u, v) && there;
+    if (!kAny && yes) {
+      tbest = t;   // the hit distance (hit.t is not kept during the walk)
+      hit.u = u;
+      hit.v = v;
+      hit.slot = slot;
+      hit.inst = inst;
+    }
+    return kAny && yes;
+  }
 };
 
+// Interior steps of wave_step's lanes while interior steps keep the
+// majority of the wave's BLAS lanes.
+template <bool kFast, bool kAny, bool kCount, bool kPrims>
+__device__ __forceinline__ void interior_run(Walker<kAny, kCount, kPrims>& w, const DevScene& S, TravStack& st,
+                                             TravCount& c) {
+  int ni, nl;
+  do {
+    if (kCount && first_active_lane()) ++c.int_iters;
+    if (ent_interior(w.e)) w.template interior_step<kFast>(S, st, c);
+    ni = lanes_of(ent_interior(w.e));
+    nl = lanes_of(ent_leaf(w.e));
+  } while (ni != 0 && ni >= nl);
+}
+
 // One scheduled run of a wave's walks. Every lane holding a ray names the
-// kind of step it needs next (TLAS entry, held leaf, or interior node pair);
+// kind of step it needs next (TLAS entry, leaf, or interior node pair);
 // the kind most lanes need runs, on those lanes only, while the others wait:
 // interior and leaf steps repeat while their kind keeps the majority of the
 // wave's BLAS lanes, TLAS steps while at least half of the lanes that began
@@ -678,40 +756,13 @@ struct Walker {
 // and work counts are the reference's. Scheduling by majority rather than
 // letting every lane finish a whole descent before any leaf is tested keeps
 // more lanes of each iteration busy (a wave's descents differ in length).
-// True on lanes whose ray finished (closest: `found` / `hit`; any: `found` =
-// occluded). Every lane of the wave must reach it.
-// Interior steps of wave_step's lanes while interior steps keep the
-// majority of the wave's BLAS lanes.
-template <bool kFast, bool kAny, bool kCount, bool kPrims>
-__device__ __forceinline__ void interior_run(Walker<kAny, kCount, kPrims>& w, const DevScene& S, TravStack& st,
-                                             TravCount& c, int& k, int& ni, int& nl, bool& done) {
-  constexpr int kLeaf = 1, kInterior = 2, kWait = 3;
-  for (;;) {
-    if (kCount && first_active_lane()) ++c.int_iters;
-    if (k == kInterior) {
-      w.template interior_step<kFast>(S, st, c);
-      if (st.overflow) {
-        w.end_instance();
-        done = true;
-        k = -1;
-      } else {
-        k = w.leaf != 0u ? kLeaf : (ent_interior(w.e) ? kInterior : kWait);
-      }
-    }
-    ni = __popcll(__ballot(k == kInterior));
-    nl = __popcll(__ballot(k == kLeaf));
-    if (ni == 0 || ni < nl) break;
-  }
-}
-
+// Lanes without a ray (Walker::idle) and finished ones take no part. Every
+// lane of the wave must reach it.
 template <bool kAny, bool kCount, bool kPrims>
-__device__ __forceinline__ bool wave_step(Walker<kAny, kCount, kPrims>& w, const DevScene& S, TravStack& st,
-                                          TravCount& c, bool active) {
-  constexpr int kTlas = 0, kLeaf = 1, kInterior = 2, kWait = 3;
-  int k = active ? w.next_kind() : -1;
-  const int nt = __popcll(__ballot(k == kTlas));
-  int nl = __popcll(__ballot(k == kLeaf)), ni = __popcll(__ballot(k == kInterior));
-  bool done = false;
+__device__ __forceinline__ void wave_step(Walker<kAny, kCount, kPrims>& w, const DevScene& S, TravStack& st,
+                                          TravCount& c) {
+  const int nt = lanes_of(w.e == kEntEnd && !st.empty());
+  int nl = lanes_of(ent_leaf(w.e)), ni = lanes_of(ent_interior(w.e));
   if (ni >= nl && ni >= nt) {
     // the hardware min/max slab test when every walking lane's ray allows it
     // (a wave-uniform choice). The two runs are separate loops: with one
@@ -719,40 +770,30 @@ __device__ __forceinline__ bool wave_step(Walker<kAny, kCount, kPrims>& w, const
     // distances before the branch, and the min/max instructions then
     // re-canonicalised each of them (a value from another block may be a
     // signalling NaN), 12 more instructions per node pair.
-    if (__ballot(k == kInterior && !w.fast) == 0ull) interior_run<true>(w, S, st, c, k, ni, nl, done);
-    else interior_run<false>(w, S, st, c, k, ni, nl, done);
+    if (ni == 0) return;
+    if (ballot(ent_interior(w.e) && !w.fast) == 0ull) interior_run<true>(w, S, st, c);
+    else interior_run<false>(w, S, st, c);
   } else if (nl >= nt) {
-    for (;;) {
+    do {
       if (kCount && first_active_lane()) ++c.leaf_iters;
-      if (k == kLeaf) {
+      if (ent_leaf(w.e)) {
         if (kCount) ++c.leaf_steps;
-        if (w.leaf_step(S, st, c)) {
-          done = true;
-          k = -1;
-        } else {
-          k = w.leaf != 0u ? kLeaf : (ent_interior(w.e) ? kInterior : kWait);
-        }
+        w.leaf_step(S, st, c);
       }
-      nl = __popcll(__ballot(k == kLeaf));
-      ni = __popcll(__ballot(k == kInterior));
-      if (nl == 0 || nl < ni) break;
-    }
+      nl = lanes_of(ent_leaf(w.e));
+      ni = lanes_of(ent_interior(w.e));
+    } while (nl != 0 && nl >= ni);
   } else {
-    for (;;) {
-      if (k == kTlas) {
-        if (w.tlas_step(S, st, c) || st.overflow) {
-          if (st.overflow) w.end_instance();
-          done = true;
-          k = -1;
-        } else if (w.blas_base >= 0) {
-          k = kWait;
-        }
+    bool part = w.e == kEntEnd && !st.empty();   // in this run until it enters a BLAS or ends
+    int n0;
+    do {
+      if (part) {
+        w.tlas_step(S, st, c);
+        part = w.e == kEntEnd && !st.empty();
       }
-      const int n0 = __popcll(__ballot(k == kTlas));
-      if (n0 == 0 || 2 * n0 < nt) break;
-    }
+      n0 = lanes_of(part);
+    } while (n0 != 0 && 2 * n0 >= nt);
   }
-  return done;
 }
 
 // Whole walk of one ray per lane (the ray-batch API), with work counts.
@@ -762,18 +803,17 @@ __device__ __forceinline__ bool walk_scene(const DevScene& S, f3 o, f3 d, float 
                                            HitRef& hit, TravStack& st, TravCount& c) {
   Walker<kAny> w;
   w.begin(S, o, d, tmin, tmax, st);
-  bool done = !valid;
-  for (uint32_t guard = 0; __ballot(!done) != 0ull; ++guard) {
+  if (!valid) w.stop(st);
+  for (uint32_t guard = 0; ballot(!w.finished(st)) != 0ull; ++guard) {
     if (guard >= kWaveStepLimit) {
-      w.stuck = true;
+      st.overflow = true;
       break;
     }
-    if (wave_step(w, S, st, c, !done)) done = true;
+    wave_step(w, S, st, c);
   }
-  if (w.stuck) st.overflow = true;
   hit = w.hit;
-  hit.t = w.found ? w.tbest : 0.f;
-  return valid && w.found;
+  hit.t = w.found() ? w.tbest : 0.f;
+  return valid && w.found();
 }
 
 }  // namespace xnh

@@ -252,8 +252,11 @@ __device__ __forceinline__ void flush_counts(unsigned long long* stats, const Tr
 
 __device__ __forceinline__ TravStack make_stack(uint32_t* spill, int lds_depth) {
   TravStack st;
-  st.lds_col = static_cast<int>(threadIdx.x);
-  st.lds_stride = static_cast<int>(blockDim.x);
+  // the dynamic LDS's byte address (its low 32 bits as a generic pointer)
+  const int32_t base = static_cast<int32_t>(reinterpret_cast<uintptr_t>((TravStack::LdsWord*)trav_lds));
+  st.row = static_cast<int32_t>(4u * blockDim.x);
+  st.bottom = base + static_cast<int32_t>(4u * threadIdx.x) - st.row;
+  st.last = st.bottom + lds_depth * st.row;
   st.spill = spill + (static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x);
   st.spill_stride = static_cast<int>(gridDim.x * blockDim.x);
   st.lds_depth = lds_depth;

@@ -93,6 +93,7 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchVie
   const unsigned long long below = (1ull << lane) - 1ull;
   uint32_t my = kIdle;
   Walker<kAny, kCount, kPrims> w;
+  w.idle(st);
   uint32_t pbase = 0, pnext = 0, pend = 0;   // wave-uniform pool: entries pbase + [pnext, pend) of chunk pci
   int pci = 0;
   // Units are taken from the cursor several at a time: one global atomic
@@ -212,7 +213,8 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchVie
     if (kCount && lane == 0) ++c.round_iters;
     if (kCount && my != kIdle) ++c.round_lanes;
     const DevScene& S = job_scene(B.jobs, uniform(v.ch[pci].job));
-    if (wave_step(w, S, st, c, my != kIdle)) {
+    wave_step(w, S, st, c);
+    if (my != kIdle && w.finished(st)) {
       overflow |= st.overflow;
       finish(my, w);
       ++rays;
@@ -240,7 +242,7 @@ struct SortPool<false> {
 };
 
 template <bool kCount, bool kPrims, bool kCamera>
-__global__ void __launch_bounds__(256) k_closest(WaveBuffers B, int qi, int cursor, int lds_depth) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kCount || kPrims ? 4 : 5))) k_closest(WaveBuffers B, int qi, int cursor, int lds_depth) {
   __shared__ BatchView v;
   __shared__ SortPool<!kCamera> sp;
   const uint32_t* counts = B.counters + ctr_path(qi, 0, 0);
@@ -273,7 +275,7 @@ __global__ void __launch_bounds__(256) k_closest(WaveBuffers B, int qi, int curs
         tmax = __builtin_huge_valf();
       },
       [&](uint32_t i, const Walker<false, kCount, kPrims>& w) {
-        B.hit[i] = make_float4(w.found ? w.tbest : 0.f, w.hit.u, w.hit.v, __int_as_float(w.found ? w.hit.inst : -1));
+        B.hit[i] = make_float4(w.found() ? w.tbest : 0.f, w.hit.u, w.hit.v, __int_as_float(w.hit.inst));
         B.hit_slot[i] = w.hit.slot;
       });
   flush_counts_block(B.stats, c, rays, false, kCount);
@@ -696,7 +698,7 @@ __global__ void __launch_bounds__(256) k_shadow(WaveBuffers B, int cursor, int l
         tmax = r1.z;
       },
       [&](uint32_t i, const Walker<true, kCount, kPrims>& w) {
-        if (!w.found) {
+        if (!w.found()) {
           const uint32_t k = __float_as_uint(B.sh1[i].w);
           const float4 cv = B.sh_c[i];
           float4 acc = B.l_nee[k];

@@ -560,7 +560,7 @@ int alloc_waves(xnh_ctx* c) {
   if (rc == XNH_OK) rc = dev_alloc(c, c->wave_allocs, &B.counters, static_cast<size_t>(kNumCtr));
   if (rc == XNH_OK) rc = dev_alloc(c, c->wave_allocs, &B.stats, static_cast<size_t>(kNumStat));
   if (rc == XNH_OK) {
-    const size_t spill = static_cast<size_t>(kMaxStack - c->lds_depth) * c->grid_trace * c->block;
+    const size_t spill = static_cast<size_t>(kMaxStack + 1 - c->lds_depth) * c->grid_trace * c->block;
     rc = dev_alloc(c, c->wave_allocs, &B.spill, spill);
   }
   if (rc != XNH_OK) {
@@ -1859,7 +1859,7 @@ static int trace_common(xnh_ctx* c, const xnh_ray* rays, int32_t n, bool any, vo
     if (any) rc = dev_alloc(c, tmp, reinterpret_cast<uint8_t**>(&d_out), static_cast<size_t>(n));
     else rc = dev_alloc(c, tmp, reinterpret_cast<float**>(&d_out), static_cast<size_t>(n) * 16);
   }
-  if (rc == XNH_OK) rc = dev_alloc(c, tmp, &d_spill, static_cast<size_t>(kMaxStack - c->lds_depth) * threads);
+  if (rc == XNH_OK) rc = dev_alloc(c, tmp, &d_spill, static_cast<size_t>(kMaxStack + 1 - c->lds_depth) * threads);
   if (rc == XNH_OK) rc = dev_alloc(c, tmp, &d_stats, static_cast<size_t>(kNumStat));
   if (rc == XNH_OK) rc = dev_alloc(c, tmp, &d_ovf, 1);
   if (rc != XNH_OK) {
