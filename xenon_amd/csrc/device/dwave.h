@@ -193,41 +193,6 @@ __device__ __forceinline__ unsigned long long wave_sum(unsigned long long v) {
 
 // Wave-reduced ray and (with `work`) traversal counters; `any` selects the
 // shadow slots.
-// The persistent traversal kernels' counts, summed over the work-group and
-// added with one atomic per counter and work-group: the waves of a launch
-// finish together, and one same-address atomic per wave at the end made a
-// serial tail. Every thread of the work-group must reach it (256 threads).
-__device__ __forceinline__ void flush_counts_block(unsigned long long* stats, const TravCount& c, uint32_t rays,
-                                                   bool any, bool work) {
-  constexpr int kN = 10;
-  __shared__ unsigned long long red[kN][256 / 64];
-  const int w = static_cast<int>(threadIdx.x >> 6), nw = static_cast<int>(blockDim.x >> 6);
-  const unsigned long long v[kN] = {
-      wave_sum(rays),
-      work ? wave_sum(c.node_tests) : 0ull,
-      work ? wave_sum(c.interior) : 0ull,
-      work ? wave_sum(c.tri_tests) : 0ull,
-      work ? wave_sum(c.inst_visits) : 0ull,
-      work ? wave_sum(c.int_iters) : 0ull,
-      work ? wave_sum(c.leaf_iters) : 0ull,
-      work ? wave_sum(c.leaf_steps) : 0ull,
-      work ? wave_sum(c.round_iters) : 0ull,
-      work ? wave_sum(c.round_lanes) : 0ull};
-  if (lane_id() == 0)
-    for (int k = 0; k < kN; ++k) red[k][w] = v[k];
-  __syncthreads();
-  if (threadIdx.x < static_cast<unsigned>(kN)) {
-    unsigned long long t = 0;
-    for (int k = 0; k < nw; ++k) t += red[threadIdx.x][k];
-    const int k = static_cast<int>(threadIdx.x);
-    int slot;
-    if (k == 0) slot = any ? kStShadow : kStClosest;
-    else if (k < 5) slot = (any ? kStShNodeTests : kStNodeTests) + k - 1;
-    else slot = (any ? kStShIntIters : kStIntIters) + k - 5;
-    if (t) atomicAdd(&stats[slot], t);
-  }
-}
-
 __device__ __forceinline__ void flush_counts(unsigned long long* stats, const TravCount& c, uint32_t rays, bool any,
                                              bool work = true) {
   const unsigned long long r = wave_sum(rays);
@@ -386,38 +351,89 @@ struct BatchView {
 // with mul 1 (path queue) or 2 (shadow queue); null: prefix over pixels.
 // A count is clamped to its segment (segment 0 of a path queue may hold the
 // chunk's whole region: depth 0), so reads stay inside the chunk's region
-// even if an append ever overflowed a segment. Block-wide; ends with a
-// barrier.
+// even if an append ever overflowed a segment. Every work-group of every
+// launch runs this first, so its dependent loads are few (batch index, then
+// the chunks and their number, then the counts) and the sums over chunks
+// are a scan by one wave (one thread adding up 64 chunks' counts took 10 us
+// of each launch). Block-wide; ends with a barrier.
 __device__ __forceinline__ void load_batch(BatchView& v, const WaveBuffers& B, const uint32_t* counts,
                                            bool pixels, uint32_t mul = 1u) {
-  if (threadIdx.x == 0) {
-    v.batch = static_cast<int>(B.counters[kBatch]);
-    v.nch = B.nchunks[v.batch];
+  const int tid = static_cast<int>(threadIdx.x);
+  const int batch = static_cast<int>(B.counters[kBatch]);
+  const int nch = B.nchunks[batch];
+  if (tid == 0) {
+    v.batch = batch;
+    v.nch = nch;
+    v.prefix[0] = 0u;
   }
+  if (tid < nch) v.ch[tid] = B.chunks[batch * kMaxChunks + tid];
   __syncthreads();
-  if (static_cast<int>(threadIdx.x) < v.nch) v.ch[threadIdx.x] = B.chunks[v.batch * kMaxChunks + threadIdx.x];
-  __syncthreads();
-  if (counts)
-    for (int t = static_cast<int>(threadIdx.x); t < v.nch * kQSeg; t += static_cast<int>(blockDim.x)) {
+  if (counts) {
+    for (int t = tid; t < nch * kQSeg; t += static_cast<int>(blockDim.x)) {
       const int ci = t / kQSeg, x = t % kQSeg;
       const uint32_t qseg = static_cast<uint32_t>(v.ch[ci].qseg);
       const uint32_t room = mul * ((mul == 1u && x == 0) ? static_cast<uint32_t>(kQSeg) * qseg : qseg);
       v.cnt[ci][x] = min(counts[t * kCtrStride], room);
     }
-  __syncthreads();
-  if (threadIdx.x == 0) {
+    __syncthreads();
+  }
+  static_assert(kMaxChunks == 64, "one lane per chunk");
+  if (tid < 64) {
     uint32_t acc = 0;
-    v.prefix[0] = 0;
-    for (int c = 0; c < v.nch; ++c) {
-      if (pixels) {
-        acc += static_cast<uint32_t>(v.ch[c].npix);
-      } else {
-        for (int x = 0; x < kQSeg; ++x) acc += (v.cnt[c][x] + 63u) >> 6;
-      }
-      v.prefix[c + 1] = acc;
+    if (tid < nch) {
+      if (pixels) acc = static_cast<uint32_t>(v.ch[tid].npix);
+      else
+        for (int x = 0; x < kQSeg; ++x) acc += (v.cnt[tid][x] + 63u) >> 6;
     }
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t t = __shfl_up(acc, o);
+      if (tid >= o) acc += t;
+    }
+    if (tid < nch) v.prefix[tid + 1] = acc;
   }
   __syncthreads();
+}
+
+// The persistent traversal kernels' counts. Every entry of the launch's queue
+// is one ray, so without work counters the first work-group adds the queue's
+// length (every work-group adding its own rays was a thousand atomics on one
+// address at the end of each launch). The counting variants sum over the
+// work-group and add with one atomic per counter and work-group; every
+// thread of the work-group must reach it (256 threads). `any` selects the
+// shadow slots.
+template <bool kWork>
+__device__ __forceinline__ void flush_counts_block(unsigned long long* stats, const BatchView& v, const TravCount& c,
+                                                   uint32_t rays, bool any) {
+  if constexpr (!kWork) {
+    if (blockIdx.x == 0 && threadIdx.x < 64u) {
+      unsigned long long n = 0;
+      if (static_cast<int>(threadIdx.x) < v.nch)
+        for (int x = 0; x < kQSeg; ++x) n += v.cnt[threadIdx.x][x];
+      n = wave_sum(n);
+      if (threadIdx.x == 0 && n) atomicAdd(&stats[any ? kStShadow : kStClosest], n);
+    }
+  } else {
+    constexpr int kN = 10;
+    __shared__ unsigned long long red[kN][256 / 64];
+    const int w = static_cast<int>(threadIdx.x >> 6), nw = static_cast<int>(blockDim.x >> 6);
+    const unsigned long long n[kN] = {
+        wave_sum(rays),         wave_sum(c.node_tests), wave_sum(c.interior),    wave_sum(c.tri_tests),
+        wave_sum(c.inst_visits), wave_sum(c.int_iters),  wave_sum(c.leaf_iters),  wave_sum(c.leaf_steps),
+        wave_sum(c.round_iters), wave_sum(c.round_lanes)};
+    if (lane_id() == 0)
+      for (int k = 0; k < kN; ++k) red[k][w] = n[k];
+    __syncthreads();
+    if (threadIdx.x < static_cast<unsigned>(kN)) {
+      unsigned long long t = 0;
+      for (int k = 0; k < nw; ++k) t += red[threadIdx.x][k];
+      const int k = static_cast<int>(threadIdx.x);
+      int slot;
+      if (k == 0) slot = any ? kStShadow : kStClosest;
+      else if (k < 5) slot = (any ? kStShNodeTests : kStNodeTests) + k - 1;
+      else slot = (any ? kStShIntIters : kStIntIters) + k - 5;
+      if (t) atomicAdd(&stats[slot], t);
+    }
+  }
 }
 
 // Last chunk c with prefix[c] <= u: the (non-empty) chunk holding item u.

@@ -82,13 +82,18 @@ __global__ void __launch_bounds__(256) k_raygen(WaveBuffers B) {
 // changes no ray's result.
 // Must be reached by every lane of the wave.
 // ---------------------------------------------------------------------------
+// Units a wave takes at once when `left` are left: what is left over
+// `parts`, 1 to 16.
+__device__ __forceinline__ uint32_t fetch_size(uint32_t left, uint32_t parts) {
+  return max(1u, min(16u, left / parts));
+}
+
 template <bool kAny, bool kCount, bool kPrims, bool kSort, class Load, class Finish>
 __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchView& v, uint32_t* cursor,
                                             uint32_t seg, TravStack& st, TravCount& c, uint32_t& rays,
                                             bool& overflow, const float4* ray1, uint16_t* slist, uint32_t* sbase,
                                             Load load, Finish finish) {
   constexpr uint32_t kIdle = 0xFFFFFFFFu;
-  const uint32_t total = v.prefix[v.nch];
   const int lane = lane_id();
   const unsigned long long below = (1ull << lane) - 1ull;
   uint32_t my = kIdle;
@@ -110,9 +115,27 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchVie
   const uint32_t batch_units =
       v.nch > 0 ? static_cast<uint32_t>(v.ch[v.nch - 1].base + v.ch[v.nch - 1].cap) >> 6 : 0u;
   const uint32_t share = batch_units < 64u * gwaves ? 2u : 4u;
-  uint32_t seen = 0;              // the first unit of this wave's last fetch
-  uint32_t ucur = 0, uend = 0;    // fetched units not yet taken (wave-uniform)
-  bool exhausted = false;
+  // A launch of fewer units than the grid has waves hands out parts of
+  // units, down to 4 entries, as long as there are waves to take them: such a
+  // launch lasts as long as its slowest wave, and a wave of fewer rays takes
+  // turns between fewer kinds of step (below, units and the cursor count
+  // these parts). Whole units only: 1.3M-triangle mesh at 1920x1080x1 8.51
+  // instead of 8.16 ms, primitives at 801x449x33 7.83 instead of 7.60 ms;
+  // down to 8 or 16 entries: in between.
+  uint32_t split = 0;
+  while (split < 4u && (v.prefix[v.nch] << (split + 1u)) <= gwaves) ++split;
+  const uint32_t part = 64u >> split, pmask = (1u << split) - 1u;
+  const uint32_t total = v.prefix[v.nch] << split;
+  // Every wave's first units are its own share by its place in the grid; the
+  // cursor hands out what follows them. A launch with no more than that
+  // takes no atomic at all (one per wave, only to learn that nothing is
+  // left, cost a launch of 5120 waves 60 us: a 256x256x1 Cornell frame spent
+  // 2.0 of 2.2 ms in such launches and takes 0.75 ms now).
+  const uint32_t first_units = fetch_size(total, share * gwaves);
+  const uint32_t dealt = first_units * gwaves;
+  uint32_t seen = (blockIdx.x * (blockDim.x >> 6) + static_cast<uint32_t>(uniform(static_cast<int>(threadIdx.x >> 6)))) * first_units;
+  uint32_t ucur = min(seen, total), uend = min(seen + first_units, total);   // fetched units not yet taken (wave-uniform)
+  bool exhausted = dealt >= total;
   bool stuck = false;
   for (uint32_t guard = 0;; ++guard) {
     if (guard >= kWaveStepLimit) {
@@ -123,11 +146,10 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchVie
     if (act != ~0ull) {
       if (pnext >= pend) {
         if (ucur >= uend && !exhausted) {
-          const uint32_t left = total > seen ? total - seen : 0u;
-          const uint32_t per = max(1u, min(16u, left / (share * gwaves)));
+          const uint32_t per = fetch_size(total - seen, share * gwaves);
           uint32_t u0 = 0;
           if (lane == 0) u0 = atomicAdd(cursor, per);
-          u0 = static_cast<uint32_t>(uniform(static_cast<int>(__shfl(u0, 0))));
+          u0 = dealt + static_cast<uint32_t>(uniform(static_cast<int>(__shfl(u0, 0))));
           if (u0 >= total) {
             exhausted = true;
           } else {
@@ -139,13 +161,13 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchVie
         if (ucur < uend) {
           // a unit of another job waits until the wave has drained (the
           // rays in flight in a wave share one scene)
-          const int ci = uniform(find_chunk(v, ucur));
+          const int ci = uniform(find_chunk(v, ucur >> split));
           if (act == 0ull || v.ch[ci].job == v.ch[pci].job) {
             pci = ci;
             if constexpr (kSort) {
               // the fetched units that lie in this chunk (1 to 16), keyed by
               // octant (4 bits per unit and lane; 8 = no entry)
-              const uint32_t n = min(uend, v.prefix[ci + 1]) - ucur;
+              const uint32_t n = min(uend, v.prefix[ci + 1] << split) - ucur;
               uint32_t keys0 = 0u, keys1 = 0u;
               // every lane has taken its entry of the last pool before the
               // order is rewritten
@@ -154,8 +176,10 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchVie
               __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
               for (uint32_t j = 0; j < n; ++j) {
                 uint32_t first, lim;
-                const uint32_t b = unit_segment(v, ci, ucur + j - v.prefix[ci], seg, first, lim) + first;
-                const uint32_t cnt = lim > first ? min(64u, lim - first) : 0u;
+                uint32_t b = unit_segment(v, ci, ((ucur + j) >> split) - v.prefix[ci], seg, first, lim);
+                first += ((ucur + j) & pmask) * part;
+                b += first;
+                const uint32_t cnt = lim > first ? min(part, lim - first) : 0u;
                 if (lane == 0) sbase[j] = b;
                 uint32_t key = 8u;
                 if (static_cast<uint32_t>(lane) < cnt)
@@ -182,9 +206,9 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchVie
               ucur += n;
             } else {
               uint32_t first, lim;
-              pbase = unit_segment(v, ci, ucur - v.prefix[ci], seg, first, lim);
-              pnext = first;
-              pend = min(first + 64u, lim);
+              pbase = unit_segment(v, ci, (ucur >> split) - v.prefix[ci], seg, first, lim);
+              pnext = first + (ucur & pmask) * part;
+              pend = min(pnext + part, lim);   // none past the segment's last entry
               ++ucur;
             }
           }
@@ -209,7 +233,9 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchVie
         pnext = min(pend, pnext + static_cast<uint32_t>(__popcll(idle)));
       }
     }
-    if (__ballot(my != kIdle) == 0ull) break;
+    // (a part of a segment's last unit may hold no entry: a wave without rays
+    // goes on while it has units; its step below does nothing)
+    if (exhausted && ucur >= uend && __ballot(my != kIdle) == 0ull) break;
     if (kCount && lane == 0) ++c.round_iters;
     if (kCount && my != kIdle) ++c.round_lanes;
     const DevScene& S = job_scene(B.jobs, uniform(v.ch[pci].job));
@@ -217,7 +243,7 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchVie
     if (my != kIdle && w.finished(st)) {
       overflow |= st.overflow;
       finish(my, w);
-      ++rays;
+      if (kCount) ++rays;
       my = kIdle;
     }
   }
@@ -242,7 +268,7 @@ struct SortPool<false> {
 };
 
 template <bool kCount, bool kPrims, bool kCamera>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kCount || kPrims ? 4 : 5))) k_closest(WaveBuffers B, int qi, int cursor, int lds_depth) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kCount ? 4 : 5))) k_closest(WaveBuffers B, int qi, int cursor, int lds_depth) {
   __shared__ BatchView v;
   __shared__ SortPool<!kCamera> sp;
   const uint32_t* counts = B.counters + ctr_path(qi, 0, 0);
@@ -278,7 +304,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kCount
         B.hit[i] = make_float4(w.found() ? w.tbest : 0.f, w.hit.u, w.hit.v, __int_as_float(w.hit.inst));
         B.hit_slot[i] = w.hit.slot;
       });
-  flush_counts_block(B.stats, c, rays, false, kCount);
+  flush_counts_block<kCount>(B.stats, v, c, rays, false);
   if (overflow) atomicAdd(&B.counters[kOverflow], 1u);
 }
 
@@ -300,7 +326,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kCount
 // amortise the window's class loads over more entries; at four waves per
 // SIMD (128 VGPRs, a few bytes spilled) the plain kernel beat three waves
 // without the spill (benchmark k_shade 225 -> 217 ms per two steps). The
-// guided kernel keeps its three waves.
+// guided kernel keeps its three waves. A launch of fewer units than eight
+// per wave of the grid takes smaller windows, as many as give every wave
+// one: its time is the passes of one wave, one after the other, and waves
+// stood idle (256x256x1 Cornell frame: 79 -> 19 us a launch; 1920x1080x1
+// mesh frame: 105 -> 65 us).
 
 template <bool kGuided>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGuided ? 3 : 4))) k_shade(WaveBuffers B, int qi, int depth) {
@@ -318,8 +348,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGuide
   const uint32_t lane = static_cast<uint32_t>(lane_id());
   const unsigned long long below = (1ull << lane) - 1ull;
   const uint32_t waves = gridDim.x * (blockDim.x >> 6);
-  for (uint32_t u0 = (blockIdx.x * (blockDim.x >> 6) + wv) * kShadeWin; u0 < total; u0 += waves * kShadeWin) {
-    const uint32_t nu = min(kShadeWin, total - u0);
+  const uint32_t win = max(1u, min(kShadeWin, (total + waves - 1u) / waves));   // units per window
+  for (uint32_t u0 = (blockIdx.x * (blockDim.x >> 6) + wv) * win; u0 < total; u0 += waves * win) {
+    const uint32_t nu = min(win, total - u0);
     const int ci0 = uniform(find_chunk(v, u0));
     const bool sorted = uniform(find_chunk(v, u0 + nu - 1)) == ci0;
     // every unit's first queue entry and entry count (wave-uniform; lane u
@@ -578,7 +609,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGuide
                 // one atomic per wave, on the record segment of this window
                 // (windows go to the segments in turn, so no segment takes
                 // more than one window's entries over an equal share)
-                const uint32_t rs = B.rec_cap / kQSeg, rx = (u0 / kShadeWin) % kQSeg;
+                const uint32_t rs = B.rec_cap / kQSeg, rx = (u0 / win) % kQSeg;
                 uint32_t r = wave_append(&B.counters[ctr_rec(static_cast<int>(rx))], rec);
                 if (rec) {
                   if (r < rs) {
@@ -680,7 +711,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGuide
 // to their path's per-slot NEE sum (one writer per (slot, light kind)).
 // ---------------------------------------------------------------------------
 template <bool kCount, bool kPrims>
-__global__ void __launch_bounds__(256) k_shadow(WaveBuffers B, int cursor, int lds_depth) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kCount ? 4 : 5))) k_shadow(WaveBuffers B, int cursor, int lds_depth) {
   __shared__ BatchView v;
   const uint32_t* counts = B.counters + ctr_shadow(0, 0);
   load_batch(v, B, counts, false, 2u);
@@ -708,7 +739,7 @@ __global__ void __launch_bounds__(256) k_shadow(WaveBuffers B, int cursor, int l
           B.l_nee[k] = acc;
         }
       });
-  flush_counts_block(B.stats, c, rays, true, kCount);
+  flush_counts_block<kCount>(B.stats, v, c, rays, true);
   if (overflow) atomicAdd(&B.counters[kOverflow], 1u);
 }
 
