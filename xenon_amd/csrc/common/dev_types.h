@@ -219,17 +219,19 @@ enum Ctr : int {
   kWatchdog = 3,                         // waves that hit an iteration bound (see dtrace.h)
   kSegOverflow = 4,                      // appends past a queue segment's end (dropped; never expected)
   kCnt = 16,                                        // [queue][chunk][segment] live paths (stride kCtrStride)
-  kShCnt = kCnt + 2 * kMaxChunks * kQSeg * kCtrStride,  // [chunk][segment] shadow rays
-  kCursor = kShCnt + kMaxChunks * kQSeg * kCtrStride,   // per-launch work cursors of a batch
+  // [set][chunk][segment] shadow rays: depth d's are counted in set d & 1, so
+  // that the launch that walks them can clear the next depth's
+  kShCnt = kCnt + 2 * kMaxChunks * kQSeg * kCtrStride,
+  kCursor = kShCnt + 2 * kMaxChunks * kQSeg * kCtrStride,   // per-launch work cursors of a batch
   kNumCursors = 2 * 64 + 4,
   // [segment] guiding training records of the batch (stride kCtrStride)
   kRecCnt = (kCursor + kNumCursors + kCtrStride - 1) / kCtrStride * kCtrStride,
   kNumCtr = kRecCnt + kQSeg * kCtrStride
 };
 
-// Counter of segment x of chunk ci: path queue q, shadow queue.
+// Counter of segment x of chunk ci: path queue q, shadow counter set q.
 constexpr int ctr_path(int q, int ci, int x) { return kCnt + ((q * kMaxChunks + ci) * kQSeg + x) * kCtrStride; }
-constexpr int ctr_shadow(int ci, int x) { return kShCnt + (ci * kQSeg + x) * kCtrStride; }
+constexpr int ctr_shadow(int q, int ci, int x) { return kShCnt + ((q * kMaxChunks + ci) * kQSeg + x) * kCtrStride; }
 // 64-entry units per window of the shading kernel
 constexpr uint32_t kShadeWin = 8;
 

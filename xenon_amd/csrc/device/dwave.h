@@ -346,51 +346,116 @@ struct BatchView {
   uint32_t prefix[kMaxChunks + 1];
 };
 
-// Loads the batch and builds prefix[] from the segment counts. counts: the
-// queue's counter of chunk 0, segment 0, as ctr_path / ctr_shadow give it,
-// with mul 1 (path queue) or 2 (shadow queue); null: prefix over pixels.
-// A count is clamped to its segment (segment 0 of a path queue may hold the
-// chunk's whole region: depth 0), so reads stay inside the chunk's region
-// even if an append ever overflowed a segment. Every work-group of every
-// launch runs this first, so its dependent loads are few (batch index, then
-// the chunks and their number, then the counts) and the sums over chunks
-// are a scan by one wave (one thread adding up 64 chunks' counts took 10 us
-// of each launch). Block-wide; ends with a barrier.
-__device__ __forceinline__ void load_batch(BatchView& v, const WaveBuffers& B, const uint32_t* counts,
-                                           bool pixels, uint32_t mul = 1u) {
+// One queue's view in the traversal kernels: its segments' entry counts and
+// the prefix sums of units over chunks.
+struct TraceQueue {
+  uint32_t cnt[kMaxChunks][kQSeg];
+  uint32_t prefix[kMaxChunks + 1];
+};
+struct TraceChunk {
+  int32_t job, qbase, qseg;
+};
+// What the traversal of bounce and shadow rays needs of the batch.
+struct TraceView {
+  int nch;
+  uint32_t batch_units;   // units of the batch at depth 0
+  TraceChunk ch[kMaxChunks];
+  TraceQueue q[2];        // the path queue, the shadow queue
+};
+// A queue as find_chunk, unit_segment and trace_queue take it (a BatchView
+// has the same members).
+struct TraceUnits {
+  const int& nch;
+  const TraceChunk* ch;
+  const uint32_t (*cnt)[kQSeg];
+  const uint32_t* prefix;
+  __device__ __forceinline__ TraceUnits(const TraceView& v, int q)
+      : nch(v.nch), ch(v.ch), cnt(v.q[q].cnt), prefix(v.q[q].prefix) {}
+};
+
+// A queue's segment counts. counts: its counter of chunk 0, segment 0, as
+// ctr_path / ctr_shadow give it, with mul 1 (path queue) or 2 (shadow
+// queue). A count is clamped to its segment (segment 0 of a path queue may
+// hold the chunk's whole region: depth 0), so reads stay inside the chunk's
+// region even if an append ever overflowed a segment.
+template <class Chunk>
+__device__ __forceinline__ void load_counts(uint32_t (*cnt)[kQSeg], const Chunk* ch, int nch, const uint32_t* counts,
+                                            uint32_t mul) {
+  for (int t = static_cast<int>(threadIdx.x); t < nch * kQSeg; t += static_cast<int>(blockDim.x)) {
+    const int ci = t / kQSeg, x = t % kQSeg;
+    const uint32_t qseg = static_cast<uint32_t>(ch[ci].qseg);
+    const uint32_t room = mul * ((mul == 1u && x == 0) ? static_cast<uint32_t>(kQSeg) * qseg : qseg);
+    cnt[ci][x] = counts ? min(counts[t * kCtrStride], room) : 0u;
+  }
+}
+__device__ __forceinline__ uint32_t chunk_units(const uint32_t (*cnt)[kQSeg], int ci) {
+  uint32_t acc = 0;
+  for (int x = 0; x < kQSeg; ++x) acc += (cnt[ci][x] + 63u) >> 6;
+  return acc;
+}
+// Prefix sums over chunks by the work-group's first wave, lane t holding
+// chunk t's `acc` (a scan: one thread adding up 64 chunks' counts took 10 us
+// of each launch).
+__device__ __forceinline__ void scan_chunks(uint32_t* prefix, uint32_t acc, int nch) {
+  static_assert(kMaxChunks == 64, "one lane per chunk");
+  const int lane = static_cast<int>(threadIdx.x);
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t t = __shfl_up(acc, o);
+    if (lane >= o) acc += t;
+  }
+  if (lane == 0) prefix[0] = 0u;
+  if (lane < nch) prefix[lane + 1] = acc;
+}
+
+// Loads the batch and builds prefix[] from the segment counts (see
+// load_counts), or, with counts null, over pixels. Every work-group of every
+// launch starts with it, so its dependent loads are few: batch index, then
+// the chunks and their number, then the counts. Block-wide; ends with a
+// barrier.
+__device__ __forceinline__ void load_batch(BatchView& v, const WaveBuffers& B, const uint32_t* counts, bool pixels) {
   const int tid = static_cast<int>(threadIdx.x);
   const int batch = static_cast<int>(B.counters[kBatch]);
   const int nch = B.nchunks[batch];
   if (tid == 0) {
     v.batch = batch;
     v.nch = nch;
-    v.prefix[0] = 0u;
   }
   if (tid < nch) v.ch[tid] = B.chunks[batch * kMaxChunks + tid];
   __syncthreads();
   if (counts) {
-    for (int t = tid; t < nch * kQSeg; t += static_cast<int>(blockDim.x)) {
-      const int ci = t / kQSeg, x = t % kQSeg;
-      const uint32_t qseg = static_cast<uint32_t>(v.ch[ci].qseg);
-      const uint32_t room = mul * ((mul == 1u && x == 0) ? static_cast<uint32_t>(kQSeg) * qseg : qseg);
-      v.cnt[ci][x] = min(counts[t * kCtrStride], room);
-    }
+    load_counts(v.cnt, v.ch, nch, counts, 1u);
     __syncthreads();
   }
-  static_assert(kMaxChunks == 64, "one lane per chunk");
   if (tid < 64) {
     uint32_t acc = 0;
-    if (tid < nch) {
-      if (pixels) acc = static_cast<uint32_t>(v.ch[tid].npix);
-      else
-        for (int x = 0; x < kQSeg; ++x) acc += (v.cnt[tid][x] + 63u) >> 6;
-    }
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t t = __shfl_up(acc, o);
-      if (tid >= o) acc += t;
-    }
-    if (tid < nch) v.prefix[tid + 1] = acc;
+    if (tid < nch) acc = pixels ? static_cast<uint32_t>(v.ch[tid].npix) : chunk_units(v.cnt, tid);
+    scan_chunks(v.prefix, acc, nch);
   }
+  __syncthreads();
+}
+
+// The same for the traversal of a path queue (counts) and a shadow queue
+// (shadow_counts); either may be null: no units of it.
+__device__ __forceinline__ void load_trace(TraceView& v, const WaveBuffers& B, const uint32_t* counts,
+                                           const uint32_t* shadow_counts) {
+  const int tid = static_cast<int>(threadIdx.x);
+  const int batch = static_cast<int>(B.counters[kBatch]);
+  const int nch = B.nchunks[batch];
+  if (tid < nch) {
+    const DevChunk& ck = B.chunks[batch * kMaxChunks + tid];
+    v.ch[tid] = TraceChunk{ck.job, ck.qbase, ck.qseg};
+    if (tid == nch - 1) v.batch_units = static_cast<uint32_t>(ck.base + ck.cap) >> 6;
+  }
+  if (tid == 0) {
+    v.nch = nch;
+    if (nch == 0) v.batch_units = 0u;
+  }
+  __syncthreads();
+  load_counts(v.q[0].cnt, v.ch, nch, counts, 1u);
+  load_counts(v.q[1].cnt, v.ch, nch, shadow_counts, 2u);
+  __syncthreads();
+  if (tid < 64)
+    for (int k = 0; k < 2; ++k) scan_chunks(v.q[k].prefix, tid < nch ? chunk_units(v.q[k].cnt, tid) : 0u, nch);
   __syncthreads();
 }
 
@@ -402,13 +467,13 @@ __device__ __forceinline__ void load_batch(BatchView& v, const WaveBuffers& B, c
 // thread of the work-group must reach it (256 threads). `any` selects the
 // shadow slots.
 template <bool kWork>
-__device__ __forceinline__ void flush_counts_block(unsigned long long* stats, const BatchView& v, const TravCount& c,
-                                                   uint32_t rays, bool any) {
+__device__ __forceinline__ void flush_counts_block(unsigned long long* stats, const uint32_t (*cnt)[kQSeg], int nch,
+                                                   const TravCount& c, uint32_t rays, bool any) {
   if constexpr (!kWork) {
     if (blockIdx.x == 0 && threadIdx.x < 64u) {
       unsigned long long n = 0;
-      if (static_cast<int>(threadIdx.x) < v.nch)
-        for (int x = 0; x < kQSeg; ++x) n += v.cnt[threadIdx.x][x];
+      if (static_cast<int>(threadIdx.x) < nch)
+        for (int x = 0; x < kQSeg; ++x) n += cnt[threadIdx.x][x];
       n = wave_sum(n);
       if (threadIdx.x == 0 && n) atomicAdd(&stats[any ? kStShadow : kStClosest], n);
     }
@@ -433,11 +498,13 @@ __device__ __forceinline__ void flush_counts_block(unsigned long long* stats, co
       else slot = (any ? kStShIntIters : kStIntIters) + k - 5;
       if (t) atomicAdd(&stats[slot], t);
     }
+    __syncthreads();   // red may be written again
   }
 }
 
 // Last chunk c with prefix[c] <= u: the (non-empty) chunk holding item u.
-__device__ __forceinline__ int find_chunk(const BatchView& v, uint32_t u) {
+template <class View>
+__device__ __forceinline__ int find_chunk(const View& v, uint32_t u) {
   int lo = 0, hi = v.nch;
   while (hi - lo > 1) {
     const int mid = (lo + hi) >> 1;
@@ -451,7 +518,8 @@ __device__ __forceinline__ int find_chunk(const BatchView& v, uint32_t u) {
 // position of its segment's first entry (mul = 1 path queue, 2 shadow
 // queue) and sets its first entry's offset in that segment and the
 // segment's entry count.
-__device__ __forceinline__ uint32_t unit_segment(const BatchView& v, int ci, uint32_t uc, uint32_t mul, uint32_t& first,
+template <class View>
+__device__ __forceinline__ uint32_t unit_segment(const View& v, int ci, uint32_t uc, uint32_t mul, uint32_t& first,
                                                  uint32_t& lim) {
   uint32_t acc = 0;
   int x = 0;
@@ -462,7 +530,7 @@ __device__ __forceinline__ uint32_t unit_segment(const BatchView& v, int ci, uin
   }
   first = (uc - acc) * 64u;
   lim = v.cnt[ci][x];
-  const DevChunk& ck = v.ch[ci];
+  const auto& ck = v.ch[ci];
   return mul * (static_cast<uint32_t>(ck.qbase) + static_cast<uint32_t>(x) * static_cast<uint32_t>(ck.qseg));
 }
 

@@ -4,11 +4,12 @@
 // paths in flight, through this stream-ordered sequence (no host reads
 // between kernels; every work count lives in device memory):
 //
-//   raygen ─► [ closest(d) ─► shade(d) ─► shadow(d) ]  d = 0 .. max_bounces-1
-//          ─► accumulate
+//   raygen ─► camera ─► shade(0) ─► [ trace(d) ─► shade(d) ]  d = 1 .. max_bounces-1
+//          ─► trace(shadow rays of the last depth) ─► accumulate
 //
-// closest / shadow are persistent: a grid sized to fill the chip, each wave
-// fetching 64 queue entries at a time from a device cursor, so divergent
+// trace(d) walks the closest hits of depth d and the shadow rays of depth
+// d - 1. camera and trace are persistent: a grid sized to fill the chip, each
+// wave fetching 64-entry units of the queues, so divergent
 // traversal work is balanced across waves. shade appends survivors and
 // shadow rays with one atomic per wave (ballot + popcount compaction), so
 // the next bounce's queue is dense and every queue access is coalesced.
@@ -51,7 +52,8 @@ __global__ void __launch_bounds__(256) k_raygen(WaveBuffers B) {
     const DevChunk& ck = v.ch[ci];
     B.counters[ctr_path(0, ci, x)] = (x == 0 && B.jobs[ck.job].maxb > 0) ? static_cast<uint32_t>(ck.cap) : 0u;
     B.counters[ctr_path(1, ci, x)] = 0u;
-    B.counters[ctr_shadow(ci, x)] = 0u;
+    B.counters[ctr_shadow(0, ci, x)] = 0u;
+    B.counters[ctr_shadow(1, ci, x)] = 0u;
   }
   if (tid < kNumCursors) B.counters[kCursor + tid] = 0u;
   if (tid < kQSeg) B.counters[ctr_rec(tid)] = 0u;
@@ -67,12 +69,82 @@ __global__ void __launch_bounds__(256) k_raygen(WaveBuffers B) {
 }
 
 // ---------------------------------------------------------------------------
+// Work of a traversal launch, as one wave takes it: 64-entry units, numbered
+// through the launch's queues one after the other.
+//
+// Units are taken from the cursor several at a time: one global atomic
+// on one address serves only ~85 M operations per second on the whole
+// device, so a fetch per 64-entry unit capped a launch at ~5 G rays/s.
+// A fetch takes up to 16 units, fewer as the queue runs out (what is left
+// per 4 waves of the grid, as this wave last saw it), so the launch
+// does not end with a few waves walking long private batches. Batches of
+// fewer than 64 units per wave (a 512x512 frame at 64 samples on the
+// whole device) walk short queues at every depth: there the fetches'
+// own cost outweighs the balance at the end of a launch, and a fetch
+// takes up to twice as much (what is left per 2 waves).
+//
+// A launch of fewer units than the grid has waves hands out parts of
+// units, down to 4 entries, as long as there are waves to take them: such a
+// launch lasts as long as its slowest wave, and a wave of fewer rays takes
+// turns between fewer kinds of step (below, units and the cursor count
+// these parts). Whole units only: 1.3M-triangle mesh at 1920x1080x1 8.51
+// instead of 8.16 ms, primitives at 801x449x33 7.83 instead of 7.60 ms;
+// down to 8 or 16 entries: in between.
+//
+// Every wave's first units are its own share by its place in the grid; the
+// cursor hands out what follows them. A launch with no more than that
+// takes no atomic at all (one per wave, only to learn that nothing is
+// left, cost a launch of 5120 waves 60 us: a 256x256x1 Cornell frame spent
+// 2.0 of 2.2 ms in such launches).
+// ---------------------------------------------------------------------------
+struct Units {
+  uint32_t* cursor;
+  uint32_t split;          // log2 of the parts a unit is handed out in
+  uint32_t total, dealt;   // units of the launch; of these, given out by place
+  uint32_t parts;          // a fetch takes what is left over `parts`
+  uint32_t seen;           // the first unit of this wave's last fetch
+  uint32_t cur, end;       // fetched units not yet taken
+  bool exhausted;
+  __device__ __forceinline__ static uint32_t fetch_size(uint32_t left, uint32_t parts) {
+    return max(1u, min(16u, left / parts));
+  }
+  __device__ __forceinline__ Units(uint32_t* cursor_, uint32_t units, uint32_t batch_units) : cursor(cursor_) {
+    const uint32_t waves = gridDim.x * (blockDim.x >> 6);
+    parts = (batch_units < 64u * waves ? 2u : 4u) * waves;
+    split = 0;
+    while (split < 4u && (units << (split + 1u)) <= waves) ++split;
+    total = units << split;
+    const uint32_t mine = fetch_size(total, parts);
+    dealt = mine * waves;
+    seen = (blockIdx.x * (blockDim.x >> 6) + static_cast<uint32_t>(uniform(static_cast<int>(threadIdx.x >> 6)))) * mine;
+    cur = min(seen, total);
+    end = min(seen + mine, total);
+    exhausted = dealt >= total;
+  }
+  __device__ __forceinline__ void fetch() {
+    const uint32_t per = fetch_size(total - seen, parts);
+    uint32_t u = 0;
+    if (lane_id() == 0) u = atomicAdd(cursor, per);
+    u = dealt + static_cast<uint32_t>(uniform(static_cast<int>(__shfl(u, 0))));
+    if (u >= total) {
+      exhausted = true;
+    } else {
+      cur = u;
+      end = min(u + per, total);
+      seen = u;
+    }
+  }
+};
+
+// ---------------------------------------------------------------------------
 // Persistent traversal of one queue with per-lane refill. Waves take
-// 64-entry units from a device cursor into a wave-local pool; a lane whose
+// units into a wave-local pool; a lane whose
 // ray is finished takes the next pool entry at once, so a wave keeps all
 // lanes busy until the queue runs dry instead of waiting for its slowest
 // ray. A unit lies in one chunk; the rays in flight in a wave always share
 // one job (and scene): a unit of another job waits until the wave drains.
+// The queue's units are [lo, hi) of the launch's (in parts); returns once
+// this wave has none left in that range, with its walks finished.
 // seg: queue entries per chunk sample slot (1 path queue, 2 shadow queue).
 // kSort: the pool is all fetched units of one chunk (up to 16, 1024 rays)
 // at once, ordered by the direction octant of their rays (bits 1-3 of
@@ -82,14 +154,8 @@ __global__ void __launch_bounds__(256) k_raygen(WaveBuffers B) {
 // changes no ray's result.
 // Must be reached by every lane of the wave.
 // ---------------------------------------------------------------------------
-// Units a wave takes at once when `left` are left: what is left over
-// `parts`, 1 to 16.
-__device__ __forceinline__ uint32_t fetch_size(uint32_t left, uint32_t parts) {
-  return max(1u, min(16u, left / parts));
-}
-
-template <bool kAny, bool kCount, bool kPrims, bool kSort, class Load, class Finish>
-__device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchView& v, uint32_t* cursor,
+template <bool kAny, bool kCount, bool kPrims, bool kSort, class View, class Load, class Finish>
+__device__ __forceinline__ void trace_queue(const WaveBuffers& B, const View& v, Units& un, uint32_t lo, uint32_t hi,
                                             uint32_t seg, TravStack& st, TravCount& c, uint32_t& rays,
                                             bool& overflow, const float4* ray1, uint16_t* slist, uint32_t* sbase,
                                             Load load, Finish finish) {
@@ -101,41 +167,7 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchVie
   w.idle(st);
   uint32_t pbase = 0, pnext = 0, pend = 0;   // wave-uniform pool: entries pbase + [pnext, pend) of chunk pci
   int pci = 0;
-  // Units are taken from the cursor several at a time: one global atomic
-  // on one address serves only ~85 M operations per second on the whole
-  // device, so a fetch per 64-entry unit capped a launch at ~5 G rays/s.
-  // A fetch takes up to 16 units, fewer as the queue runs out (what is left
-  // per 4 waves of the grid, as this wave last saw it), so the launch
-  // does not end with a few waves walking long private batches. Batches of
-  // fewer than 64 units per wave (a 512x512 frame at 64 samples on the
-  // whole device) walk short queues at every depth: there the fetches'
-  // own cost outweighs the balance at the end of a launch, and a fetch
-  // takes up to twice as much (what is left per 2 waves).
-  const uint32_t gwaves = gridDim.x * (blockDim.x >> 6);
-  const uint32_t batch_units =
-      v.nch > 0 ? static_cast<uint32_t>(v.ch[v.nch - 1].base + v.ch[v.nch - 1].cap) >> 6 : 0u;
-  const uint32_t share = batch_units < 64u * gwaves ? 2u : 4u;
-  // A launch of fewer units than the grid has waves hands out parts of
-  // units, down to 4 entries, as long as there are waves to take them: such a
-  // launch lasts as long as its slowest wave, and a wave of fewer rays takes
-  // turns between fewer kinds of step (below, units and the cursor count
-  // these parts). Whole units only: 1.3M-triangle mesh at 1920x1080x1 8.51
-  // instead of 8.16 ms, primitives at 801x449x33 7.83 instead of 7.60 ms;
-  // down to 8 or 16 entries: in between.
-  uint32_t split = 0;
-  while (split < 4u && (v.prefix[v.nch] << (split + 1u)) <= gwaves) ++split;
-  const uint32_t part = 64u >> split, pmask = (1u << split) - 1u;
-  const uint32_t total = v.prefix[v.nch] << split;
-  // Every wave's first units are its own share by its place in the grid; the
-  // cursor hands out what follows them. A launch with no more than that
-  // takes no atomic at all (one per wave, only to learn that nothing is
-  // left, cost a launch of 5120 waves 60 us: a 256x256x1 Cornell frame spent
-  // 2.0 of 2.2 ms in such launches and takes 0.75 ms now).
-  const uint32_t first_units = fetch_size(total, share * gwaves);
-  const uint32_t dealt = first_units * gwaves;
-  uint32_t seen = (blockIdx.x * (blockDim.x >> 6) + static_cast<uint32_t>(uniform(static_cast<int>(threadIdx.x >> 6)))) * first_units;
-  uint32_t ucur = min(seen, total), uend = min(seen + first_units, total);   // fetched units not yet taken (wave-uniform)
-  bool exhausted = dealt >= total;
+  const uint32_t part = 64u >> un.split, pmask = (1u << un.split) - 1u;
   bool stuck = false;
   for (uint32_t guard = 0;; ++guard) {
     if (guard >= kWaveStepLimit) {
@@ -145,29 +177,19 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchVie
     const unsigned long long act = __ballot(my != kIdle);
     if (act != ~0ull) {
       if (pnext >= pend) {
-        if (ucur >= uend && !exhausted) {
-          const uint32_t per = fetch_size(total - seen, share * gwaves);
-          uint32_t u0 = 0;
-          if (lane == 0) u0 = atomicAdd(cursor, per);
-          u0 = dealt + static_cast<uint32_t>(uniform(static_cast<int>(__shfl(u0, 0))));
-          if (u0 >= total) {
-            exhausted = true;
-          } else {
-            ucur = u0;
-            uend = min(u0 + per, total);
-            seen = u0;
-          }
-        }
-        if (ucur < uend) {
+        if (un.cur >= un.end && !un.exhausted) un.fetch();
+        const uint32_t stop = min(un.end, hi);
+        if (un.cur < stop) {
+          const uint32_t ucur = un.cur - lo, uend = stop - lo;   // within the queue
           // a unit of another job waits until the wave has drained (the
           // rays in flight in a wave share one scene)
-          const int ci = uniform(find_chunk(v, ucur >> split));
+          const int ci = uniform(find_chunk(v, ucur >> un.split));
           if (act == 0ull || v.ch[ci].job == v.ch[pci].job) {
             pci = ci;
             if constexpr (kSort) {
               // the fetched units that lie in this chunk (1 to 16), keyed by
               // octant (4 bits per unit and lane; 8 = no entry)
-              const uint32_t n = min(uend, v.prefix[ci + 1] << split) - ucur;
+              const uint32_t n = min(uend, v.prefix[ci + 1] << un.split) - ucur;
               uint32_t keys0 = 0u, keys1 = 0u;
               // every lane has taken its entry of the last pool before the
               // order is rewritten
@@ -176,7 +198,7 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchVie
               __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
               for (uint32_t j = 0; j < n; ++j) {
                 uint32_t first, lim;
-                uint32_t b = unit_segment(v, ci, ((ucur + j) >> split) - v.prefix[ci], seg, first, lim);
+                uint32_t b = unit_segment(v, ci, ((ucur + j) >> un.split) - v.prefix[ci], seg, first, lim);
                 first += ((ucur + j) & pmask) * part;
                 b += first;
                 const uint32_t cnt = lim > first ? min(part, lim - first) : 0u;
@@ -203,13 +225,13 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchVie
               __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
               pnext = 0;
               pend = pos;
-              ucur += n;
+              un.cur += n;
             } else {
               uint32_t first, lim;
-              pbase = unit_segment(v, ci, (ucur >> split) - v.prefix[ci], seg, first, lim);
+              pbase = unit_segment(v, ci, (ucur >> un.split) - v.prefix[ci], seg, first, lim);
               pnext = first + (ucur & pmask) * part;
               pend = min(pnext + part, lim);   // none past the segment's last entry
-              ++ucur;
+              ++un.cur;
             }
           }
         }
@@ -235,7 +257,7 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchVie
     }
     // (a part of a segment's last unit may hold no entry: a wave without rays
     // goes on while it has units; its step below does nothing)
-    if (exhausted && ucur >= uend && __ballot(my != kIdle) == 0ull) break;
+    if ((un.cur >= hi || (un.exhausted && un.cur >= un.end)) && __ballot(my != kIdle) == 0ull) break;
     if (kCount && lane == 0) ++c.round_iters;
     if (kCount && my != kIdle) ++c.round_lanes;
     const DevScene& S = job_scene(B.jobs, uniform(v.ch[pci].job));
@@ -251,60 +273,113 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const BatchVie
 }
 
 // ---------------------------------------------------------------------------
-// closest: persistent closest-hit traversal of queue qi (kCount: with the
-// traversal work counters; kCamera: depth 0, whose rays are the chunks'
-// camera rays, rebuilt from the entry index).
+// camera: closest hits of depth 0, whose rays are the chunks' camera rays,
+// rebuilt from the entry index (kCount: with the traversal work counters).
 // ---------------------------------------------------------------------------
-// Per-wave LDS of the octant-ordered pool (bounce rays only).
-template <bool kOn>
-struct SortPool {
-  uint16_t list[256 / 64][16 * 64];
-  uint32_t base[256 / 64][16];
-};
-template <>
-struct SortPool<false> {
-  uint16_t list[1][1];
-  uint32_t base[1][1];
-};
+template <class Walk>
+__device__ __forceinline__ void store_hit(const WaveBuffers& B, uint32_t i, const Walk& w) {
+  B.hit[i] = make_float4(w.found() ? w.tbest : 0.f, w.hit.u, w.hit.v, __int_as_float(w.hit.inst));
+  B.hit_slot[i] = w.hit.slot;
+}
 
-template <bool kCount, bool kPrims, bool kCamera>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kCount ? 4 : 5))) k_closest(WaveBuffers B, int qi, int cursor, int lds_depth) {
+template <bool kCount, bool kPrims>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kCount ? 4 : 5))) k_camera(WaveBuffers B, int cursor, int lds_depth) {
   __shared__ BatchView v;
-  __shared__ SortPool<!kCamera> sp;
-  const uint32_t* counts = B.counters + ctr_path(qi, 0, 0);
-  load_batch(v, B, counts, false);
-  if (blockIdx.x == 0)
-    for (int t = static_cast<int>(threadIdx.x); t < v.nch * kQSeg; t += static_cast<int>(blockDim.x)) {
-      B.counters[ctr_path(1 - qi, t / kQSeg, t % kQSeg)] = 0u;
-      B.counters[ctr_shadow(t / kQSeg, t % kQSeg)] = 0u;
-    }
-  const PathQueue q = B.q[qi];
+  load_batch(v, B, B.counters + ctr_path(0, 0, 0), false);
   TravStack st = make_stack(B.spill, lds_depth);
   TravCount c{0, 0, 0, 0};
   uint32_t rays = 0;
   bool overflow = false;
-  const uint32_t wv = kCamera ? 0u : threadIdx.x >> 6;
-  trace_queue<false, kCount, kPrims, !kCamera>(
-      B, v, &B.counters[kCursor + cursor], 1u, st, c, rays, overflow, q.ray1, sp.list[wv], sp.base[wv],
+  const uint32_t units = v.prefix[v.nch];
+  Units un(&B.counters[kCursor + cursor], units,
+           v.nch > 0 ? static_cast<uint32_t>(v.ch[v.nch - 1].base + v.ch[v.nch - 1].cap) >> 6 : 0u);
+  trace_queue<false, kCount, kPrims, false>(
+      B, v, un, 0u, un.total, 1u, st, c, rays, overflow, nullptr, nullptr, nullptr,
       [&](uint32_t i, int ci, f3& o, f3& d, float& tmin, float& tmax) {
-        if constexpr (kCamera) {
-          const DevChunk& ck = v.ch[ci];
-          const CameraPath p = camera_path(ck, job_rec(B.jobs, uniform(ck.job)), i);
-          o = p.o;
-          d = p.d;
-        } else {
-          const float4 r0 = q.ray0[i], r1 = q.ray1[i];
-          o = f3{r0.x, r0.y, r0.z};
-          d = f3{r0.w, r1.x, r1.y};
-        }
+        const DevChunk& ck = v.ch[ci];
+        const CameraPath p = camera_path(ck, job_rec(B.jobs, uniform(ck.job)), i);
+        o = p.o;
+        d = p.d;
         tmin = kBounceOffset;
         tmax = __builtin_huge_valf();
       },
-      [&](uint32_t i, const Walker<false, kCount, kPrims>& w) {
-        B.hit[i] = make_float4(w.found() ? w.tbest : 0.f, w.hit.u, w.hit.v, __int_as_float(w.hit.inst));
-        B.hit_slot[i] = w.hit.slot;
+      [&](uint32_t i, const Walker<false, kCount, kPrims>& w) { store_hit(B, i, w); });
+  flush_counts_block<kCount>(B.stats, v.cnt, v.nch, c, rays, false);
+  if (overflow) atomicAdd(&B.counters[kOverflow], 1u);
+}
+
+// ---------------------------------------------------------------------------
+// trace: the closest hits of path queue qi (depth >= 1) and the shadow rays
+// of the depth before (counter set 1 - sh_next), whose unoccluded
+// contributions are added to their path's per-slot NEE sum (one writer per
+// (slot, light kind)). The two are independent, and each alone ends with a
+// tail, the longest walks of its queue on a few waves; walked in one launch,
+// the shadow rays fill the closest hits' tail and one tail is left.
+// Against one launch each: 256x256x1 Cornell frame 0.73 -> 0.59 ms,
+// 1920x1080x1 mesh frame 8.1 -> 6.9 ms, primitives 801x449x33 7.65 -> 6.87 ms,
+// Cornell 512x512x64 13.3 -> 12.6 ms, mesh 1920x1080x256 268 -> 264 ms.
+// Clears the counters the shading of this depth appends to (path queue
+// 1 - qi, shadow set sh_next). `what`: kTraceClosest | kTraceShadow (one
+// alone after the last depth, and where the two are timed apart).
+// ---------------------------------------------------------------------------
+// Per-wave LDS of the octant-ordered pool.
+struct SortPool {
+  uint16_t list[256 / 64][16 * 64];
+  uint32_t base[256 / 64][16];
+};
+
+template <bool kCount, bool kPrims>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kCount ? 4 : 5))) k_trace(WaveBuffers B, int qi, int sh_next, int what, int cursor, int lds_depth) {
+  __shared__ TraceView v;
+  __shared__ SortPool sp;
+  load_trace(v, B, (what & kTraceClosest) ? B.counters + ctr_path(qi, 0, 0) : nullptr,
+             (what & kTraceShadow) ? B.counters + ctr_shadow(1 - sh_next, 0, 0) : nullptr);
+  if (blockIdx.x == 0 && (what & kTraceClosest))
+    for (int t = static_cast<int>(threadIdx.x); t < v.nch * kQSeg; t += static_cast<int>(blockDim.x)) {
+      B.counters[ctr_path(1 - qi, t / kQSeg, t % kQSeg)] = 0u;
+      B.counters[ctr_shadow(sh_next, t / kQSeg, t % kQSeg)] = 0u;
+    }
+  const PathQueue q = B.q[qi];
+  TravStack st = make_stack(B.spill, lds_depth);
+  TravCount c{0, 0, 0, 0}, cs{0, 0, 0, 0};
+  uint32_t rays = 0, shadow_rays = 0;
+  bool overflow = false;
+  const uint32_t wv = threadIdx.x >> 6;
+  const TraceUnits vp(v, 0), vs(v, 1);
+  Units un(&B.counters[kCursor + cursor], vp.prefix[v.nch] + vs.prefix[v.nch], v.batch_units);
+  const uint32_t mid = vp.prefix[v.nch] << un.split;
+  trace_queue<false, kCount, kPrims, true>(
+      B, vp, un, 0u, mid, 1u, st, c, rays, overflow, q.ray1, sp.list[wv], sp.base[wv],
+      [&](uint32_t i, int, f3& o, f3& d, float& tmin, float& tmax) {
+        const float4 r0 = q.ray0[i], r1 = q.ray1[i];
+        o = f3{r0.x, r0.y, r0.z};
+        d = f3{r0.w, r1.x, r1.y};
+        tmin = kBounceOffset;
+        tmax = __builtin_huge_valf();
+      },
+      [&](uint32_t i, const Walker<false, kCount, kPrims>& w) { store_hit(B, i, w); });
+  trace_queue<true, kCount, kPrims, false>(
+      B, vs, un, mid, un.total, 2u, st, cs, shadow_rays, overflow, nullptr, nullptr, nullptr,
+      [&](uint32_t i, int, f3& o, f3& d, float& tmin, float& tmax) {
+        const float4 r0 = B.sh0[i], r1 = B.sh1[i];
+        o = f3{r0.x, r0.y, r0.z};
+        d = f3{r0.w, r1.x, r1.y};
+        tmin = kShadowOff;
+        tmax = r1.z;
+      },
+      [&](uint32_t i, const Walker<true, kCount, kPrims>& w) {
+        if (!w.found()) {
+          const uint32_t k = __float_as_uint(B.sh1[i].w);
+          const float4 cv = B.sh_c[i];
+          float4 acc = B.l_nee[k];
+          acc.x = acc.x + cv.x;
+          acc.y = acc.y + cv.y;
+          acc.z = acc.z + cv.z;
+          B.l_nee[k] = acc;
+        }
       });
-  flush_counts_block<kCount>(B.stats, v, c, rays, false);
+  flush_counts_block<kCount>(B.stats, v.q[0].cnt, v.nch, c, rays, false);
+  flush_counts_block<kCount>(B.stats, v.q[1].cnt, v.nch, cs, shadow_rays, true);
   if (overflow) atomicAdd(&B.counters[kOverflow], 1u);
 }
 
@@ -663,7 +738,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGuide
     // queue
     const uint32_t xs = blockIdx.x % kQSeg;
     uint32_t ia, is, in;
-    wave_append_pass(&B.counters[ctr_shadow(ci, static_cast<int>(xs))], want_a, want_s, ia, is,
+    wave_append_pass(&B.counters[ctr_shadow(depth & 1, ci, static_cast<int>(xs))], want_a, want_s, ia, is,
                      &B.counters[ctr_path(1 - qi, ci, static_cast<int>(xs))], want_n, in);
     {
       // a segment holds what its group can append (kSegSlack); an append
@@ -704,43 +779,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGuide
     // every lane has read its positions before the next window writes them
     __builtin_amdgcn_wave_barrier();
   }
-}
-
-// ---------------------------------------------------------------------------
-// shadow: persistent any-hit traversal; unoccluded contributions are added
-// to their path's per-slot NEE sum (one writer per (slot, light kind)).
-// ---------------------------------------------------------------------------
-template <bool kCount, bool kPrims>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kCount ? 4 : 5))) k_shadow(WaveBuffers B, int cursor, int lds_depth) {
-  __shared__ BatchView v;
-  const uint32_t* counts = B.counters + ctr_shadow(0, 0);
-  load_batch(v, B, counts, false, 2u);
-  TravStack st = make_stack(B.spill, lds_depth);
-  TravCount c{0, 0, 0, 0};
-  uint32_t rays = 0;
-  bool overflow = false;
-  trace_queue<true, kCount, kPrims, false>(
-      B, v, &B.counters[kCursor + cursor], 2u, st, c, rays, overflow, nullptr, nullptr, nullptr,
-      [&](uint32_t i, int, f3& o, f3& d, float& tmin, float& tmax) {
-        const float4 r0 = B.sh0[i], r1 = B.sh1[i];
-        o = f3{r0.x, r0.y, r0.z};
-        d = f3{r0.w, r1.x, r1.y};
-        tmin = kShadowOff;
-        tmax = r1.z;
-      },
-      [&](uint32_t i, const Walker<true, kCount, kPrims>& w) {
-        if (!w.found()) {
-          const uint32_t k = __float_as_uint(B.sh1[i].w);
-          const float4 cv = B.sh_c[i];
-          float4 acc = B.l_nee[k];
-          acc.x = acc.x + cv.x;
-          acc.y = acc.y + cv.y;
-          acc.z = acc.z + cv.z;
-          B.l_nee[k] = acc;
-        }
-      });
-  flush_counts_block<kCount>(B.stats, v, c, rays, true);
-  if (overflow) atomicAdd(&B.counters[kOverflow], 1u);
 }
 
 // ---------------------------------------------------------------------------
@@ -892,7 +930,7 @@ int trace_grid(int block, int lds_depth) {
   if (hipGetDeviceProperties(&prop, dev) != hipSuccess) return -1;
   int per_cu = 0;
   const size_t lds = static_cast<size_t>(block) * lds_depth * sizeof(uint32_t);
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(k_closest<false, false, false>), block, lds) !=
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(k_trace<false, false>), block, lds) !=
       hipSuccess)
     return -1;
   if (per_cu < 1) per_cu = 1;
@@ -916,25 +954,21 @@ hipError_t launch_raygen(hipStream_t s, const WaveBuffers& B, int max_paths) {
   return hipGetLastError();
 }
 
-template <bool kCount, bool kPrims>
-void launch_closest_kind(hipStream_t s, const WaveBuffers& B, int qi, int cursor, int grid, int block, int lds_depth,
-                         size_t lds, bool camera) {
-  if (camera)
-    hipLaunchKernelGGL((k_closest<kCount, kPrims, true>), dim3(grid), dim3(block), lds, s, B, qi, cursor, lds_depth);
-  else
-    hipLaunchKernelGGL((k_closest<kCount, kPrims, false>), dim3(grid), dim3(block), lds, s, B, qi, cursor, lds_depth);
+hipError_t launch_camera(hipStream_t s, const WaveBuffers& B, int cursor, int grid, int block, int lds_depth,
+                         bool count, bool prims) {
+  const size_t lds = static_cast<size_t>(block) * lds_depth * 4;
+  const auto k = prims ? (count ? k_camera<true, true> : k_camera<false, true>)
+                       : (count ? k_camera<true, false> : k_camera<false, false>);
+  hipLaunchKernelGGL(k, dim3(grid), dim3(block), lds, s, B, cursor, lds_depth);
+  return hipGetLastError();
 }
 
-hipError_t launch_closest(hipStream_t s, const WaveBuffers& B, int qi, int cursor, int grid, int block,
-                          int lds_depth, bool count, bool prims, bool camera) {
+hipError_t launch_trace(hipStream_t s, const WaveBuffers& B, int depth, int what, int cursor, int grid, int block,
+                        int lds_depth, bool count, bool prims) {
   const size_t lds = static_cast<size_t>(block) * lds_depth * 4;
-  if (prims) {
-    if (count) launch_closest_kind<true, true>(s, B, qi, cursor, grid, block, lds_depth, lds, camera);
-    else launch_closest_kind<false, true>(s, B, qi, cursor, grid, block, lds_depth, lds, camera);
-  } else {
-    if (count) launch_closest_kind<true, false>(s, B, qi, cursor, grid, block, lds_depth, lds, camera);
-    else launch_closest_kind<false, false>(s, B, qi, cursor, grid, block, lds_depth, lds, camera);
-  }
+  const auto k = prims ? (count ? k_trace<true, true> : k_trace<false, true>)
+                       : (count ? k_trace<true, false> : k_trace<false, false>);
+  hipLaunchKernelGGL(k, dim3(grid), dim3(block), lds, s, B, depth & 1, depth & 1, what, cursor, lds_depth);
   return hipGetLastError();
 }
 
@@ -945,19 +979,6 @@ hipError_t launch_closest(hipStream_t s, const WaveBuffers& B, int qi, int curso
 hipError_t launch_shade(hipStream_t s, const WaveBuffers& B, int qi, int depth, int grid) {
   if (B.guide_alpha > 0.f && depth <= B.guide_depth) hipLaunchKernelGGL(k_shade<true>, dim3(grid), dim3(256), 0, s, B, qi, depth);
   else hipLaunchKernelGGL(k_shade<false>, dim3(grid), dim3(256), 0, s, B, qi, depth);
-  return hipGetLastError();
-}
-
-hipError_t launch_shadow(hipStream_t s, const WaveBuffers& B, int cursor, int grid, int block, int lds_depth,
-                         bool count, bool prims) {
-  const size_t lds = static_cast<size_t>(block) * lds_depth * 4;
-  if (prims) {
-    if (count) hipLaunchKernelGGL((k_shadow<true, true>), dim3(grid), dim3(block), lds, s, B, cursor, lds_depth);
-    else hipLaunchKernelGGL((k_shadow<false, true>), dim3(grid), dim3(block), lds, s, B, cursor, lds_depth);
-  } else {
-    if (count) hipLaunchKernelGGL((k_shadow<true, false>), dim3(grid), dim3(block), lds, s, B, cursor, lds_depth);
-    else hipLaunchKernelGGL((k_shadow<false, false>), dim3(grid), dim3(block), lds, s, B, cursor, lds_depth);
-  }
   return hipGetLastError();
 }
 

@@ -13,12 +13,15 @@ int trace_grid(int block, int lds_depth);
 int num_cus();
 
 hipError_t launch_raygen(hipStream_t s, const WaveBuffers& B, int max_paths);
-// camera: depth 0 (the queue's rays are the chunks' camera rays)
-hipError_t launch_closest(hipStream_t s, const WaveBuffers& B, int qi, int cursor, int grid, int block,
-                          int lds_depth, bool count, bool prims, bool camera);
-hipError_t launch_shade(hipStream_t s, const WaveBuffers& B, int qi, int depth, int grid);
-hipError_t launch_shadow(hipStream_t s, const WaveBuffers& B, int cursor, int grid, int block, int lds_depth,
+// Closest hits of depth 0 (the chunks' camera rays).
+hipError_t launch_camera(hipStream_t s, const WaveBuffers& B, int cursor, int grid, int block, int lds_depth,
                          bool count, bool prims);
+// Closest hits of depth `depth` (path queue depth & 1) and the shadow rays of
+// depth - 1, or one of the two.
+constexpr int kTraceClosest = 1, kTraceShadow = 2;
+hipError_t launch_trace(hipStream_t s, const WaveBuffers& B, int depth, int what, int cursor, int grid, int block,
+                        int lds_depth, bool count, bool prims);
+hipError_t launch_shade(hipStream_t s, const WaveBuffers& B, int qi, int depth, int grid);
 hipError_t launch_accumulate(hipStream_t s, const WaveBuffers& B, int max_pixels);
 hipError_t launch_advance(hipStream_t s, uint32_t* counters);
 hipError_t launch_average(hipStream_t s, const float4* accum, float* out, int npix, float inv_spp);

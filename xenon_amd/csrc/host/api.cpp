@@ -7,7 +7,8 @@
 // contiguous sample range of one job per chunk), all chunk tables are
 // uploaded once, and each batch runs
 //
-//   raygen -> [closest(d) -> shade(d) -> shadow(d)] d < max depth -> accumulate -> advance
+//   raygen -> camera -> shade(0) -> [trace(d) -> shade(d)] 0 < d < max depth -> trace(last shadow rays)
+//          -> accumulate -> advance
 //
 // with no host read between kernels: every work count and the batch index
 // live in device memory, so the sequence is captured once as a hipGraph and
@@ -623,25 +624,32 @@ int ensure_tables(xnh_ctx* c, size_t njobs, size_t nbatches) {
   return XNH_OK;
 }
 
-// Enqueues one batch: the whole bounce loop for `depth` bounces.
+// Enqueues one batch: the whole bounce loop for `depth` bounces. Shadow rays
+// are walked with the next depth's closest hits, except with per-kernel
+// timing (ev), which walks and times them apart.
 int enqueue_batch(xnh_ctx* c, int depth, size_t* ev) {
   hipStream_t s = c->stream;
   const int cap = c->B.capacity;
   HIP_OR_FAIL(c, launch_raygen(s, c->B, cap));
+  auto mark = [&]() { return ev ? hipEventRecord(c->prof_events[(*ev)++], s) : hipSuccess; };
+  auto trace = [&](int d, int what, int cursor) {
+    return launch_trace(s, c->B, d, what, cursor, c->grid_trace, c->block, c->lds_depth, c->counting, c->prims);
+  };
   for (int d = 0; d < depth; ++d) {
-    const int qi = d & 1;
-    if (ev) HIP_OR_FAIL(c, hipEventRecord(c->prof_events[(*ev)++], s));
-    HIP_OR_FAIL(c, launch_closest(s, c->B, qi, 2 * d, c->grid_trace, c->block, c->lds_depth, c->counting, c->prims,
-                                  d == 0));
-    if (ev) HIP_OR_FAIL(c, hipEventRecord(c->prof_events[(*ev)++], s));
+    HIP_OR_FAIL(c, mark());
+    if (d == 0)
+      HIP_OR_FAIL(c, launch_camera(s, c->B, 0, c->grid_trace, c->block, c->lds_depth, c->counting, c->prims));
+    else
+      HIP_OR_FAIL(c, trace(d, ev ? kTraceClosest : kTraceClosest | kTraceShadow, 2 * d));
+    HIP_OR_FAIL(c, mark());
     if (c->guide.on && d < c->B.guide_depth)
-      HIP_OR_FAIL(c, launch_guide_infer(s, c->B, qi, d, c->guide.net, c->guide.feat, c->grid_shade * 2));
-    if (ev) HIP_OR_FAIL(c, hipEventRecord(c->prof_events[(*ev)++], s));
-    HIP_OR_FAIL(c, launch_shade(s, c->B, qi, d, c->grid_shade));
-    if (ev) HIP_OR_FAIL(c, hipEventRecord(c->prof_events[(*ev)++], s));
-    if (ev) HIP_OR_FAIL(c, hipEventRecord(c->prof_events[(*ev)++], s));
-    HIP_OR_FAIL(c, launch_shadow(s, c->B, 2 * d + 1, c->grid_trace, c->block, c->lds_depth, c->counting, c->prims));
-    if (ev) HIP_OR_FAIL(c, hipEventRecord(c->prof_events[(*ev)++], s));
+      HIP_OR_FAIL(c, launch_guide_infer(s, c->B, d & 1, d, c->guide.net, c->guide.feat, c->grid_shade * 2));
+    HIP_OR_FAIL(c, mark());
+    HIP_OR_FAIL(c, launch_shade(s, c->B, d & 1, d, c->grid_shade));
+    HIP_OR_FAIL(c, mark());
+    HIP_OR_FAIL(c, mark());
+    if (ev || d + 1 == depth) HIP_OR_FAIL(c, trace(d + 1, kTraceShadow, 2 * d + 1));
+    HIP_OR_FAIL(c, mark());
   }
   HIP_OR_FAIL(c, launch_accumulate(s, c->B, cap));
   HIP_OR_FAIL(c, launch_advance(s, c->B.counters));
