@@ -6,8 +6,8 @@
 // triangle indices (rocPRIM's radix sort; ties keep index order), and every
 // internal node of the binary radix tree over the sorted codes is found
 // independently from the longest common prefixes of its neighbours (equal
-// codes are told apart by their positions). Subtree sizes come bottom-up,
-// then every node's place in the output is computed from its ancestors so
+// codes are told apart by their positions). A node's subtree size follows
+// from its key range, and every node's place in the output from its ancestors, so
 // that the tree has the reference's node format (blas.h:21-28): 32-byte
 // nodes, the two children of a node adjacent (right = left + 1) and after
 // it, pairs starting at odd indices (64-byte aligned after the upload's
@@ -16,8 +16,10 @@
 // Refit: boxes of any tree in that format for moved vertices: each leaf
 // takes the bounds of its triangles, and each interior node takes the union
 // of its children once both are done (the second child to arrive computes
-// it, ordered by an atomic counter per node and agent-scope fences, since
-// the eight XCDs' L2 caches are not coherent with each other).
+// it, ordered by an atomic counter per node). The eight XCDs' L2 caches are
+// not coherent with each other, so boxes pass between the threads by
+// agent-scope atomic stores and loads, which go past them; a thread waits for
+// its own stores to be acknowledged before it counts itself in.
 //
 // Every walk is bounded and every computed index is checked before it is
 // used; a violation sets the error word instead of touching memory.
@@ -90,14 +92,19 @@ __global__ void __launch_bounds__(kT) k_lb_centres(const float* vx, const float*
   if (threadIdx.x < 6) pb[6 * blockIdx.x + threadIdx.x] = red[threadIdx.x][0];
 }
 
-// The centres' bounds from the per-block bounds (one block).
-__global__ void __launch_bounds__(64) k_lb_bounds(const float* pb, int nb, float* bounds) {
-  if (threadIdx.x < 6) {
-    const bool lo = threadIdx.x < 3;
-    float v = lo ? __builtin_huge_valf() : -__builtin_huge_valf();
-    for (int k = 0; k < nb; ++k) v = lo ? fminf(v, pb[6 * k + threadIdx.x]) : fmaxf(v, pb[6 * k + threadIdx.x]);
-    bounds[threadIdx.x] = v;
+// The centres' bounds from the per-block bounds: one wave per bound, work-group
+// of six (one thread per bound read 1024 blocks' values one after the other,
+// 100 us).
+__global__ void __launch_bounds__(64 * 6) k_lb_bounds(const float* pb, int nb, float* bounds) {
+  const int w = static_cast<int>(threadIdx.x >> 6), lane = static_cast<int>(threadIdx.x & 63u);
+  const bool lo = w < 3;
+  float v = lo ? __builtin_huge_valf() : -__builtin_huge_valf();
+  for (int k = lane; k < nb; k += 64) v = lo ? fminf(v, pb[6 * k + w]) : fmaxf(v, pb[6 * k + w]);
+  for (int o = 32; o > 0; o >>= 1) {
+    const float t = __shfl_xor(v, o);
+    v = lo ? fminf(v, t) : fmaxf(v, t);
   }
+  if (lane == 0) bounds[w] = v;
 }
 
 // Morton code of each centre within the centres' bounds.
@@ -126,10 +133,11 @@ __device__ __forceinline__ int lcp(const uint32_t* keys, int n, int a, long long
 }
 
 // Internal node i of the radix tree (Karras 2012, fig. 4): its key range
-// [i, j] or [j, i], the split gamma, the two children. Node ids: internal
+// [i, j] or [j, i], the split gamma, the two children, and the nodes of its
+// subtree (a range of m leaves has 2m - 1). Node ids: internal
 // 0..n-2 (0 is the root), leaf k is n-1+k.
 __global__ void __launch_bounds__(kT) k_lb_radix(const uint32_t* keys, int n, uint32_t* left, uint32_t* right,
-                                                 uint32_t* parent, uint32_t* err) {
+                                                 uint32_t* parent, uint32_t* size, uint32_t* err) {
   const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
   if (i >= n - 1) return;
   const int d = lcp(keys, n, i, i + 1) - lcp(keys, n, i, i - 1) >= 0 ? 1 : -1;
@@ -156,39 +164,9 @@ __global__ void __launch_bounds__(kT) k_lb_radix(const uint32_t* keys, int n, ui
   const uint32_t b = hi == gamma + 1 ? static_cast<uint32_t>(n + gamma) : static_cast<uint32_t>(gamma + 1);
   left[i] = a;
   right[i] = b;
+  size[i] = static_cast<uint32_t>(2 * (hi - lo) + 1);
   parent[a] = static_cast<uint32_t>(i);
   parent[b] = static_cast<uint32_t>(i);
-}
-
-// Subtree sizes, bottom-up: the second child to reach a node sums it.
-__global__ void __launch_bounds__(kT) k_lb_sizes(int n, const uint32_t* left, const uint32_t* right,
-                                                 const uint32_t* parent, uint32_t* size, uint32_t* flag,
-                                                 uint32_t* err) {
-  const int k = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
-  if (k >= n) return;
-  const uint32_t nn = static_cast<uint32_t>(2 * n - 1);
-  uint32_t x = static_cast<uint32_t>(n - 1 + k);
-  size[x] = 1u;
-  for (int step = 0; step < kMaxWalk; ++step) {
-    const uint32_t p = parent[x];
-    if (p >= static_cast<uint32_t>(n - 1)) {
-      if (x != 0u) atomicOr(err, 2u);
-      return;
-    }
-    __threadfence();
-    if (atomicAdd(&flag[p], 1u) == 0u) return;
-    __threadfence();
-    const uint32_t a = left[p], b = right[p];
-    if (a >= nn || b >= nn) {
-      atomicOr(err, 2u);
-      return;
-    }
-    size[p] = 1u + __hip_atomic_load(&size[a], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) +
-              __hip_atomic_load(&size[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (p == 0u) return;
-    x = p;
-  }
-  atomicOr(err, 4u);
 }
 
 // Output index of every node: root 0; a node's children pair opens the
@@ -218,7 +196,11 @@ __global__ void __launch_bounds__(kT) k_lb_place(int n, const uint32_t* left, co
       atomicOr(err, 8u);
       return;
     }
-    acc += 2u + (right[pa] == a ? size[left[pa]] - 1u : 0u);
+    acc += 2u;
+    if (right[pa] == a) {   // past the left sibling's descendants (none of a leaf)
+      const uint32_t l = left[pa];
+      if (l < static_cast<uint32_t>(n - 1)) acc += size[l] - 1u;
+    }
     a = pa;
   }
   if (a != 0u || acc >= static_cast<uint64_t>(nn)) {
@@ -277,7 +259,42 @@ __global__ void __launch_bounds__(kT) k_rf_parents(const xnh_bvh_node* nodes, in
   }
 }
 
-// Leaf boxes from the vertices, then unions up to the root.
+// A node's box as the three 8-byte words it occupies, past the L2 caches.
+struct BoxWords {
+  unsigned long long w[3];
+};
+__device__ __forceinline__ void store_box(xnh_bvh_node* v, const float* lo, const float* hi) {
+  const float f[6] = {lo[0], lo[1], lo[2], hi[0], hi[1], hi[2]};
+  BoxWords b;
+  __builtin_memcpy(&b, f, sizeof b);
+  unsigned long long* p = reinterpret_cast<unsigned long long*>(v);
+  for (int k = 0; k < 3; ++k) __hip_atomic_store(p + k, b.w[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void load_box(const xnh_bvh_node* v, float* lo, float* hi) {
+  const unsigned long long* p = reinterpret_cast<const unsigned long long*>(v);
+  BoxWords b;
+  for (int k = 0; k < 3; ++k) b.w[k] = __hip_atomic_load(p + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  float f[6];
+  __builtin_memcpy(f, &b, sizeof b);
+  for (int k = 0; k < 3; ++k) {
+    lo[k] = f[k];
+    hi[k] = f[3 + k];
+  }
+}
+
+// Waits until this wave's stores have been acknowledged (vmcnt 0); the
+// wavefront fences keep the compiler from moving accesses across it.
+__device__ __forceinline__ void stores_done() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_s_waitcnt(0x0F70);   // vmcnt(0), the other counters not waited for
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Leaf boxes from the vertices, then unions up to the root: a thread carries
+// its node's box and reads only the sibling's. Bound by the chain of
+// dependent atomics and loads up the tree. Agent-scope fences instead (two a
+// level, each writing back and invalidating the XCD's whole L2) took 3450 us
+// for 300,000 triangles.
 __global__ void __launch_bounds__(kT) k_rf_boxes(xnh_bvh_node* nodes, int nn, const uint32_t* prims, int nprims,
                                                  const float* vx, const float* vy, const float* vz,
                                                  const int32_t* idx, const uint32_t* parent, uint32_t* flag,
@@ -300,10 +317,7 @@ __global__ void __launch_bounds__(kT) k_rf_boxes(xnh_bvh_node* nodes, int nn, co
       hi[k] = fmaxf(hi[k], b[k]);
     }
   }
-  for (int k = 0; k < 3; ++k) {
-    v->lo[k] = lo[k];
-    v->hi[k] = hi[k];
-  }
+  store_box(v, lo, hi);
   uint32_t x = static_cast<uint32_t>(j);
   for (int step = 0; step < kMaxWalk; ++step) {
     const uint32_t p = parent[x];
@@ -312,31 +326,22 @@ __global__ void __launch_bounds__(kT) k_rf_boxes(xnh_bvh_node* nodes, int nn, co
       atomicOr(err, 32u);
       return;
     }
-    __threadfence();
+    stores_done();
     if (atomicAdd(&flag[p], 1u) == 0u) return;
-    __threadfence();
     xnh_bvh_node* P = &nodes[p];
     const uint32_t c = P->child;
-    if (P->count != 0u || c + 1u >= static_cast<uint32_t>(nn)) {
+    if (P->count != 0u || c + 1u >= static_cast<uint32_t>(nn) || (x != c && x != c + 1u)) {
       atomicOr(err, 32u);
       return;
     }
-    const float* l0 = nodes[c].lo;
-    const float* h0 = nodes[c].hi;
-    const float* l1 = nodes[c + 1].lo;
-    const float* h1 = nodes[c + 1].hi;
+    float l2[3], h2[3];
+    load_box(&nodes[x == c ? c + 1u : c], l2, h2);
     for (int k = 0; k < 3; ++k) {
-      const float a0 = __uint_as_float(__hip_atomic_load(reinterpret_cast<const uint32_t*>(l0 + k), __ATOMIC_RELAXED,
-                                                         __HIP_MEMORY_SCOPE_AGENT));
-      const float a1 = __uint_as_float(__hip_atomic_load(reinterpret_cast<const uint32_t*>(l1 + k), __ATOMIC_RELAXED,
-                                                         __HIP_MEMORY_SCOPE_AGENT));
-      const float b0 = __uint_as_float(__hip_atomic_load(reinterpret_cast<const uint32_t*>(h0 + k), __ATOMIC_RELAXED,
-                                                         __HIP_MEMORY_SCOPE_AGENT));
-      const float b1 = __uint_as_float(__hip_atomic_load(reinterpret_cast<const uint32_t*>(h1 + k), __ATOMIC_RELAXED,
-                                                         __HIP_MEMORY_SCOPE_AGENT));
-      P->lo[k] = fminf(a0, a1);
-      P->hi[k] = fmaxf(b0, b1);
+      // left child's value first
+      lo[k] = x == c ? fminf(lo[k], l2[k]) : fminf(l2[k], lo[k]);
+      hi[k] = x == c ? fmaxf(hi[k], h2[k]) : fmaxf(h2[k], hi[k]);
     }
+    store_box(P, lo, hi);
     x = p;
   }
   atomicOr(err, 64u);
@@ -382,24 +387,22 @@ hipError_t build_blas_device(hipStream_t s, const float* vx, const float* vy, co
   uint32_t* left = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * n));
   uint32_t* right = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * n));
   uint32_t* parent = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * nn));
-  uint32_t* size = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * nn));
+  uint32_t* size = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * n));
   uint32_t* flag = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * nn));
   uint32_t* pos = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * nn));
   size_t tmp_bytes = 0;
   if (e == hipSuccess) e = rocprim::radix_sort_pairs(nullptr, tmp_bytes, k0, k1, v0, v1, static_cast<size_t>(n), 0, 30, s);
   void* tmp = alloc(tmp_bytes);
   if (e == hipSuccess) e = hipMemsetAsync(parent, 0xFF, sizeof(uint32_t) * nn, s);
-  if (e == hipSuccess) e = hipMemsetAsync(flag, 0, sizeof(uint32_t) * nn, s);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_lb_centres, dim3(nb), dim3(kT), 0, s, vx, vy, vz, idx, n, cen, pb);
-    hipLaunchKernelGGL(k_lb_bounds, dim3(1), dim3(64), 0, s, pb, nb, bounds);
+    hipLaunchKernelGGL(k_lb_bounds, dim3(1), dim3(64 * 6), 0, s, pb, nb, bounds);
     hipLaunchKernelGGL(k_lb_morton, dim3(blocks_for(n)), dim3(kT), 0, s, cen, n, bounds, k0, v0);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = rocprim::radix_sort_pairs(tmp, tmp_bytes, k0, k1, v0, v1, static_cast<size_t>(n), 0, 30, s);
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_lb_radix, dim3(blocks_for(n - 1)), dim3(kT), 0, s, k1, n, left, right, parent, err);
-    hipLaunchKernelGGL(k_lb_sizes, dim3(blocks_for(n)), dim3(kT), 0, s, n, left, right, parent, size, flag, err);
+    hipLaunchKernelGGL(k_lb_radix, dim3(blocks_for(n - 1)), dim3(kT), 0, s, k1, n, left, right, parent, size, err);
     hipLaunchKernelGGL(k_lb_place, dim3(blocks_for(nn)), dim3(kT), 0, s, n, left, right, parent, size, pos, err);
     hipLaunchKernelGGL(k_lb_emit, dim3(blocks_for(nn)), dim3(kT), 0, s, n, left, right, pos, v1, nodes, prims, err);
     e = hipGetLastError();
