@@ -18,6 +18,15 @@
 //   tnodes  3 x float4 per TLAS node: the two BLAS-style float4 plus
 //           {centre of left child, centre of right child, axis, 0} along the
 //           node's longest axis, the traversal order key of tlas.cpp:231-241
+//   tpairs  4 x float4 per TLAS node, what a walk that has reached it needs to
+//           go on, one 64-byte record: {left box lo.xyz, hi.x} {hi.yz, right
+//           box lo.xy} {lo.z, hi.xyz} {the two order keys, left link, right
+//           link}, a link being the child's node index or, for a leaf of
+//           one instance, kInstTest | instance; bits 28-29 of the left link
+//           hold the axis. Any other leaf (kTlasList in place of the axis):
+//           its own box as the left one, its instances torder[right link ..]
+//           and their number in place of the right box's lo.x
+//   ibox    2 x float4 per instance: the box of its TLAS leaf
 //   inst    4 x float4 per instance: world_to_local columns c0..c3 packed
 //           {c0.xyz, c1.x} {c1.yz, c2.xy} {c2.z, c3.xyz} and
 //           {blas root entry, instance_id, tri_base | flat<<31, light map or -1}
@@ -50,6 +59,13 @@ constexpr uint32_t kNoRoot = 0xFFFFFFFFu;
 // flag that marks a primitive in a hit's slot (slot = primitive index).
 constexpr uint32_t kPrimRoot = 0xFFFFFFFEu;
 constexpr uint32_t kPrimHit = 0x80000000u;
+// TLAS stack entries: a node index, an instance to enter, or an instance to
+// enter if its leaf's box is hit (see tpairs).
+constexpr uint32_t kInstTag = 0x80000000u;
+constexpr uint32_t kInstTest = 0xC0000000u;
+constexpr uint32_t kInstIndexMask = 0x0FFFFFFFu;
+constexpr uint32_t kTlasList = 3u;
+constexpr uint32_t kTlasAxisShift = 28;
 // Bound on the traversal iterations of one wave in a launch: far above any
 // legitimate walk (a wave's share of a 2^28-path batch of the 4096-instance
 // scene takes some 3e5 iterations), it makes every wave exit even if its
@@ -68,6 +84,8 @@ struct DevScene {
   const uint32_t* bigcnt;
   const float4* tris;
   const float4* tnodes;
+  const float4* tpairs;
+  const float4* ibox;
   const uint32_t* torder;
   const float4* inst;
   const int32_t* vidx;
@@ -85,7 +103,7 @@ struct DevScene {
   int32_t num_tnodes;
   int32_t num_lights;
   int32_t num_suns;
-  int32_t pad;
+  uint32_t troot;           // the TLAS root's link
   DevSky sky;
 };
 

@@ -257,7 +257,7 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const View& v,
           f3 o, d;
           float tmin, tmax;
           load(my, pci, o, d, tmin, tmax);
-          w.begin(S, o, d, tmin, tmax, st);
+          w.begin(S, o, d, tmin, tmax, st, c);
         }
         pnext = min(pend, pnext + static_cast<uint32_t>(__popcll(idle)));
       }

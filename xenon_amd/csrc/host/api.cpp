@@ -372,6 +372,47 @@ int flatten_upload(xnh_ctx* c, const xnh_flat_scene* fs, xnh_gpu_scene* g) {
     tnodes[3 * j + 2] = key;
   }
   std::vector<uint32_t> torder(fs->tlas_inst_indices, fs->tlas_inst_indices + fs->num_instances);
+  if (static_cast<uint32_t>(ntn) > kInstIndexMask || static_cast<uint32_t>(fs->num_instances) > kInstIndexMask)
+    return fail(c, XNH_E_INVALID, "too many TLAS nodes or instances (limit 2^28)");
+  // the pair records (dev_types.h): a leaf of one instance that no other leaf
+  // names becomes a link to that instance with the leaf's box beside it
+  std::vector<int32_t> leaf_of(std::max(fs->num_instances, 1), -1);   // -1 none, -2 several
+  for (int j = 0; j < ntn; ++j) {
+    const xnh_bvh_node& n = fs->tlas_nodes[j];
+    for (uint32_t k = 0; k < n.count; ++k) {
+      const uint32_t i = torder[n.child + k];
+      if (i >= static_cast<uint32_t>(fs->num_instances)) return fail(c, XNH_E_INVALID, "TLAS instance index out of range");
+      leaf_of[i] = (n.count == 1 && leaf_of[i] == -1) ? j : -2;
+    }
+  }
+  std::vector<float4> ibox(2 * static_cast<size_t>(std::max(fs->num_instances, 1)), f4(0.f, 0.f, 0.f, 0.f));
+  for (int i = 0; i < fs->num_instances; ++i)
+    if (leaf_of[i] >= 0) {
+      const xnh_bvh_node& n = fs->tlas_nodes[leaf_of[i]];
+      ibox[2 * i] = f4(n.lo[0], n.lo[1], n.lo[2], n.hi[0]);
+      ibox[2 * i + 1] = f4(n.hi[1], n.hi[2], 0.f, 0.f);
+    }
+  auto tlas_link = [&](uint32_t j) -> uint32_t {
+    const xnh_bvh_node& n = fs->tlas_nodes[j];
+    return (n.count == 1 && leaf_of[torder[n.child]] == static_cast<int32_t>(j)) ? kInstTest | torder[n.child] : j;
+  };
+  std::vector<float4> tpairs(4 * static_cast<size_t>(std::max(ntn, 1)), f4(0.f, 0.f, 0.f, 0.f));
+  for (int j = 0; j < ntn; ++j) {
+    const xnh_bvh_node& n = fs->tlas_nodes[j];
+    float4* r = tpairs.data() + 4 * static_cast<size_t>(j);
+    if (n.count == 0) {
+      const xnh_bvh_node &l = fs->tlas_nodes[n.child], &h = fs->tlas_nodes[n.child + 1];
+      const float4 key = tnodes[3 * j + 2];
+      r[0] = f4(l.lo[0], l.lo[1], l.lo[2], l.hi[0]);
+      r[1] = f4(l.hi[1], l.hi[2], h.lo[0], h.lo[1]);
+      r[2] = f4(h.lo[2], h.hi[0], h.hi[1], h.hi[2]);
+      r[3] = f4(key.x, key.y, bits(tlas_link(n.child) | as_uint(key.z) << kTlasAxisShift), bits(tlas_link(n.child + 1)));
+    } else {
+      r[0] = f4(n.lo[0], n.lo[1], n.lo[2], n.hi[0]);
+      r[1] = f4(n.hi[1], n.hi[2], bits(n.count), 0.f);
+      r[3] = f4(0.f, 0.f, bits(kTlasList << kTlasAxisShift), bits(n.child));
+    }
+  }
   // per-instance light lookup tables: first light naming (instance id, triangle)
   std::vector<int32_t> lmap;
   std::vector<float4> inst(4 * static_cast<size_t>(fs->num_instances));
@@ -469,13 +510,15 @@ int flatten_upload(xnh_ctx* c, const xnh_flat_scene* fs, xnh_gpu_scene* g) {
   HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
   free_all(g->allocs);
   DevScene S{};
-  float4 *p_bn, *p_tr, *p_tn, *p_in, *p_vn, *p_li, *p_ma, *p_su, *p_pr = nullptr, *p_pn = nullptr;
+  float4 *p_bn, *p_tr, *p_tn, *p_tp, *p_ib, *p_in, *p_vn, *p_li, *p_ma, *p_su, *p_pr = nullptr, *p_pn = nullptr;
   uint32_t *p_to, *p_po = nullptr, *p_bc, *p_ik;
   int32_t *p_vi, *p_tm, *p_lm;
   int rc = dev_upload(c, g->allocs, &p_bn, bnodes);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_bc, bigcnt);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_tr, tris);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_tn, tnodes);
+  if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_tp, tpairs);
+  if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_ib, ibox);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_to, torder);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_in, inst);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_vi, vidx);
@@ -497,6 +540,9 @@ int flatten_upload(xnh_ctx* c, const xnh_flat_scene* fs, xnh_gpu_scene* g) {
   S.bigcnt = p_bc;
   S.tris = p_tr;
   S.tnodes = p_tn;
+  S.tpairs = p_tp;
+  S.ibox = p_ib;
+  S.troot = ntn > 0 ? tlas_link(0) : 0u;
   S.torder = p_to;
   S.inst = p_in;
   S.vidx = p_vi;
@@ -523,7 +569,7 @@ int flatten_upload(xnh_ctx* c, const xnh_flat_scene* fs, xnh_gpu_scene* g) {
   S.sky.intensity = fs->sky.intensity;
   g->S = S;
   g->bytes = 0;
-  for (const auto* v : {&bnodes, &tris, &tnodes, &inst, &vnrm, &lights, &mats, &suns, &prims, &pnodes})
+  for (const auto* v : {&bnodes, &tris, &tnodes, &tpairs, &ibox, &inst, &vnrm, &lights, &mats, &suns, &prims, &pnodes})
     g->bytes += v->size() * 16;
   g->bytes += (torder.size() + vidx.size() + tmat.size() + lmap.size() + porder.size() + bigcnt.size() +
                ikind.size()) * 4;
