@@ -462,6 +462,16 @@ __device__ __forceinline__ f3 prim_normal(const PrimRec& p, f3 o, f3 d, float tm
 __device__ __forceinline__ bool ent_interior(uint32_t e) { return e < (1u << kEntShift); }
 __device__ __forceinline__ bool ent_leaf(uint32_t e) { return e - (1u << kEntShift) < kEntEnd - (1u << kEntShift); }
 
+// The arrays of the interior and leaf steps, kept in scalar registers by the
+// persistent kernels (the others are read from the job's record where they
+// are used).
+struct SceneTables {
+  const float4* bnodes;
+  const float4* tris;
+  __device__ __forceinline__ explicit SceneTables(const DevScene& S) : bnodes(S.bnodes), tris(S.tris) {}
+  __device__ __forceinline__ SceneTables() : bnodes(nullptr), tris(nullptr) {}
+};
+
 // kPrims: the scene may hold analytic primitives (a variant, because their
 // walk raises the register count of the whole kernel).
 template <bool kAny, bool kCount = true, bool kPrims = true>
@@ -675,8 +685,8 @@ struct Walker {
   // continue with the nearer hit one, push the farther; with no child hit,
   // continue with the entry on top of the stack.
   template <bool kFast>
-  __device__ __forceinline__ void interior_step(const DevScene& S, TravStack& st, TravCount& c) {
-    const float4* pair = S.bnodes + 2 * static_cast<size_t>(e);
+  __device__ __forceinline__ void interior_step(const SceneTables& T, TravStack& st, TravCount& c) {
+    const float4* pair = T.bnodes + 2 * static_cast<size_t>(e);
     const float4 la = gld4(pair, 0), lb = gld4(pair, 1), ra = gld4(pair, 2), rb = gld4(pair, 3);
     const uint32_t below = st.below();
     float tn0, tn1;
@@ -722,17 +732,17 @@ struct Walker {
   // Tests the leaf e and continues with the entry on top of the stack. The
   // first two triangles (a leaf of the reference's builder holds at most
   // two) are fetched together.
-  __device__ __forceinline__ void leaf_step(const DevScene& S, TravStack& st, TravCount& c) {
+  __device__ __forceinline__ void leaf_step(const DevScene& S, const SceneTables& T, TravStack& st, TravCount& c) {
     uint32_t count = e >> kEntShift;
     const uint32_t first = e & kEntIndexMask;
-    const TriRec r0 = load_tri(S.tris, first);
-    const TriRec r1 = load_tri(S.tris, count > 1u ? first + 1u : first);
+    const TriRec r0 = load_tri(T.tris, first);
+    const TriRec r1 = load_tri(T.tris, count > 1u ? first + 1u : first);
     const uint32_t below = st.below();
     bool ended = test_tri(r0, first, true, c);
     if (!kAny || !ended) ended = test_tri(r1, first + 1u, count > 1u, c);
     if (ballot(count > 2u) != 0ull) {   // larger leaves (equal centres, other builders)
       if (count == kEntBigLeaf) count = gld1(S.bigcnt, first);
-      for (uint32_t k = 2; k < count && !(kAny && ended); ++k) ended = test_tri(load_tri(S.tris, first + k), first + k, true, c);
+      for (uint32_t k = 2; k < count && !(kAny && ended); ++k) ended = test_tri(load_tri(T.tris, first + k), first + k, true, c);
     }
     if (kAny && ended) {
       occluded = true;
@@ -765,12 +775,12 @@ struct Walker {
 // Interior steps of wave_step's lanes while interior steps keep the
 // majority of the wave's BLAS lanes.
 template <bool kFast, bool kAny, bool kCount, bool kPrims>
-__device__ __forceinline__ void interior_run(Walker<kAny, kCount, kPrims>& w, const DevScene& S, TravStack& st,
+__device__ __forceinline__ void interior_run(Walker<kAny, kCount, kPrims>& w, const SceneTables& T, TravStack& st,
                                              TravCount& c) {
   int ni, nl;
   do {
     if (kCount && first_active_lane()) ++c.int_iters;
-    if (ent_interior(w.e)) w.template interior_step<kFast>(S, st, c);
+    if (ent_interior(w.e)) w.template interior_step<kFast>(T, st, c);
     ni = lanes_of(ent_interior(w.e));
     nl = lanes_of(ent_leaf(w.e));
   } while (ni != 0 && ni >= nl);
@@ -787,48 +797,57 @@ __device__ __forceinline__ void interior_run(Walker<kAny, kCount, kPrims>& w, co
 // and work counts are the reference's. Scheduling by majority rather than
 // letting every lane finish a whole descent before any leaf is tested keeps
 // more lanes of each iteration busy (a wave's descents differ in length).
-// Lanes without a ray (Walker::idle) and finished ones take no part. Every
-// lane of the wave must reach it.
+// Lanes without a ray (Walker::idle) and finished ones take no part. Runs
+// follow each other until `rest` lanes take no part (the caller then gives
+// them rays) or kTurns are done: going round the caller's loop between two
+// runs cost as much as an interior step (Cornell 512x512x64 12.4 -> 12.0 ms,
+// 1.3M-triangle mesh 1920x1080x256 240.7 -> 236.5 ms). With primitives, whose
+// long instance steps leave lanes finished for longer, one run at a time
+// (801x449x33 6.38 against 6.50 ms). Every lane of the wave must reach it.
+constexpr int kTurns = 64;
 template <bool kAny, bool kCount, bool kPrims>
-__device__ __forceinline__ void wave_step(Walker<kAny, kCount, kPrims>& w, const DevScene& S, TravStack& st,
-                                          TravCount& c) {
-  const int nt = lanes_of(w.e == kEntEnd && !st.empty());
-  int nl = lanes_of(ent_leaf(w.e)), ni = lanes_of(ent_interior(w.e));
-  if (ni >= nl && ni >= nt) {
-    // the hardware min/max slab test when every walking lane's ray allows it
-    // (a wave-uniform choice). The two runs are separate loops: with one
-    // loop and the choice inside it, the compiler computed the slab
-    // distances before the branch, and the min/max instructions then
-    // re-canonicalised each of them (a value from another block may be a
-    // signalling NaN), 12 more instructions per node pair.
-    if (ni == 0) return;
-    if (ballot(ent_interior(w.e) && !w.fast) == 0ull) interior_run<true>(w, S, st, c);
-    else interior_run<false>(w, S, st, c);
-  } else if (nl >= nt) {
-    do {
-      if (kCount && first_active_lane()) ++c.leaf_iters;
-      if (ent_leaf(w.e)) {
-        if (kCount) ++c.leaf_steps;
-        w.leaf_step(S, st, c);
-      }
-      nl = lanes_of(ent_leaf(w.e));
-      ni = lanes_of(ent_interior(w.e));
-    } while (nl != 0 && nl >= ni);
-  } else {
-    // in this run until it enters a BLAS or ends; each turn takes the kind,
-    // node or instance, that more of its lanes need
-    bool part = w.e == kEntEnd && !st.empty();
-    int n0;
-    do {
-      const bool instance = Walker<kAny, kCount, kPrims>::is_instance(st.tos);
-      if (lanes_of(part && !instance) >= lanes_of(part && instance)) {
-        if (part && !instance) w.node_step(S, st, c);
-      } else {
-        if (part && instance) w.instance_step(S, st, c);
-      }
-      part = part && w.e == kEntEnd && !st.empty();
-      n0 = lanes_of(part);
-    } while (n0 != 0 && 2 * n0 >= nt);
+__device__ __forceinline__ void wave_step(Walker<kAny, kCount, kPrims>& w, const DevScene& S, const SceneTables& T,
+                                          TravStack& st, TravCount& c, int rest) {
+  for (int turn = 0; turn < (kPrims ? 1 : kTurns); ++turn) {
+    const int nt = lanes_of(w.e == kEntEnd && !st.empty());
+    int nl = lanes_of(ent_leaf(w.e)), ni = lanes_of(ent_interior(w.e));
+    if (64 - (nt + nl + ni) >= rest && turn > 0) return;
+    if (ni >= nl && ni >= nt) {
+      // the hardware min/max slab test when every walking lane's ray allows it
+      // (a wave-uniform choice). The two runs are separate loops: with one
+      // loop and the choice inside it, the compiler computed the slab
+      // distances before the branch, and the min/max instructions then
+      // re-canonicalised each of them (a value from another block may be a
+      // signalling NaN), 12 more instructions per node pair.
+      if (ni == 0) return;
+      if (ballot(ent_interior(w.e) && !w.fast) == 0ull) interior_run<true>(w, T, st, c);
+      else interior_run<false>(w, T, st, c);
+    } else if (nl >= nt) {
+      do {
+        if (kCount && first_active_lane()) ++c.leaf_iters;
+        if (ent_leaf(w.e)) {
+          if (kCount) ++c.leaf_steps;
+          w.leaf_step(S, T, st, c);
+        }
+        nl = lanes_of(ent_leaf(w.e));
+        ni = lanes_of(ent_interior(w.e));
+      } while (nl != 0 && nl >= ni);
+    } else {
+      // in this run until it enters a BLAS or ends; each turn takes the kind,
+      // node or instance, that more of its lanes need
+      bool part = w.e == kEntEnd && !st.empty();
+      int n0;
+      do {
+        const bool instance = Walker<kAny, kCount, kPrims>::is_instance(st.tos);
+        if (lanes_of(part && !instance) >= lanes_of(part && instance)) {
+          if (part && !instance) w.node_step(S, st, c);
+        } else {
+          if (part && instance) w.instance_step(S, st, c);
+        }
+        part = part && w.e == kEntEnd && !st.empty();
+        n0 = lanes_of(part);
+      } while (n0 != 0 && 2 * n0 >= nt);
+    }
   }
 }
 
@@ -838,6 +857,7 @@ template <bool kAny>
 __device__ __forceinline__ bool walk_scene(const DevScene& S, f3 o, f3 d, float tmin, float tmax, bool valid,
                                            HitRef& hit, TravStack& st, TravCount& c) {
   Walker<kAny> w;
+  const SceneTables T(S);
   w.begin(S, o, d, tmin, tmax, st, c);
   if (!valid) w.stop(st);
   for (uint32_t guard = 0; ballot(!w.finished(st)) != 0ull; ++guard) {
@@ -845,7 +865,7 @@ __device__ __forceinline__ bool walk_scene(const DevScene& S, f3 o, f3 d, float 
       st.overflow = true;
       break;
     }
-    wave_step(w, S, st, c);
+    wave_step(w, S, T, st, c, 64);
   }
   hit = w.hit;
   hit.t = w.found() ? w.tbest : 0.f;

@@ -160,13 +160,15 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const View& v,
                                             bool& overflow, const float4* ray1, uint16_t* slist, uint32_t* sbase,
                                             Load load, Finish finish) {
   constexpr uint32_t kIdle = 0xFFFFFFFFu;
+  constexpr int kRefill = kPrims ? 24 : 32;
   const int lane = lane_id();
   const unsigned long long below = (1ull << lane) - 1ull;
   uint32_t my = kIdle;
   Walker<kAny, kCount, kPrims> w;
   w.idle(st);
   uint32_t pbase = 0, pnext = 0, pend = 0;   // wave-uniform pool: entries pbase + [pnext, pend) of chunk pci
-  int pci = 0;
+  int pci = 0, job = 0;
+  SceneTables tables;
   const uint32_t part = 64u >> un.split, pmask = (1u << un.split) - 1u;
   bool stuck = false;
   for (uint32_t guard = 0;; ++guard) {
@@ -180,8 +182,8 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const View& v,
     // wave as much for one lane as for all. Every idle lane at once: 1.3M-
     // triangle mesh 1920x1080x256 265 ms, 4096 instances 359 ms, Cornell
     // 512x512x64 12.8 ms; 16 together 253, 349, 12.3; 24: 247, 347, 12.3; 32:
-    // 250, 347, 12.2.
-    constexpr int kRefill = 24;
+    // 250, 347, 12.2. With wave_step going on by itself until then: mesh 237
+    // and Cornell 12.2 ms at 24, 235 and 11.8 at 32, 242 and 12.1 at 40.
     if (act == 0ull || __popcll(~act) >= kRefill) {
       if (pnext >= pend) {
         if (un.cur >= un.end && !un.exhausted) un.fetch();
@@ -191,8 +193,11 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const View& v,
           // a unit of another job waits until the wave has drained (the
           // rays in flight in a wave share one scene)
           const int ci = uniform(find_chunk(v, ucur >> un.split));
-          if (act == 0ull || v.ch[ci].job == v.ch[pci].job) {
+          const int cjob = uniform(v.ch[ci].job);
+          if (act == 0ull || cjob == job) {
             pci = ci;
+            job = cjob;
+            tables = SceneTables(job_scene(B.jobs, job));
             if constexpr (kSort) {
               // the fetched units that lie in this chunk (1 to 16), keyed by
               // octant (4 bits per unit and lane; 8 = no entry)
@@ -246,7 +251,7 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const View& v,
       if (pnext < pend) {
         const unsigned long long idle = ~act;
         const uint32_t rank = static_cast<uint32_t>(__popcll(idle & below));
-        const DevScene& S = job_scene(B.jobs, uniform(v.ch[pci].job));
+        const DevScene& S = job_scene(B.jobs, job);
         if (my == kIdle && pnext + rank < pend) {
           if constexpr (kSort) {
             const uint32_t t = slist[pnext + rank];
@@ -267,8 +272,7 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const View& v,
     if ((un.cur >= hi || (un.exhausted && un.cur >= un.end)) && __ballot(my != kIdle) == 0ull) break;
     if (kCount && lane == 0) ++c.round_iters;
     if (kCount && my != kIdle) ++c.round_lanes;
-    const DevScene& S = job_scene(B.jobs, uniform(v.ch[pci].job));
-    wave_step(w, S, st, c);
+    wave_step(w, job_scene(B.jobs, job), tables, st, c, kRefill);
     if (my != kIdle && w.finished(st)) {
       overflow |= st.overflow;
       finish(my, w);
