@@ -290,7 +290,7 @@ enum Stat : int {
 
 // Output stage (image.hip): the device state of one NoiseStats computation
 // (math/image.h:11-31 plus the radix-select state) and its scratch.
-constexpr int kImgMaxBlocks = 2048;                 // partial-sum blocks of one pass
+constexpr int kImgMaxBlocks = 1024;                 // work-groups (and partial sums) of one pass
 constexpr int64_t kImgMaxPixels = int64_t(1) << 26; // 8192 x 8192
 struct ImgState {
   float avg, edge, eps;        // average luminance, edge threshold, epsilon
@@ -298,17 +298,20 @@ struct ImgState {
   uint32_t count, pad;         // counted (interior, non-edge) pixels
   uint32_t rank[2];            // median, 95th percentile: rank left inside the prefix
   uint32_t prefix[2];          // bits of the selected key found so far
-  uint32_t hist[512];          // [target][digit] of the current pass
+  // digit counts of the three passes (11, 11 and 10 bits): the first shared
+  // by both targets, then [target][digit]
+  uint32_t hist0[2048], hist1[2][2048], hist2[2][1024];
 };
 // The allocation-free NoiseStats entry point's static scratch: images of at
 // most 2^22 pixels (2048 x 2048), luminance and keys 16 MiB each plus the
 // per-block partials and the state, 256-byte aligned.
 constexpr int64_t kImgStaticMaxPixels = int64_t(1) << 22;
-constexpr size_t kImgStaticScratchBytes = 33605888;   // 32.05 MiB
+constexpr size_t kImgStaticScratchBytes = 33620224;   // 32.05 MiB
 struct ImgScratch {
   float* lum;                  // W*H luminance
   uint32_t* key;               // W*H residual keys
-  double* part;                // 2 * kImgMaxBlocks partial sums
+  double* part;                // kImgMaxBlocks partial luminance sums
+  double* part2;               // 2 * kImgMaxBlocks partial residual sums
   float* pmax;                 // kImgMaxBlocks partial maxima
   uint32_t* pcnt;              // kImgMaxBlocks partial counts
   ImgState* st;

@@ -11,9 +11,18 @@
 // only where a double sum lands within its own rounding error of a float
 // rounding boundary. The median and 95th percentile are selected exactly:
 // the residuals are non-negative floats, whose bit patterns order like the
-// values, and a four-pass radix select (8 bits a pass, both ranks at once)
-// finds the k-th smallest pattern with k computed as the reference computes
-// it. Nothing leaves the device until the 64-byte result.
+// values, and a three-pass radix select (11, 11 and 10 bits, both ranks at
+// once) finds the k-th smallest pattern with k computed as the reference
+// computes it. Nothing leaves the device until the result.
+//
+// NoiseStats is five launches. Bound at 1920x1080 by launches and their
+// latency rather than by the 33 MB it moves: every work-group adds the few
+// hundred partial results of the launch before itself instead of leaving
+// that to a launch of one work-group, the first digit is counted where the
+// keys are made, and a pass has at most 1024 work-groups, because each adds
+// its counts to the same words and one address takes about 85 M atomics a
+// second. 73 us of the device's time; 2048 work-groups, four 8-bit passes and a
+// one-thread scan of each took 12 launches and 205 us.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
@@ -27,6 +36,9 @@ namespace {
 
 constexpr int kImgThreads = 256;
 constexpr uint32_t kNoKey = 0xFFFFFFFFu;   // above every non-negative float's bit pattern
+constexpr int kImgHistWords = 2048 + 2 * 2048 + 2 * 1024;
+static_assert(sizeof(ImgState::hist0) + sizeof(ImgState::hist1) + sizeof(ImgState::hist2) == 4 * kImgHistWords,
+              "digit counts follow each other");
 
 __device__ __forceinline__ double wave_sumd(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
@@ -77,11 +89,15 @@ __global__ void __launch_bounds__(kImgThreads) k_img_from_accum(const float4* ac
 }
 
 // image.h:127-135 and 137-146: luminance, and per-block double sums of it.
-__global__ void __launch_bounds__(kImgThreads) k_img_lum(const float* img, int n, float* lum, double* part) {
+// Clears the digit counts of the passes that follow.
+__global__ void __launch_bounds__(kImgThreads) k_img_lum(const float* img, int n, float* lum, double* part,
+                                                         ImgState* st) {
   __shared__ double red[kImgThreads / 64];
+  const int tid = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+  const int stride = static_cast<int>(gridDim.x * blockDim.x);
+  for (int k = tid; k < kImgHistWords; k += stride) st->hist0[k] = 0u;   // hist0, hist1 and hist2 follow each other
   double acc = 0.0;
-  for (int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x); i < n;
-       i += static_cast<int>(gridDim.x * blockDim.x)) {
+  for (int i = tid; i < n; i += stride) {
     const float r = img[3 * static_cast<size_t>(i)], g = img[3 * static_cast<size_t>(i) + 1],
                 b = img[3 * static_cast<size_t>(i) + 2];
     const float l = 0.2126f * r + 0.7152f * g + 0.0722f * b;
@@ -92,32 +108,31 @@ __global__ void __launch_bounds__(kImgThreads) k_img_lum(const float* img, int n
   if (threadIdx.x == 0) part[blockIdx.x] = t;
 }
 
-// image.h:51-57: average luminance, edge threshold and epsilon.
-__global__ void __launch_bounds__(kImgThreads) k_img_prep(const double* part, int nb, int n, ImgState* st) {
-  __shared__ double red[kImgThreads / 64];
-  double acc = 0.0;
-  for (int k = static_cast<int>(threadIdx.x); k < nb; k += static_cast<int>(blockDim.x)) acc += part[k];
-  const double t = block_sumd(acc, red);
-  if (threadIdx.x == 0) {
-    const float avg = static_cast<float>(t / static_cast<double>(n));
-    st->avg = avg;
-    st->edge = std_max(1e-6f, avg * 0.1f);
-    st->eps = std_max(1e-8f, avg * avg * 1e-4f);
-  }
-}
-
-// image.h:63-98 for every interior pixel: the edge test, the residual
+// image.h:51-57 (average luminance, edge threshold and epsilon, by every
+// work-group in the same order) and image.h:63-98 for every interior pixel:
+// the edge test, the residual
 // against the blur and its two normalised forms. key[i] is the absolute
 // form's bit pattern for a counted pixel, kNoKey otherwise; per block the
-// double sums of both forms, the maximum and the count.
-__global__ void __launch_bounds__(kImgThreads) k_img_resid(const float* lum, int w, int h, const ImgState* st,
-                                                           uint32_t* key, double* part2, float* pmax,
+// double sums of both forms, the maximum and the count. The keys' first
+// digits are counted on the way.
+__global__ void __launch_bounds__(kImgThreads) k_img_resid(const float* lum, int w, int h, const double* part,
+                                                           ImgState* st, uint32_t* key, double* part2, float* pmax,
                                                            uint32_t* pcnt) {
   __shared__ double red[kImgThreads / 64];
   __shared__ float redm[kImgThreads / 64];
   __shared__ uint32_t redc[kImgThreads / 64];
-  const float edge = st->edge, eps = st->eps;
+  __shared__ uint32_t lh[2048];
   const int n = w * h;
+  double sum = 0.0;
+  for (int k = static_cast<int>(threadIdx.x); k < static_cast<int>(gridDim.x); k += kImgThreads) sum += part[k];
+  for (int k = static_cast<int>(threadIdx.x); k < 2048; k += kImgThreads) lh[k] = 0u;
+  const float avg = static_cast<float>(block_sumd(sum, red) / static_cast<double>(n));
+  const float edge = std_max(1e-6f, avg * 0.1f), eps = std_max(1e-8f, avg * avg * 1e-4f);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    st->avg = avg;
+    st->edge = edge;
+    st->eps = eps;
+  }
   double s2 = 0.0, s1 = 0.0;
   float mx = 0.f;
   uint32_t cnt = 0u;
@@ -152,6 +167,7 @@ __global__ void __launch_bounds__(kImgThreads) k_img_resid(const float* lum, int
         mx = gt_max(mx, q1);
         ++cnt;
         k = __float_as_uint(q1);
+        if (k != kNoKey) atomicAdd(&lh[k >> 21], 1u);
       }
     }
     key[i] = k;
@@ -166,6 +182,8 @@ __global__ void __launch_bounds__(kImgThreads) k_img_resid(const float* lum, int
     redc[wv] = wc;
   }
   __syncthreads();
+  for (int k = static_cast<int>(threadIdx.x); k < 2048; k += kImgThreads)
+    if (lh[k]) atomicAdd(&st->hist0[k], lh[k]);
   if (threadIdx.x == 0) {
     float m = 0.f;
     uint32_t c = 0u;
@@ -180,22 +198,62 @@ __global__ void __launch_bounds__(kImgThreads) k_img_resid(const float* lum, int
   }
 }
 
+// The digit whose count holds the given rank, and the rank within it (block
+// of kImgThreads threads, kBins a multiple of that; every thread gets both).
+struct Pick {
+  uint32_t digit, rank;
+};
+template <int kBins>
+__device__ Pick block_pick(const uint32_t* hist, uint32_t rank) {
+  __shared__ uint32_t wsum[kImgThreads / 64];
+  __shared__ Pick found;
+  constexpr int per = kBins / kImgThreads;
+  const int lane = static_cast<int>(threadIdx.x & 63u), wv = static_cast<int>(threadIdx.x >> 6);
+  const int b0 = static_cast<int>(threadIdx.x) * per;
+  uint32_t c[per], sum = 0u;
+  for (int k = 0; k < per; ++k) {
+    c[k] = hist[b0 + k];
+    sum += c[k];
+  }
+  uint32_t inc = sum;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t t = __shfl_up(inc, o);
+    if (lane >= o) inc += t;
+  }
+  if (threadIdx.x == 0) found = Pick{0u, rank};
+  if (lane == 63) wsum[wv] = inc;
+  __syncthreads();
+  uint32_t cum = inc - sum;
+  for (int k = 0; k < wv; ++k) cum += wsum[k];
+  for (int k = 0; k < per; ++k) {
+    if (rank >= cum && rank < cum + c[k]) found = Pick{static_cast<uint32_t>(b0 + k), rank - cum};
+    cum += c[k];
+  }
+  __syncthreads();
+  const Pick r = found;
+  __syncthreads();
+  return r;
+}
+
 // image.h:100-118: totals, the three means, and the two ranks
-// k = (size_t)(p * (float)(n - 1)) of image.h:176-186.
-__global__ void __launch_bounds__(kImgThreads) k_img_final(const double* part2, const float* pmax,
-                                                           const uint32_t* pcnt, int nb, ImgState* st) {
+// k = (size_t)(p * (float)(n - 1)) of image.h:176-186, their first digits, and
+// the counts of the second digits of the keys that carry them.
+__global__ void __launch_bounds__(kImgThreads) k_img_second(const uint32_t* key, int n, const double* part2,
+                                                            const float* pmax, const uint32_t* pcnt, ImgState* st) {
   __shared__ double red[kImgThreads / 64];
   __shared__ float redm[kImgThreads / 64];
   __shared__ uint32_t redc[kImgThreads / 64];
+  __shared__ uint32_t lh[2][2048];
   double s2 = 0.0, s1 = 0.0;
   float mx = 0.f;
   uint32_t cnt = 0u;
-  for (int k = static_cast<int>(threadIdx.x); k < nb; k += static_cast<int>(blockDim.x)) {
+  for (int k = static_cast<int>(threadIdx.x); k < static_cast<int>(gridDim.x); k += kImgThreads) {
     s2 += part2[2 * k];
     s1 += part2[2 * k + 1];
     mx = gt_max(mx, pmax[k]);
     cnt += pcnt[k];
   }
+  for (int k = static_cast<int>(threadIdx.x); k < 4096; k += kImgThreads) lh[k >> 11][k & 2047] = 0u;
   const double t2 = block_sumd(s2, red);
   const double t1 = block_sumd(s1, red);
   const float wm = wave_gt_max(mx);
@@ -206,69 +264,72 @@ __global__ void __launch_bounds__(kImgThreads) k_img_final(const double* part2, 
     redc[wv] = wc;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    float m = 0.f;
-    uint32_t c = 0u;
-    for (int k = 0; k < nw; ++k) {
-      m = gt_max(m, redm[k]);
-      c += redc[k];
-    }
+  float m = 0.f;
+  uint32_t c = 0u;
+  for (int k = 0; k < nw; ++k) {
+    m = gt_max(m, redm[k]);
+    c += redc[k];
+  }
+  Pick p[2] = {{0u, 0u}, {0u, 0u}};
+  if (c > 0u) {
+    p[0] = block_pick<2048>(st->hist0, static_cast<uint32_t>(0.50f * static_cast<float>(c - 1u)));
+    p[1] = block_pick<2048>(st->hist0, static_cast<uint32_t>(0.95f * static_cast<float>(c - 1u)));
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
     st->count = c;
     st->max_abs = m;
-    st->mean_sq = 0.f;
-    st->mean_abs = 0.f;
-    st->rank[0] = st->rank[1] = 0u;
-    if (c > 0u) {
-      st->mean_sq = static_cast<float>(t2 / static_cast<double>(c));
-      st->mean_abs = static_cast<float>(t1 / static_cast<double>(c));
-      st->rank[0] = static_cast<uint32_t>(0.50f * static_cast<float>(c - 1u));
-      st->rank[1] = static_cast<uint32_t>(0.95f * static_cast<float>(c - 1u));
+    st->mean_sq = c > 0u ? static_cast<float>(t2 / static_cast<double>(c)) : 0.f;
+    st->mean_abs = c > 0u ? static_cast<float>(t1 / static_cast<double>(c)) : 0.f;
+    for (int t = 0; t < 2; ++t) {
+      st->prefix[t] = p[t].digit;
+      st->rank[t] = p[t].rank;
     }
-    st->prefix[0] = st->prefix[1] = 0u;
   }
-  for (int k = static_cast<int>(threadIdx.x); k < 512; k += static_cast<int>(blockDim.x)) st->hist[k] = 0u;
-}
-
-// One radix-select pass: histogram of digit `pass` (most significant first)
-// of the keys that carry each target's prefix so far.
-__global__ void __launch_bounds__(kImgThreads) k_img_hist(const uint32_t* key, int n, ImgState* st, int pass) {
-  __shared__ uint32_t lh[512];
-  for (int k = static_cast<int>(threadIdx.x); k < 512; k += static_cast<int>(blockDim.x)) lh[k] = 0u;
-  __syncthreads();
-  const int shift = 24 - 8 * pass;
-  const uint32_t p0 = st->prefix[0], p1 = st->prefix[1];
   for (int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x); i < n;
        i += static_cast<int>(gridDim.x * blockDim.x)) {
     const uint32_t k = key[i];
     if (k == kNoKey) continue;
-    const uint32_t d = (k >> shift) & 255u;
-    const uint32_t hi = pass == 0 ? 0u : (k >> (shift + 8));
-    if (hi == p0) atomicAdd(&lh[d], 1u);
-    if (hi == p1) atomicAdd(&lh[256 + d], 1u);
+    for (int t = 0; t < 2; ++t)
+      if ((k >> 21) == p[t].digit) atomicAdd(&lh[t][(k >> 10) & 2047u], 1u);
   }
   __syncthreads();
-  for (int k = static_cast<int>(threadIdx.x); k < 512; k += static_cast<int>(blockDim.x))
-    if (lh[k]) atomicAdd(&st->hist[k], lh[k]);
+  for (int k = static_cast<int>(threadIdx.x); k < 4096; k += kImgThreads)
+    if (lh[k >> 11][k & 2047]) atomicAdd(&st->hist1[k >> 11][k & 2047], lh[k >> 11][k & 2047]);
 }
 
-// The digit whose bin holds each target's rank; the rank becomes the rank
-// within that bin, and the histogram is cleared for the next pass.
-__global__ void __launch_bounds__(64) k_img_pick(ImgState* st) {
-  const int t = static_cast<int>(threadIdx.x);
-  if (t < 2 && st->count > 0u) {
-    uint32_t cum = 0u, r = st->rank[t];
-    for (uint32_t d = 0; d < 256u; ++d) {
-      const uint32_t c = st->hist[256 * t + d];
-      if (r < cum + c) {
-        st->prefix[t] = (st->prefix[t] << 8) | d;
-        st->rank[t] = r - cum;
-        break;
-      }
-      cum += c;
-    }
+// The second digits, and the counts of the last ten bits of the keys that
+// carry both. prefix and rank of st are the first digit's (written by the
+// launch before).
+__global__ void __launch_bounds__(kImgThreads) k_img_third(const uint32_t* key, int n, ImgState* st) {
+  __shared__ uint32_t lh[2][1024];
+  for (int k = static_cast<int>(threadIdx.x); k < 2048; k += kImgThreads) lh[k >> 10][k & 1023] = 0u;
+  uint32_t pre[2] = {0u, 0u};
+  if (st->count > 0u)
+    for (int t = 0; t < 2; ++t) pre[t] = (st->prefix[t] << 11) | block_pick<2048>(st->hist1[t], st->rank[t]).digit;
+  __syncthreads();
+  for (int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x); i < n;
+       i += static_cast<int>(gridDim.x * blockDim.x)) {
+    const uint32_t k = key[i];
+    if (k == kNoKey) continue;
+    for (int t = 0; t < 2; ++t)
+      if ((k >> 10) == pre[t]) atomicAdd(&lh[t][k & 1023u], 1u);
   }
   __syncthreads();
-  for (int k = t; k < 512; k += static_cast<int>(blockDim.x)) st->hist[k] = 0u;
+  for (int k = static_cast<int>(threadIdx.x); k < 2048; k += kImgThreads)
+    if (lh[k >> 10][k & 1023]) atomicAdd(&st->hist2[k >> 10][k & 1023], lh[k >> 10][k & 1023]);
+}
+
+// The selected keys (one work-group).
+__global__ void __launch_bounds__(kImgThreads) k_img_select(ImgState* st) {
+  if (st->count == 0u) return;
+  uint32_t keys[2];
+  for (int t = 0; t < 2; ++t) {
+    const Pick b = block_pick<2048>(st->hist1[t], st->rank[t]);
+    const Pick c = block_pick<1024>(st->hist2[t], b.rank);
+    keys[t] = (((st->prefix[t] << 11) | b.digit) << 10) | c.digit;
+  }
+  __syncthreads();   // every thread has read prefix and rank
+  if (threadIdx.x < 2) st->prefix[threadIdx.x] = threadIdx.x == 0 ? keys[0] : keys[1];
 }
 
 // main.cpp:28-30 with the writer's vertical flip: file row r is framebuffer
@@ -301,15 +362,12 @@ hipError_t launch_img_from_accum(hipStream_t s, const float4* accum, float inv_s
 
 hipError_t launch_noise_stats(hipStream_t s, const float* img, int w, int h, ImgScratch sc) {
   const int n = w * h, nb = img_blocks(n);
-  hipLaunchKernelGGL(k_img_lum, dim3(nb), dim3(kImgThreads), 0, s, img, n, sc.lum, sc.part);
-  hipLaunchKernelGGL(k_img_prep, dim3(1), dim3(kImgThreads), 0, s, sc.part, nb, n, sc.st);
-  hipLaunchKernelGGL(k_img_resid, dim3(nb), dim3(kImgThreads), 0, s, sc.lum, w, h, sc.st, sc.key, sc.part,
+  hipLaunchKernelGGL(k_img_lum, dim3(nb), dim3(kImgThreads), 0, s, img, n, sc.lum, sc.part, sc.st);
+  hipLaunchKernelGGL(k_img_resid, dim3(nb), dim3(kImgThreads), 0, s, sc.lum, w, h, sc.part, sc.st, sc.key, sc.part2,
                      sc.pmax, sc.pcnt);
-  hipLaunchKernelGGL(k_img_final, dim3(1), dim3(kImgThreads), 0, s, sc.part, sc.pmax, sc.pcnt, nb, sc.st);
-  for (int pass = 0; pass < 4; ++pass) {
-    hipLaunchKernelGGL(k_img_hist, dim3(nb), dim3(kImgThreads), 0, s, sc.key, n, sc.st, pass);
-    hipLaunchKernelGGL(k_img_pick, dim3(1), dim3(64), 0, s, sc.st);
-  }
+  hipLaunchKernelGGL(k_img_second, dim3(nb), dim3(kImgThreads), 0, s, sc.key, n, sc.part2, sc.pmax, sc.pcnt, sc.st);
+  hipLaunchKernelGGL(k_img_third, dim3(nb), dim3(kImgThreads), 0, s, sc.key, n, sc.st);
+  hipLaunchKernelGGL(k_img_select, dim3(1), dim3(kImgThreads), 0, s, sc.st);
   return hipGetLastError();
 }
 
@@ -317,15 +375,15 @@ hipError_t launch_noise_stats(hipStream_t s, const float* img, int w, int h, Img
 // One static device array per GPU, carved into the ImgScratch fields for
 // images of at most kImgStaticMaxPixels. The launch sequence above writes
 // every scratch word it later reads within the same call (the partial sums
-// per block, the keys per pixel; k_img_final clears the histogram and the
-// radix-select state), so nothing needs clearing between calls. Calls that
+// per block, the keys per pixel; k_img_lum clears the digit counts), so nothing needs clearing between calls. Calls that
 // overlap on one GPU share the array and race.
 namespace {
 constexpr size_t align256(size_t x) { return (x + 255u) & ~static_cast<size_t>(255u); }
 constexpr size_t kStOffLum = 0;
 constexpr size_t kStOffKey = align256(kStOffLum + sizeof(float) * kImgStaticMaxPixels);
 constexpr size_t kStOffPart = align256(kStOffKey + sizeof(uint32_t) * kImgStaticMaxPixels);
-constexpr size_t kStOffPmax = align256(kStOffPart + sizeof(double) * 2 * kImgMaxBlocks);
+constexpr size_t kStOffPart2 = align256(kStOffPart + sizeof(double) * kImgMaxBlocks);
+constexpr size_t kStOffPmax = align256(kStOffPart2 + sizeof(double) * 2 * kImgMaxBlocks);
 constexpr size_t kStOffPcnt = align256(kStOffPmax + sizeof(float) * kImgMaxBlocks);
 constexpr size_t kStOffState = align256(kStOffPcnt + sizeof(uint32_t) * kImgMaxBlocks);
 constexpr size_t kStBytes = align256(kStOffState + sizeof(ImgState));
@@ -365,6 +423,7 @@ hipError_t img_static_scratch(int device, ImgScratch* sc) {
   sc->lum = reinterpret_cast<float*>(base + kStOffLum);
   sc->key = reinterpret_cast<uint32_t*>(base + kStOffKey);
   sc->part = reinterpret_cast<double*>(base + kStOffPart);
+  sc->part2 = reinterpret_cast<double*>(base + kStOffPart2);
   sc->pmax = reinterpret_cast<float*>(base + kStOffPmax);
   sc->pcnt = reinterpret_cast<uint32_t*>(base + kStOffPcnt);
   sc->st = reinterpret_cast<ImgState*>(base + kStOffState);

@@ -23,6 +23,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <cstdio>
 #include <cstring>
 #include <new>
@@ -1221,7 +1222,8 @@ int ensure_out(xnh_ctx* c, int64_t npix) {
   if (rc == XNH_OK) rc = dev_alloc(c, o.allocs, &o.rgb8, static_cast<size_t>(3 * npix));
   if (rc == XNH_OK) rc = dev_alloc(c, o.allocs, &o.sc.lum, static_cast<size_t>(npix));
   if (rc == XNH_OK) rc = dev_alloc(c, o.allocs, &o.sc.key, static_cast<size_t>(npix));
-  if (rc == XNH_OK) rc = dev_alloc(c, o.allocs, &o.sc.part, static_cast<size_t>(2 * kImgMaxBlocks));
+  if (rc == XNH_OK) rc = dev_alloc(c, o.allocs, &o.sc.part, static_cast<size_t>(kImgMaxBlocks));
+  if (rc == XNH_OK) rc = dev_alloc(c, o.allocs, &o.sc.part2, static_cast<size_t>(2 * kImgMaxBlocks));
   if (rc == XNH_OK) rc = dev_alloc(c, o.allocs, &o.sc.pmax, static_cast<size_t>(kImgMaxBlocks));
   if (rc == XNH_OK) rc = dev_alloc(c, o.allocs, &o.sc.pcnt, static_cast<size_t>(kImgMaxBlocks));
   if (rc == XNH_OK) rc = dev_alloc(c, o.allocs, &o.sc.st, 1);
@@ -1258,8 +1260,8 @@ namespace {
 // Reads the device state of a finished NoiseStats computation into `out`
 // (math/image.h:100-118).
 int read_noise_stats(xnh_ctx* c, const ImgState* dst, int32_t w, int32_t h, xnh_noise_stats* out) {
-  ImgState st;
-  HIP_OR_FAIL(c, hipMemcpyAsync(&st, dst, sizeof st, hipMemcpyDeviceToHost, c->stream));
+  ImgState st;   // (without the digit counts)
+  HIP_OR_FAIL(c, hipMemcpyAsync(&st, dst, offsetof(ImgState, hist0), hipMemcpyDeviceToHost, c->stream));
   HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
   const int interior = (w - 2) * (h - 2);
   out->total_interior_pixel_count = interior;
