@@ -21,6 +21,7 @@ struct GuideNet {
   const uint16_t* grid;   // FP16 bits [level][slot][feature]
   const uint16_t* w;      // FP16 bits, kWTotal, row-major per layer
   const uint16_t* wt;     // FP16 bits, kWTotal, as MFMA operand tiles (guide.h)
+  const uint16_t* wf;     // the same in the training kernel's tile order
   float lo[3], inv_ext[3];   // position normalisation to the unit cube
   int32_t t_log2;            // table entries per level = 2^t_log2
   int32_t res[kGLevels];     // lattice resolution per level

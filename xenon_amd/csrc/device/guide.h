@@ -209,19 +209,51 @@ __device__ __forceinline__ f4v mma_tile(const _Float16* A, int lda, int r0, cons
   return acc + acc16;
 }
 
-// wave: Y (64 x N) = act(X (64 x K) W (K x N)); X, Y in LDS, W global.
-// relu: store FP16 ReLU output; else store FP32 (Y32).
-__device__ __forceinline__ void dense_fwd(const _Float16* X, int K, const _Float16* W, int N, _Float16* Y, float* Y32) {
-  const int lane = static_cast<int>(threadIdx.x & 63u);
-  for (int rt = 0; rt < 4; ++rt)
-    for (int ct = 0; ct < N / 16; ++ct) {
-      const f4v acc = mma_tile<false, false>(X, K, 16 * rt, W, N, 16 * ct, K);
+// wave: Y (64 x N) = act(X (64 x K) W (K x N)); X and Y rows in LDS (strides
+// ldx, ldy), wf: the layer's weights as row-order operand tiles in global
+// memory (row_tiled_index). A tile of weights is one 16-byte load per lane,
+// used for all 64 samples; the order of the sums is mma_tile's.
+// relu: store FP16 ReLU output to Y; else the first `cols` FP32 sums to Y32.
+// Row-order tiles of a K x N matrix: 32-input tile (ct, kt) at (ct (K/32) +
+// kt) 512, lane l's eight values W[32 kt + 8 (l/16) + j][16 ct + l % 16] at + 8
+// l + j; a last 16-input tile as in tiled_index.
+__device__ __forceinline__ int row_tiled_index(int k, int n, int K, int N) {
+  const int nkb = K >> 5, ct = n >> 4, li = n & 15;
+  if (k < (nkb << 5)) return ((ct * nkb + (k >> 5)) * 64 + ((k & 31) >> 3) * 16 + li) * 8 + (k & 7);
+  const int kk = k - (nkb << 5);
+  return (N >> 4) * nkb * 512 + (ct * 64 + (kk >> 2) * 16 + li) * 4 + (kk & 3);
+}
+template <int K, int N>
+__device__ __forceinline__ void dense_fwd(const _Float16* X, int ldx, const uint16_t* wf, _Float16* Y, float* Y32,
+                                          int ldy, int cols) {
+  typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+  constexpr int KB = K / 32;
+  const int lane = static_cast<int>(threadIdx.x & 63u), li = lane & 15, g = lane >> 4;
+  const _Float16* w = reinterpret_cast<const _Float16*>(wf);
+  for (int ct = 0; ct < N / 16; ++ct) {
+    h8 b[KB];
+    h4v b16;
+    for (int kt = 0; kt < KB; ++kt) b[kt] = *reinterpret_cast<const h8*>(w + (ct * KB + kt) * 512 + lane * 8);
+    if (K & 16) b16 = *reinterpret_cast<const h4v*>(w + (N / 16) * KB * 512 + ct * 256 + lane * 4);
+    for (int rt = 0; rt < 4; ++rt) {
+      const _Float16* x = X + (16 * rt + li) * ldx;
+      f4v acc = {0.f, 0.f, 0.f, 0.f};
+      for (int kt = 0; kt < KB; ++kt)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(*reinterpret_cast<const h8*>(x + 32 * kt + 8 * g), b[kt], acc, 0, 0,
+                                                     0);
+      if (K & 16) {
+        // its own accumulator (see mma_tile)
+        const f4v zero = {0.f, 0.f, 0.f, 0.f};
+        acc += __builtin_amdgcn_mfma_f32_16x16x16f16(*reinterpret_cast<const h4v*>(x + 32 * KB + 4 * g), b16, zero, 0, 0, 0);
+      }
+      const int col = 16 * ct + li;
       for (int j = 0; j < 4; ++j) {
-        const int r = 16 * rt + 4 * (lane >> 4) + j, col = 16 * ct + (lane & 15);
-        if (Y) Y[r * N + col] = static_cast<_Float16>(fmaxf(acc[j], 0.f));
-        else Y32[r * N + col] = acc[j];
+        const int r = 16 * rt + 4 * g + j;
+        if (Y) Y[r * ldy + col] = static_cast<_Float16>(fmaxf(acc[j], 0.f));
+        else if (col < cols) Y32[r * ldy + col] = acc[j];
       }
     }
+  }
   __syncthreads();
 }
 
@@ -335,16 +367,6 @@ __device__ __forceinline__ void guide_mlp_wave(_Float16* act, const h4v* wl) {
 __device__ __forceinline__ void guide_forward_wave(const GuideNet& net, f3 p, f3 n, _Float16* act, const h4v* wl) {
   guide_encode(net, p, n, act + (threadIdx.x & 63u) * kGIn);
   guide_mlp_wave(act, wl);
-}
-
-// wave: the full forward pass; lds_x holds the encodings (64 x 48).
-__device__ __forceinline__ void mlp_forward(const GuideNet& net, const _Float16* X, _Float16* H1, _Float16* H2,
-                                            _Float16* H3, float* out) {
-  const _Float16* w = reinterpret_cast<const _Float16*>(net.w);
-  dense_fwd(X, kGIn, w + kW1, kGHid, H1, nullptr);
-  dense_fwd(H1, kGHid, w + kW2, kGHid, H2, nullptr);
-  dense_fwd(H2, kGHid, w + kW3, kGHid, H3, nullptr);
-  dense_fwd(H3, kGHid, w + kW4, kGOut, nullptr, out);
 }
 
 // ---- mixture -----------------------------------------------------------------

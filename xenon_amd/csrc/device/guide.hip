@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstdint>
 
 #include "dbsdf.h"
 #include "dwave.h"
@@ -107,46 +108,100 @@ __device__ __forceinline__ float loss_grad(const float* raw, f3 w, float lam, fl
   return -lam * logf(q);
 }
 
-// wave: dW (K x N, global FP32) = A^T (K x 64) * G (64 x N); A: 64 x K rows.
+// Operand of a contraction over the 64 samples: 16 columns of a row-major
+// LDS matrix (row stride ld), lane l holding samples 32 s + 8 (l / 16) + j, j =
+// 0..7, of column c0 + l % 16 in step s.
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+struct SampleOp {
+  h8 v[2];
+};
+__device__ __forceinline__ SampleOp sample_op(const _Float16* A, int ld, int c0) {
+  const int lane = glane(), li = lane & 15, g = lane >> 4;
+  SampleOp o;
+  for (int s = 0; s < 2; ++s)
+    for (int j = 0; j < 8; ++j) o.v[s][j] = A[(32 * s + 8 * g + j) * ld + c0 + li];
+  return o;
+}
+
+// wave: dW (K x N, global FP32) = A^T (K x 64) * G (64 x N); A: 64 x K rows,
+// G: 64 rows of stride kGHid. Each column's operand is gathered once (64 or
+// 48 of them; gathered again for each of the 16 tiles they were four times
+// the LDS reads).
 // dW is this work-group's own slice of the partial-gradient buffer (summed
 // over work-groups by k_wgrad_reduce), so plain stores suffice.
-__device__ __forceinline__ void weight_grad(const _Float16* A, int K, const _Float16* G, int N, float* dW) {
+template <int K, int N>
+__device__ __forceinline__ void weight_grad(const _Float16* A, const _Float16* G, float* dW) {
   const int lane = glane();
-  for (int rt = 0; rt < K / 16; ++rt)
+  SampleOp b[N / 16];
+#pragma unroll
+  for (int ct = 0; ct < N / 16; ++ct) b[ct] = sample_op(G, kGHid, 16 * ct);
+  for (int rt = 0; rt < K / 16; ++rt) {
+    const SampleOp a = sample_op(A, K, 16 * rt);
+#pragma unroll
     for (int ct = 0; ct < N / 16; ++ct) {
-      const f4v acc = mma_tile<true, false>(A, K, 16 * rt, G, N, 16 * ct, 64);
+      f4v acc = {0.f, 0.f, 0.f, 0.f};
+      for (int s = 0; s < 2; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a.v[s], b[ct].v[s], acc, 0, 0, 0);
       for (int j = 0; j < 4; ++j) {
         const int r = 16 * rt + 4 * (lane >> 4) + j, col = 16 * ct + (lane & 15);
         dW[r * N + col] = acc[j];
       }
     }
+  }
+  __syncthreads();   // G is rewritten next
 }
 
-// wave: Gout (64 x K) = (G (64 x N) * W^T) masked by (H > 0) when H != null;
-// W: K x N row-major global. FP16 result, or FP32 into Gout32.
-__device__ __forceinline__ void input_grad(const _Float16* G, int N, const _Float16* W, int K, const _Float16* H,
-                                           _Float16* Gout, float* Gout32) {
+// wave: G (64 rows of stride kGHid, N columns) becomes G * W^T (K columns)
+// masked by (H > 0), FP16, in place: a 16-row tile is read whole before it is
+// written. W: K x N row-major global.
+template <int N, int K>
+__device__ __forceinline__ void input_grad(_Float16* G, const _Float16* W, const _Float16* H) {
   const int lane = glane();
-  for (int rt = 0; rt < 4; ++rt)
-    for (int ct = 0; ct < K / 16; ++ct) {
-      const f4v acc = mma_tile<false, true>(G, N, 16 * rt, W, N, 16 * ct, N);
+  for (int rt = 0; rt < 4; ++rt) {
+    f4v acc[K / 16];
+#pragma unroll
+    for (int ct = 0; ct < K / 16; ++ct) acc[ct] = mma_tile<false, true>(G, kGHid, 16 * rt, W, N, 16 * ct, N);
+    __syncthreads();
+#pragma unroll
+    for (int ct = 0; ct < K / 16; ++ct)
       for (int j = 0; j < 4; ++j) {
         const int r = 16 * rt + 4 * (lane >> 4) + j, col = 16 * ct + (lane & 15);
-        float v = acc[j];
-        if (H && !(static_cast<float>(H[r * K + col]) > 0.f)) v = 0.f;
-        if (Gout) Gout[r * K + col] = static_cast<_Float16>(fminf(fmaxf(v, -kHalfMax), kHalfMax));
-        else Gout32[r * K + col] = v;
+        const float v = static_cast<float>(H[r * K + col]) > 0.f ? acc[ct][j] : 0.f;
+        G[r * kGHid + col] = static_cast<_Float16>(fminf(fmaxf(v, -kHalfMax), kHalfMax));
       }
-    }
+  }
   __syncthreads();
 }
 
+// The gradient of the hash-grid features (the first 32 inputs), FP32 rows of
+// stride kFRow written over G: last row tile first, so that a tile's rows
+// (16 kFRow floats from 16 rt kFRow) fall on rows of G already read.
+constexpr int kFRow = 40;
+__device__ __forceinline__ void feature_grad(const _Float16* G, const _Float16* W, float* F) {
+  const int lane = glane();
+  for (int rt = 3; rt >= 0; --rt) {
+    f4v acc[2];
+#pragma unroll
+    for (int ct = 0; ct < 2; ++ct) acc[ct] = mma_tile<false, true>(G, kGHid, 16 * rt, W, kGHid, 16 * ct, kGHid);
+    __syncthreads();
+#pragma unroll
+    for (int ct = 0; ct < 2; ++ct)
+      for (int j = 0; j < 4; ++j) F[(16 * rt + 4 * (lane >> 4) + j) * kFRow + 16 * ct + (lane & 15)] = acc[ct][j];
+  }
+  __syncthreads();
+}
+
+// 40 KB: four work-groups (one wave each) on a CU's 160 KB, one per SIMD. The
+// gradient rows G and the FP32 rows F (raw outputs before, feature gradients
+// after back-propagation) take turns in one region.
 struct TrainLds {
   _Float16 X[64 * kGIn];
   _Float16 H1[64 * kGHid], H2[64 * kGHid], H3[64 * kGHid];
-  _Float16 Ga[64 * kGHid], Gb[64 * kGHid];
-  float F[64 * kGOut];
+  union {
+    _Float16 G[64 * kGHid];
+    float F[64 * kFRow];
+  };
 };
+static_assert(sizeof(TrainLds) == 40960 && kFRow >= 5 * kGLobes, "four work-groups per CU");
 
 }  // namespace
 
@@ -429,8 +484,9 @@ __global__ void __launch_bounds__(256) k_guide_select(WaveBuffers B, const float
   if (threadIdx.x == 0 && t > 0.f) atomicAdd(lam_sum, t);
 }
 
-// Rearranges the FP16 row-major weights into MFMA operand tiles.
-__global__ void __launch_bounds__(256) k_tile_weights(const uint16_t* w, uint16_t* wt) {
+// Rearranges the FP16 row-major weights into MFMA operand tiles: wt for the
+// register-resident forward pass, wf for the training kernel's.
+__global__ void __launch_bounds__(256) k_tile_weights(const uint16_t* w, uint16_t* wt, uint16_t* wf) {
   const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
   if (i >= kWTotal) return;
   int off, K, N;
@@ -445,18 +501,22 @@ __global__ void __launch_bounds__(256) k_tile_weights(const uint16_t* w, uint16_
   }
   const int r = i - off, k = r / N, c = r - k * N;
   wt[off + tiled_index(k, c, K, N)] = w[i];
+  wf[off + row_tiled_index(k, c, K, N)] = w[i];
 }
 
 // Forward + loss + backward over n training samples; accumulates the
 // gradients of sum_i l_i into grid_g (L x T x 2) and w_g (kWTotal), and the
 // summed loss into loss_sum.
+// fg non-null: the gradients of the grid's features go there instead (fstride
+// samples a level), for k_guide_scatter.
 // With n_dev non-null the record count is cnt = min(*n_dev, n); the kernel
 // trains on slice `slice` of `nslices` equal parts of [0, cnt) and takes
 // lam_scale = cnt / *lam_sum_dev (the batch mean of lambda scaled to 1).
 __global__ void __launch_bounds__(64) k_guide_train(GuideNet net, int n, const float* pos, const float* nrm,
                                                     const float* dir, const float* lam, float lam_scale,
                                                     const uint32_t* n_dev, const float* lam_sum_dev, int slice,
-                                                    int nslices, float* grid_g, float* w_part, float* loss_sum) {
+                                                    int nslices, float* grid_g, float* w_part, float* loss_sum,
+                                                    float2* fg, size_t fstride) {
   __shared__ __align__(16) TrainLds s;
   float* w_g = w_part + static_cast<size_t>(blockIdx.x) * kWTotal;   // this work-group's weight gradients
   int begin = 0;
@@ -477,30 +537,37 @@ __global__ void __launch_bounds__(64) k_guide_train(GuideNet net, int n, const f
   const float lm = ok ? lam[i] * lam_scale : 0.f;
   guide_encode(net, p, nn, s.X + lane * kGIn);
   __syncthreads();
-  mlp_forward(net, s.X, s.H1, s.H2, s.H3, s.F);
-  // output gradients -> Ga (64 x 48, FP16)
+  dense_fwd<kGIn, kGHid>(s.X, kGIn, net.wf + kW1, s.H1, nullptr, kGHid, kGHid);
+  dense_fwd<kGHid, kGHid>(s.H1, kGHid, net.wf + kW2, s.H2, nullptr, kGHid, kGHid);
+  dense_fwd<kGHid, kGHid>(s.H2, kGHid, net.wf + kW3, s.H3, nullptr, kGHid, kGHid);
+  dense_fwd<kGHid, kGOut>(s.H3, kGHid, net.wf + kW4, nullptr, s.F, kFRow, 5 * kGLobes);
+  // output gradients -> G (64 x 48, FP16), over the outputs
   float g[kGOut];
-  const float l = loss_grad(s.F + lane * kGOut, w, lm, g);
-  for (int k = 0; k < kGOut; ++k) s.Ga[lane * kGOut + k] = static_cast<_Float16>(g[k]);
+  const float l = loss_grad(s.F + lane * kFRow, w, lm, g);
+  __syncthreads();
+  for (int k = 0; k < kGOut; ++k) s.G[lane * kGHid + k] = static_cast<_Float16>(g[k]);
   const float lsum = g_wave_sumf(ok ? l : 0.f);
   if (lane == 0) atomicAdd(loss_sum, lsum);
   __syncthreads();
-  // layer 4: dW4 = H3^T G4 ; G3 = G4 W4^T * (H3 > 0)
-  weight_grad(s.H3, kGHid, s.Ga, kGOut, w_g + kW4);
+  // layer 4: dW4 = H3^T G4 ; G3 = G4 W4^T * (H3 > 0); and so on down
   const _Float16* W = reinterpret_cast<const _Float16*>(net.w);
-  input_grad(s.Ga, kGOut, W + kW4, kGHid, s.H3, s.Gb, nullptr);
-  weight_grad(s.H2, kGHid, s.Gb, kGHid, w_g + kW3);
-  input_grad(s.Gb, kGHid, W + kW3, kGHid, s.H2, s.Ga, nullptr);
-  weight_grad(s.H1, kGHid, s.Ga, kGHid, w_g + kW2);
-  input_grad(s.Ga, kGHid, W + kW2, kGHid, s.H1, s.Gb, nullptr);
-  weight_grad(s.X, kGIn, s.Gb, kGHid, w_g + kW1);
-  input_grad(s.Gb, kGHid, W + kW1, kGIn, nullptr, nullptr, s.F);
-  // hash-grid scatter of the encoding gradient (first 32 inputs)
-  if (ok) {
+  weight_grad<kGHid, kGOut>(s.H3, s.G, w_g + kW4);
+  input_grad<kGOut, kGHid>(s.G, W + kW4, s.H3);
+  weight_grad<kGHid, kGHid>(s.H2, s.G, w_g + kW3);
+  input_grad<kGHid, kGHid>(s.G, W + kW3, s.H2);
+  weight_grad<kGHid, kGHid>(s.H1, s.G, w_g + kW2);
+  input_grad<kGHid, kGHid>(s.G, W + kW2, s.H1);
+  weight_grad<kGIn, kGHid>(s.X, s.G, w_g + kW1);
+  feature_grad(s.G, W + kW1, s.F);
+  if (fg) {   // the feature gradients, level by level, for k_guide_scatter
+    const size_t at = static_cast<size_t>(blockIdx.x) * 64u + static_cast<size_t>(lane);
+    for (int lv = 0; lv < kGLevels; ++lv)
+      fg[lv * fstride + at] = make_float2(s.F[lane * kFRow + 2 * lv], s.F[lane * kFRow + 2 * lv + 1]);
+  } else if (ok) {   // hash-grid scatter of the encoding gradient (first 32 inputs)
     const f3 q = guide_unit_pos(net, p);
     const uint32_t T = 1u << net.t_log2;
     for (int lv = 0; lv < kGLevels; ++lv) {
-      const float g0 = s.F[lane * kGIn + 2 * lv], g1 = s.F[lane * kGIn + 2 * lv + 1];
+      const float g0 = s.F[lane * kFRow + 2 * lv], g1 = s.F[lane * kFRow + 2 * lv + 1];
       if (g0 == 0.f && g1 == 0.f) continue;
       float* gl = grid_g + static_cast<size_t>(lv) * T * 2u;
       for (int c = 0; c < 8; ++c) {
@@ -513,6 +580,96 @@ __global__ void __launch_bounds__(64) k_guide_train(GuideNet net, int n, const f
       }
     }
   }
+}
+
+// Adds the feature gradients of a k_guide_train launch to the grid's: a
+// work-group takes a table (kScatterSlots consecutive slots of one level) and
+// one of the level's parts of the samples, and sums in LDS what falls on its
+// slots. Where a level has one part it adds the sums to grid_g, which no
+// other work-group touches then; with more it writes them to `part` for
+// k_grid_reduce. Bound by the LDS adds (a wave's takes about 170 cycles), so
+// every level, which has the same number of them, gets as many work-groups.
+// In place of 256 global atomics a sample, at 18.6 G/s nine tenths of a
+// training step: 65536 samples of 2^15 slots, 913 us for k_guide_train with the
+// atomics, 68 without them, 100 here and 10 in k_grid_reduce (174 here where
+// every table had as many work-groups).
+struct ScatterPlan {
+  int32_t first[kGLevels + 1];   // first work-group of each level
+  int32_t tables[kGLevels], parts[kGLevels];
+};
+
+__global__ void __launch_bounds__(1024) k_guide_scatter(GuideNet net, ScatterPlan plan, int n, const float* pos,
+                                                        const uint32_t* n_dev, int slice, int nslices,
+                                                        const float2* fg, size_t fstride, float2* part, float* grid_g) {
+  __shared__ float tab[2][kScatterSlots];
+  int begin = 0;
+  if (n_dev) {
+    const uint32_t cnt = min(*n_dev, static_cast<uint32_t>(n));
+    begin = static_cast<int>((static_cast<uint64_t>(cnt) * slice) / nslices);
+    n = static_cast<int>((static_cast<uint64_t>(cnt) * (slice + 1)) / nslices);
+  }
+  int lv = 0;
+  while (static_cast<int>(blockIdx.x) >= plan.first[lv + 1]) ++lv;
+  const uint32_t local = blockIdx.x - static_cast<uint32_t>(plan.first[lv]), nt = static_cast<uint32_t>(plan.tables[lv]);
+  const uint32_t s0 = (local % nt) * kScatterSlots, y = local / nt, parts = static_cast<uint32_t>(plan.parts[lv]);
+  for (uint32_t k = threadIdx.x; k < kScatterSlots; k += blockDim.x) tab[0][k] = tab[1][k] = 0.f;
+  __syncthreads();
+  const uint64_t len = n > begin ? static_cast<uint64_t>(n - begin) : 0u;
+  const int i1 = begin + static_cast<int>(len * (y + 1u) / parts);
+  for (int i = begin + static_cast<int>(len * y / parts) + static_cast<int>(threadIdx.x); i < i1;
+       i += static_cast<int>(blockDim.x)) {
+    const float2 g = fg[lv * fstride + static_cast<size_t>(i - begin)];
+    if (g.x == 0.f && g.y == 0.f) continue;
+    const f3 q = guide_unit_pos(net, f3{pos[3 * static_cast<size_t>(i)], pos[3 * static_cast<size_t>(i) + 1],
+                                        pos[3 * static_cast<size_t>(i) + 2]});
+    for (int c = 0; c < 8; ++c) {
+      uint32_t slot;
+      float wt;
+      grid_corner(net, q, lv, c, slot, wt);
+      const uint32_t at = slot - s0;
+      if (wt == 0.f || at >= static_cast<uint32_t>(kScatterSlots)) continue;
+      atomicAdd(&tab[0][at], wt * g.x);
+      atomicAdd(&tab[1][at], wt * g.y);
+    }
+  }
+  __syncthreads();
+  if (parts > 1u) {
+    float2* to = part + static_cast<size_t>(blockIdx.x) * kScatterSlots;
+    for (uint32_t k = threadIdx.x; k < kScatterSlots; k += blockDim.x) to[k] = make_float2(tab[0][k], tab[1][k]);
+    return;
+  }
+  const uint32_t T = 1u << net.t_log2;
+  float2* gl = reinterpret_cast<float2*>(grid_g) + static_cast<size_t>(lv) * T + s0;
+  const uint32_t most = min(static_cast<uint32_t>(kScatterSlots), T - s0);
+  for (uint32_t k = threadIdx.x; k < most; k += blockDim.x) {
+    const float a = tab[0][k], b = tab[1][k];
+    if (a != 0.f || b != 0.f) {
+      const float2 v = gl[k];
+      gl[k] = make_float2(v.x + a, v.y + b);
+    }
+  }
+}
+
+// Adds the sums of a slot's parts to grid_g, a thread a slot: one pass over
+// the partial tables (at most kScatterTables of them, 34 MB). blockIdx.y is
+// the level.
+__global__ void __launch_bounds__(256) k_grid_reduce(ScatterPlan plan, int t_log2, const float2* part, float* grid_g) {
+  const int lv = static_cast<int>(blockIdx.y), parts = plan.parts[lv];
+  const uint32_t slot = blockIdx.x * 256u + threadIdx.x, table = slot / kScatterSlots;
+  const uint32_t nt = static_cast<uint32_t>(plan.tables[lv]);
+  if (parts == 1 || table >= nt || slot >= (1u << t_log2)) return;
+  const size_t step = static_cast<size_t>(nt) * kScatterSlots;
+  const float2* from = part + static_cast<size_t>(plan.first[lv]) * kScatterSlots + slot;
+  float a = 0.f, b = 0.f;
+  for (int p = 0; p < parts; ++p) {
+    const float2 v = from[p * step];
+    a += v.x;
+    b += v.y;
+  }
+  if (a == 0.f && b == 0.f) return;
+  float2* to = reinterpret_cast<float2*>(grid_g) + (static_cast<size_t>(lv) << t_log2) + slot;
+  const float2 v = *to;
+  *to = make_float2(v.x + a, v.y + b);
 }
 
 // Sums the per-work-group weight gradients of a k_guide_train launch into
@@ -595,8 +752,40 @@ hipError_t launch_guide_train(hipStream_t s, const GuideNet& net, int n, const f
                               float* w_g, float* loss_sum) {
   if (n <= 0) return hipSuccess;
   const int blocks = guide_train_blocks(n, n_dev != nullptr, nslices);
+  // k_guide_scatter for calls of more than 4096 samples and grids of up to
+  // 2^20 slots a level. A work-group goes over its samples' corners whether or
+  // not they fall on its table, so its cost grows with the tables; that of the
+  // atomics does not. A whole call with host samples and an Adam step,
+  // scatter / atomics: 65536 samples, 2^15 slots 0.52 / 1.23 ms, 2^17
+  // 0.53 / 1.25, 2^19 0.69 / 1.31, 2^20 0.94 / 1.45, 2^21 1.35 / 1.67, 2^22
+  // 2.00 / 2.08; 8192 samples, 2^14 0.33 / 0.37, 2^17 0.25 / 0.29, 2^20
+  // 0.46 / 0.48, 2^21 0.71 / 0.69; 4096 samples, 2^14 0.25 / 0.25, 2^17
+  // 0.22 / 0.21; 2048 samples, 2^14 0.20 / 0.18 (two launches more).
+  const int most = blocks * 64;   // samples
+  const bool scatter = net.t_log2 <= 20 && most > 2 * kScatterSamples;
+  ScatterPlan plan{};
+  int tables_most = 1;
+  for (int l = 0; l < kGLevels; ++l) {
+    const uint64_t d = static_cast<uint64_t>(net.res[l]) + 1u, T = uint64_t(1) << net.t_log2;
+    const uint64_t slots = std::min(d * d * d, T);
+    plan.tables[l] = static_cast<int32_t>((slots + kScatterSlots - 1) / kScatterSlots);
+    plan.parts[l] = std::max(1, std::min(kScatterTables / kGLevels / plan.tables[l], most / kScatterSamples));
+    plan.first[l + 1] = plan.first[l] + plan.tables[l] * plan.parts[l];
+    if (plan.parts[l] > 1) tables_most = std::max(tables_most, plan.tables[l]);
+  }
+  const size_t fstride = static_cast<size_t>(blocks) * 64u;
+  float2* fg = scatter ? reinterpret_cast<float2*>(w_part + static_cast<size_t>(blocks) * kWTotal) : nullptr;
+  float2* part = scatter ? fg + static_cast<size_t>(kGLevels) * fstride : nullptr;
   hipLaunchKernelGGL(k_guide_train, dim3(blocks), dim3(64), 0, s, net, n, pos, nrm, dir, lam, lam_scale, n_dev,
-                     lam_sum_dev, slice, nslices, grid_g, w_part, loss_sum);
+                     lam_sum_dev, slice, nslices, grid_g, w_part, loss_sum, fg, fstride);
+  if (scatter) {
+    hipLaunchKernelGGL(k_guide_scatter, dim3(plan.first[kGLevels]), dim3(1024), 0, s, net, plan, n, pos, n_dev, slice,
+                       nslices, static_cast<const float2*>(fg), fstride, part, grid_g);
+    // (the first levels have several parts: those of few tables; their
+    // work-groups, at most kScatterTables, index `part`)
+    hipLaunchKernelGGL(k_grid_reduce, dim3(tables_most * (kScatterSlots / 256), kGLevels), dim3(256), 0, s, plan,
+                         net.t_log2, static_cast<const float2*>(part), grid_g);
+  }
   const dim3 rgrid((kWTotal + 255) / 256, (blocks + kRedChunk - 1) / kRedChunk);
   hipLaunchKernelGGL(k_wgrad_reduce, rgrid, dim3(256), 0, s, w_part, w_g, n, n_dev, slice, nslices);
   return hipGetLastError();
@@ -633,8 +822,8 @@ hipError_t launch_guide_collect(hipStream_t s, const WaveBuffers& B, float* lam_
   return hipGetLastError();
 }
 
-hipError_t launch_tile_weights(hipStream_t s, const uint16_t* w, uint16_t* wt) {
-  hipLaunchKernelGGL(k_tile_weights, dim3((kWTotal + 255) / 256), dim3(256), 0, s, w, wt);
+hipError_t launch_tile_weights(hipStream_t s, const uint16_t* w, uint16_t* wt, uint16_t* wf) {
+  hipLaunchKernelGGL(k_tile_weights, dim3((kWTotal + 255) / 256), dim3(256), 0, s, w, wt, wf);
   return hipGetLastError();
 }
 

@@ -36,8 +36,15 @@ hipError_t launch_guide_eval(hipStream_t s, const GuideNet& net, int n, const fl
                              float* raw);
 hipError_t launch_guide_query(hipStream_t s, const GuideNet& net, int n, const float* pos, const float* nrm,
                               const float* u, float* dir, float* pdf);
-// Work-groups of one launch_guide_train call (each needs kWTotal floats of
-// w_part): n records, or with device counts the largest slice of n.
+// Work-groups of one launch_guide_train call: n records, or with device
+// counts the largest slice of n. w_part has kTrainPart floats for each (its
+// weight gradients and its 64 samples' feature gradients), and kScatterPart
+// for k_guide_scatter's partial tables.
+constexpr size_t kTrainPart = kWTotal + 64 * kGLevels * kGFeat;
+constexpr int kScatterSlots = 16384;     // grid slots of a table: two features each, 128 KB of LDS
+constexpr int kScatterTables = 256;      // partial tables at most
+constexpr int kScatterSamples = 2048;    // samples a part of the scatter has at least
+constexpr size_t kScatterPart = size_t(kScatterTables) * kScatterSlots * kGFeat;
 int guide_train_blocks(int n, bool device_count, int nslices);
 // Forward/backward over the records; grid gradients are added to grid_g,
 // weight gradients go through w_part (per work-group) and are added to w_g.
@@ -48,7 +55,7 @@ hipError_t launch_guide_train(hipStream_t s, const GuideNet& net, int n, const f
 hipError_t launch_guide_adam(hipStream_t s, float* master, uint16_t* half_copy, float* grad, float* m, float* v,
                              size_t count, float lr, float b1, float b2, float eps, float bc1, float bc2,
                              float grad_scale, const uint32_t* n_dev, uint32_t cap, int nslices);
-hipError_t launch_tile_weights(hipStream_t s, const uint16_t* w, uint16_t* wt);
+hipError_t launch_tile_weights(hipStream_t s, const uint16_t* w, uint16_t* wt, uint16_t* wf);
 // Guide mixtures for the hits of queue qi (encode, then MLP); feat: 6 uint4
 // per queue entry of scratch.
 hipError_t launch_guide_infer(hipStream_t s, const WaveBuffers& B, int qi, int depth, const GuideNet& net, uint4* feat,

@@ -55,6 +55,7 @@ struct GuideState {
   float *w_m = nullptr, *w_g = nullptr, *w_am = nullptr, *w_av = nullptr;
   uint16_t* w_h = nullptr;
   uint16_t* w_t = nullptr;        // FP16 weights as MFMA operand tiles
+  uint16_t* w_f = nullptr;        // the same in the training kernel's tile order
   float* loss = nullptr;
   size_t ngrid = 0;
   int step = 0;
@@ -729,7 +730,7 @@ int ensure_graph(xnh_ctx* c, int depth) {
   return XNH_OK;
 }
 
-// Room for the per-work-group weight gradients of a training launch of
+// Room for the per-work-group gradients of a training launch of
 // `blocks` work-groups.
 static int ensure_wpart(xnh_ctx* c, int blocks) {
   GuideState& g = c->guide;
@@ -742,7 +743,7 @@ static int ensure_wpart(xnh_ctx* c, int blocks) {
     g.w_part = nullptr;
     g.w_part_blocks = 0;
   }
-  const int rc = dev_alloc(c, g.allocs, &g.w_part, static_cast<size_t>(blocks) * kWTotal);
+  const int rc = dev_alloc(c, g.allocs, &g.w_part, static_cast<size_t>(blocks) * kTrainPart + kScatterPart);
   if (rc != XNH_OK) return rc;
   g.w_part_blocks = blocks;
   return XNH_OK;
@@ -781,7 +782,7 @@ int guide_train_batch(xnh_ctx* c) {
                                      bc1, bc2, 1.f, g.t_n, static_cast<uint32_t>(R), K));
     HIP_OR_FAIL(c, launch_guide_adam(s, g.w_m, g.w_h, g.w_g, g.w_am, g.w_av, size_t(kWTotal), lr, b1, b2, eps, bc1,
                                      bc2, 1.f, g.t_n, static_cast<uint32_t>(R), K));
-    HIP_OR_FAIL(c, launch_tile_weights(s, g.w_h, g.w_t));
+    HIP_OR_FAIL(c, launch_tile_weights(s, g.w_h, g.w_t, g.w_f));
   }
   const float a = g.cfg.warmup_steps > 0
                       ? g.cfg.guide_fraction * std::min(1.f, static_cast<float>(g.step) / g.cfg.warmup_steps)
@@ -1679,6 +1680,7 @@ int xnh_guide_enable(xnh_ctx* c, const xnh_guide_config* cfg_in) {
   if (rc == XNH_OK) rc = dev_alloc(c, g.allocs, &g.w_av, size_t(kWTotal));
   if (rc == XNH_OK) rc = dev_alloc(c, g.allocs, &g.w_h, size_t(kWTotal));
   if (rc == XNH_OK) rc = dev_alloc(c, g.allocs, &g.w_t, size_t(kWTotal));
+  if (rc == XNH_OK) rc = dev_alloc(c, g.allocs, &g.w_f, size_t(kWTotal));
   if (rc == XNH_OK) rc = dev_alloc(c, g.allocs, &g.loss, size_t(1));
   const size_t R = static_cast<size_t>(cfg.train_batch);
   // records: one per guided vertex of a recording path, at most 2^25 a
@@ -1714,6 +1716,7 @@ int xnh_guide_enable(xnh_ctx* c, const xnh_guide_config* cfg_in) {
   g.net.grid = g.grid_h;
   g.net.w = g.w_h;
   g.net.wt = g.w_t;
+  g.net.wf = g.w_f;
   g.mix_stride = static_cast<uint32_t>(gq);
   g.slot_cap = static_cast<uint32_t>(gcap);
   g.rec_cap = static_cast<uint32_t>(RC);
@@ -1756,7 +1759,7 @@ int xnh_guide_set_params(xnh_ctx* c, const float* grid, const float* w) {
   HIP_OR_FAIL(c, hipMemcpyAsync(g.w_m, w, size_t(kWTotal) * 4, hipMemcpyHostToDevice, s));
   HIP_OR_FAIL(c, launch_to_half(s, g.grid_m, g.grid_h, g.ngrid));
   HIP_OR_FAIL(c, launch_to_half(s, g.w_m, g.w_h, size_t(kWTotal)));
-  HIP_OR_FAIL(c, launch_tile_weights(s, g.w_h, g.w_t));
+  HIP_OR_FAIL(c, launch_tile_weights(s, g.w_h, g.w_t, g.w_f));
   for (float* p : {g.grid_g, g.grid_am, g.grid_av}) HIP_OR_FAIL(c, hipMemsetAsync(p, 0, g.ngrid * 4, s));
   for (float* p : {g.w_g, g.w_am, g.w_av}) HIP_OR_FAIL(c, hipMemsetAsync(p, 0, size_t(kWTotal) * 4, s));
   HIP_OR_FAIL(c, hipStreamSynchronize(s));
@@ -1846,7 +1849,7 @@ static int guide_step(xnh_ctx* c, int n, const float* dp, const float* dn, const
                                      bc1, bc2, gs, nullptr, 0u, 1));
     HIP_OR_FAIL(c, launch_guide_adam(s, g.w_m, g.w_h, g.w_g, g.w_am, g.w_av, size_t(kWTotal), lr, b1, b2, eps, bc1,
                                      bc2, gs, nullptr, 0u, 1));
-    HIP_OR_FAIL(c, launch_tile_weights(s, g.w_h, g.w_t));
+    HIP_OR_FAIL(c, launch_tile_weights(s, g.w_h, g.w_t, g.w_f));
   }
   return XNH_OK;
 }
