@@ -98,9 +98,9 @@ __device__ __forceinline__ float Lambda_ggx(f3 w, float ax, float ay) {
   const float a2 = (cp * ax) * (cp * ax) + (sp * ay) * (sp * ay);
   return (-1.f + sqrtf(1.f + a2 * t2)) * 0.5f;
 }
-__device__ __forceinline__ float G1_ggx(f3 w, float ax, float ay) { return 1.f / (1.f + Lambda_ggx(w, ax, ay)); }
+__device__ __forceinline__ float G1_ggx(f3 w, float ax, float ay) { return recip(1.f + Lambda_ggx(w, ax, ay)); }
 __device__ __forceinline__ float G2_ggx(f3 o, f3 i, float ax, float ay) {
-  return 1.f / (1.f + Lambda_ggx(o, ax, ay) + Lambda_ggx(i, ax, ay));
+  return recip(1.f + Lambda_ggx(o, ax, ay) + Lambda_ggx(i, ax, ay));
 }
 
 __device__ __forceinline__ float fresnel_d(float ci, float ior) {
@@ -129,19 +129,21 @@ __device__ __forceinline__ f3 fresnel_s(float c, f3 f0) {
 __device__ __forceinline__ f3 cosine_dir(float u1, float u2) {
   const float r = sqrtf(u1);
   const float phi = 2.0f * kPiD * u2;
-  return f3{r * cos_r(phi), r * sin_r(phi), sqrtf(smax(0.0f, 1.0f - u1))};
+  const SinCos sc = sincos_r(phi);
+  return f3{r * sc.c, r * sc.s, sqrtf(smax(0.0f, 1.0f - u1))};
 }
 
 // Heitz 2018 visible-normal sampling (bsdf.h:164-190).
 __device__ __forceinline__ f3 vndf(f3 wo, float ax, float ay, float u1, float u2) {
   const f3 vh = normalize(f3{ax * wo.x, ay * wo.y, wo.z});
   const float l2 = vh.x * vh.x + vh.y * vh.y;
-  const f3 t1 = (l2 > 1e-7f) ? f3{-vh.y, vh.x, 0.f} * (1.f / sqrtf(l2)) : f3{1.f, 0.f, 0.f};
+  const f3 t1 = (l2 > 1e-7f) ? f3{-vh.y, vh.x, 0.f} * recip(sqrtf(l2)) : f3{1.f, 0.f, 0.f};
   const f3 t2 = cross(vh, t1);
   const float r = sqrtf(u1);
   const float phi = 2.0f * kPiD * u2;
-  const float p1 = r * cos_r(phi);
-  float p2 = r * sin_r(phi);
+  const SinCos sc = sincos_r(phi);
+  const float p1 = r * sc.c;
+  float p2 = r * sc.s;
   const float s = 0.5f * (1.0f + vh.z);
   p2 = (1.0f - s) * sqrtf(smax(0.f, 1.0f - p1 * p1)) + s * p2;
   const f3 nh = p1 * t1 + p2 * t2 + sqrtf(smax(0.f, 1.0f - p1 * p1 - p2 * p2)) * vh;

@@ -608,7 +608,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGuide
             const float d2 = len2(sdv);
             const float dist = sqrtf(d2);
             if (dist > 1e-6f) {
-              const f3 wi = sdv / dist;
+              const f3 wi = sdv * recip(dist);
               const float cl = smax(0.0f, dot(xyz(l3), -wi));
               const Frame fr(sf.gn);
               const f3 wo_l = fr.local(-d);
