@@ -363,6 +363,9 @@ int xnh_image_noise_stats_noalloc(xnh_ctx* ctx, const float* rgb_dev, int32_t wi
  * framebuffer row H-1-r). */
 int xnh_image_rgb8(xnh_ctx* ctx, const float* rgb, int32_t width, int32_t height, uint8_t* out);
 
+/* The running average as the swapchain holds it: W*H*3 floats, rows top
+ * first (cpu_tiled.cpp:224-234). */
+int xnh_read_frame(xnh_ctx* ctx, float* rgb_out);
 /* Copies the raw per-pixel sums (W*H*3) and returns the sample count. */
 int xnh_read_accum(xnh_ctx* ctx, float* sum_out, int32_t* spp_out);
 int xnh_reset(xnh_ctx* ctx);

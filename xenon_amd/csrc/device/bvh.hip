@@ -26,7 +26,6 @@
 #include <hip/hip_runtime.h>
 
 #include <cstring>
-#include <vector>
 
 #include <rocprim/rocprim.hpp>
 
@@ -364,35 +363,56 @@ hipError_t refit_blas_device(hipStream_t s, xnh_bvh_node* nodes, int nn, const u
   return hipGetLastError();
 }
 
+namespace {
+
+// The build's buffers in its scratch (a null base: only their total size).
+struct BuildMem {
+  float *cen, *pb, *bounds;
+  uint32_t *k0, *k1, *v0, *v1, *left, *right, *size, *parent, *flag, *pos;
+  char* tmp;
+  size_t tmp_bytes, total;
+  BuildMem(char* base, int n, size_t sort_bytes) : tmp_bytes(sort_bytes), total(0) {
+    const size_t N = static_cast<size_t>(n), NN = 2 * N - 1;
+    auto take = [&](size_t bytes) {
+      char* p = base + total;
+      total += (bytes + 255) & ~size_t(255);
+      return p;
+    };
+    cen = reinterpret_cast<float*>(take(12 * N));
+    pb = reinterpret_cast<float*>(take(24 * 1024));
+    bounds = reinterpret_cast<float*>(take(24));
+    for (uint32_t** p : {&k0, &k1, &v0, &v1, &left, &right, &size}) *p = reinterpret_cast<uint32_t*>(take(4 * N));
+    for (uint32_t** p : {&parent, &flag, &pos}) *p = reinterpret_cast<uint32_t*>(take(4 * NN));
+    tmp = take(sort_bytes);
+  }
+};
+
+hipError_t sort_bytes(hipStream_t s, int n, size_t* bytes) {
+  uint32_t* const none = nullptr;
+  *bytes = 0;
+  return rocprim::radix_sort_pairs(nullptr, *bytes, none, none, none, none, static_cast<size_t>(n), 0, 30, s);
+}
+
+}  // namespace
+
+hipError_t build_blas_scratch(hipStream_t s, int n, size_t* bytes) {
+  size_t sb = 0;
+  const hipError_t e = sort_bytes(s, n, &sb);
+  *bytes = BuildMem(nullptr, n, sb).total;
+  return e;
+}
+
 hipError_t build_blas_device(hipStream_t s, const float* vx, const float* vy, const float* vz, const int32_t* idx,
-                             int n, xnh_bvh_node* nodes, uint32_t* prims, uint32_t* err) {
+                             int n, xnh_bvh_node* nodes, uint32_t* prims, uint32_t* err, char* scratch) {
   if (n < 2) return hipErrorInvalidValue;   // the caller builds single-triangle trees itself
   const int nn = 2 * n - 1;
   const int nb = blocks_for(n) < 1024 ? blocks_for(n) : 1024;
-  std::vector<void*> mem;
-  hipError_t e = hipSuccess;
-  auto alloc = [&](size_t bytes) -> void* {
-    void* p = nullptr;
-    if (e == hipSuccess) e = hipMalloc(&p, bytes < 4 ? 4 : bytes);
-    if (e == hipSuccess) mem.push_back(p);
-    return p;
-  };
-  float* cen = static_cast<float*>(alloc(sizeof(float) * 3 * n));
-  float* pb = static_cast<float*>(alloc(sizeof(float) * 6 * nb));
-  float* bounds = static_cast<float*>(alloc(sizeof(float) * 6));
-  uint32_t* k0 = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * n));
-  uint32_t* k1 = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * n));
-  uint32_t* v0 = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * n));
-  uint32_t* v1 = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * n));
-  uint32_t* left = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * n));
-  uint32_t* right = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * n));
-  uint32_t* parent = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * nn));
-  uint32_t* size = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * n));
-  uint32_t* flag = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * nn));
-  uint32_t* pos = static_cast<uint32_t*>(alloc(sizeof(uint32_t) * nn));
-  size_t tmp_bytes = 0;
-  if (e == hipSuccess) e = rocprim::radix_sort_pairs(nullptr, tmp_bytes, k0, k1, v0, v1, static_cast<size_t>(n), 0, 30, s);
-  void* tmp = alloc(tmp_bytes);
+  size_t sb = 0;
+  hipError_t e = sort_bytes(s, n, &sb);
+  const BuildMem m(scratch, n, sb);
+  float *cen = m.cen, *pb = m.pb, *bounds = m.bounds;
+  uint32_t *k0 = m.k0, *k1 = m.k1, *v0 = m.v0, *v1 = m.v1, *left = m.left, *right = m.right, *size = m.size,
+           *parent = m.parent, *flag = m.flag, *pos = m.pos;
   if (e == hipSuccess) e = hipMemsetAsync(parent, 0xFF, sizeof(uint32_t) * nn, s);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_lb_centres, dim3(nb), dim3(kT), 0, s, vx, vy, vz, idx, n, cen, pb);
@@ -400,7 +420,7 @@ hipError_t build_blas_device(hipStream_t s, const float* vx, const float* vy, co
     hipLaunchKernelGGL(k_lb_morton, dim3(blocks_for(n)), dim3(kT), 0, s, cen, n, bounds, k0, v0);
     e = hipGetLastError();
   }
-  if (e == hipSuccess) e = rocprim::radix_sort_pairs(tmp, tmp_bytes, k0, k1, v0, v1, static_cast<size_t>(n), 0, 30, s);
+  if (e == hipSuccess) e = rocprim::radix_sort_pairs(m.tmp, sb, k0, k1, v0, v1, static_cast<size_t>(n), 0, 30, s);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_lb_radix, dim3(blocks_for(n - 1)), dim3(kT), 0, s, k1, n, left, right, parent, size, err);
     hipLaunchKernelGGL(k_lb_place, dim3(blocks_for(nn)), dim3(kT), 0, s, n, left, right, parent, size, pos, err);
@@ -409,9 +429,6 @@ hipError_t build_blas_device(hipStream_t s, const float* vx, const float* vy, co
   }
   // boxes: the generic refit over the emitted layout (parent and flag reused)
   if (e == hipSuccess) e = refit_blas_device(s, nodes, nn, prims, n, vx, vy, vz, idx, parent, flag, err);
-  const hipError_t es = hipStreamSynchronize(s);
-  if (e == hipSuccess) e = es;
-  for (void* p : mem) (void)hipFree(p);
   return e;
 }
 

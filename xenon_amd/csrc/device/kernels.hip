@@ -868,67 +868,75 @@ __global__ void __launch_bounds__(256) k_api_closest(DevScene S, const float4* r
                                                      uint32_t* overflow_ctr) {
   TravStack st = make_stack(spill, lds_depth);
   TravCount c{0, 0, 0, 0};
-  const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
-  const bool valid = i < n;
-  float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = make_float4(0.f, 1.f, 0.f, 0.f);
-  if (valid) {
-    a = rays[2 * i];
-    b = rays[2 * i + 1];
-  }
-  const f3 o{a.x, a.y, a.z}, d{a.w, b.x, b.y};
-  const float tmin = b.z, tmax = b.w;
-  HitRef h{0.f, 0.f, 0.f, 0u, -1};
-  const bool ok = walk_scene<false>(S, o, d, tmin, tmax, valid, h, st, c);
-  if (valid) {
-    float* out = hits + 16 * static_cast<size_t>(i);
-    if (!ok) {
-      out[0] = __builtin_huge_valf();
-      out[1] = 0.f;
-      out[2] = 0.f;
-      reinterpret_cast<int*>(out)[3] = -1;
-      reinterpret_cast<int*>(out)[4] = -1;
-      reinterpret_cast<int*>(out)[5] = -1;
-      for (int k = 6; k < 15; ++k) out[k] = 0.f;
-      reinterpret_cast<int*>(out)[15] = 0;
-    } else {
-      float u = h.u, v = h.v;
-      Surface sf;
-      if (h.slot & kPrimHit) sf = resolve_prim(S, h, load_inst(S.inst, h.inst), o, d, tmin, u, v);
-      else sf = resolve(S, h, o, d, tmin);
-      out[0] = h.t;
-      out[1] = u;
-      out[2] = v;
-      reinterpret_cast<int*>(out)[3] = sf.inst_id;
-      reinterpret_cast<int*>(out)[4] = static_cast<int>(sf.tri);
-      reinterpret_cast<int*>(out)[5] = sf.mat;
-      out[6] = sf.pos.x; out[7] = sf.pos.y; out[8] = sf.pos.z;
-      out[9] = sf.n.x; out[10] = sf.n.y; out[11] = sf.n.z;
-      out[12] = sf.gn.x; out[13] = sf.gn.y; out[14] = sf.gn.z;
-      reinterpret_cast<int*>(out)[15] = sf.front ? 1 : 0;
+  uint32_t traced = 0;
+  for (int64_t base = static_cast<int64_t>(blockIdx.x) * blockDim.x; base < n; base += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const int64_t i = base + threadIdx.x;
+    const bool valid = i < n;
+    traced += valid ? 1u : 0u;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = make_float4(0.f, 1.f, 0.f, 0.f);
+    if (valid) {
+      a = rays[2 * i];
+      b = rays[2 * i + 1];
     }
-    if (st.overflow) atomicAdd(overflow_ctr, 1u);
+    const f3 o{a.x, a.y, a.z}, d{a.w, b.x, b.y};
+    const float tmin = b.z, tmax = b.w;
+    HitRef h{0.f, 0.f, 0.f, 0u, -1};
+    const bool ok = walk_scene<false>(S, o, d, tmin, tmax, valid, h, st, c);
+    if (valid) {
+      float* out = hits + 16 * i;
+      if (!ok) {
+        out[0] = __builtin_huge_valf();
+        out[1] = 0.f;
+        out[2] = 0.f;
+        reinterpret_cast<int*>(out)[3] = -1;
+        reinterpret_cast<int*>(out)[4] = -1;
+        reinterpret_cast<int*>(out)[5] = -1;
+        for (int k = 6; k < 15; ++k) out[k] = 0.f;
+        reinterpret_cast<int*>(out)[15] = 0;
+      } else {
+        float u = h.u, v = h.v;
+        Surface sf;
+        if (h.slot & kPrimHit) sf = resolve_prim(S, h, load_inst(S.inst, h.inst), o, d, tmin, u, v);
+        else sf = resolve(S, h, o, d, tmin);
+        out[0] = h.t;
+        out[1] = u;
+        out[2] = v;
+        reinterpret_cast<int*>(out)[3] = sf.inst_id;
+        reinterpret_cast<int*>(out)[4] = static_cast<int>(sf.tri);
+        reinterpret_cast<int*>(out)[5] = sf.mat;
+        out[6] = sf.pos.x; out[7] = sf.pos.y; out[8] = sf.pos.z;
+        out[9] = sf.n.x; out[10] = sf.n.y; out[11] = sf.n.z;
+        out[12] = sf.gn.x; out[13] = sf.gn.y; out[14] = sf.gn.z;
+        reinterpret_cast<int*>(out)[15] = sf.front ? 1 : 0;
+      }
+      if (st.overflow) atomicAdd(overflow_ctr, 1u);
+    }
   }
-  flush_counts(stats, c, valid ? 1u : 0u, false);
+  flush_counts(stats, c, traced, false);
 }
 
 __global__ void __launch_bounds__(256) k_api_any(DevScene S, const float4* rays, uint8_t* occ, int n, uint32_t* spill,
                                                  int lds_depth, unsigned long long* stats, uint32_t* overflow_ctr) {
   TravStack st = make_stack(spill, lds_depth);
   TravCount c{0, 0, 0, 0};
-  const int i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
-  const bool valid = i < n;
-  float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = make_float4(0.f, 1.f, 0.f, 0.f);
-  if (valid) {
-    a = rays[2 * i];
-    b = rays[2 * i + 1];
+  uint32_t traced = 0;
+  for (int64_t base = static_cast<int64_t>(blockIdx.x) * blockDim.x; base < n; base += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+    const int64_t i = base + threadIdx.x;
+    const bool valid = i < n;
+    traced += valid ? 1u : 0u;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = make_float4(0.f, 1.f, 0.f, 0.f);
+    if (valid) {
+      a = rays[2 * i];
+      b = rays[2 * i + 1];
+    }
+    HitRef h{0.f, 0.f, 0.f, 0u, -1};
+    const bool hit = walk_scene<true>(S, f3{a.x, a.y, a.z}, f3{a.w, b.x, b.y}, b.z, b.w, valid, h, st, c);
+    if (valid) {
+      occ[i] = hit ? 1 : 0;
+      if (st.overflow) atomicAdd(overflow_ctr, 1u);
+    }
   }
-  HitRef h{0.f, 0.f, 0.f, 0u, -1};
-  const bool hit = walk_scene<true>(S, f3{a.x, a.y, a.z}, f3{a.w, b.x, b.y}, b.z, b.w, valid, h, st, c);
-  if (valid) {
-    occ[i] = hit ? 1 : 0;
-    if (st.overflow) atomicAdd(overflow_ctr, 1u);
-  }
-  flush_counts(stats, c, valid ? 1u : 0u, true);
+  flush_counts(stats, c, traced, true);
 }
 
 // ---------------------------------------------------------------------------
@@ -1010,19 +1018,19 @@ hipError_t launch_average(hipStream_t s, const float4* accum, float* out, int np
   return hipGetLastError();
 }
 
-hipError_t launch_api_closest(hipStream_t s, const DevScene& S, const float4* rays, float* hits, int n,
+hipError_t launch_api_closest(hipStream_t s, const DevScene& S, const float4* rays, float* hits, int n, int grid,
                               uint32_t* spill, int lds_depth, unsigned long long* stats, uint32_t* overflow_ctr) {
   const int block = 256;
-  hipLaunchKernelGGL(k_api_closest, dim3((n + block - 1) / block), dim3(block),
+  hipLaunchKernelGGL(k_api_closest, dim3(grid), dim3(block),
                      static_cast<size_t>(block) * lds_depth * 4, s, S, rays, hits, n, spill, lds_depth, stats,
                      overflow_ctr);
   return hipGetLastError();
 }
 
-hipError_t launch_api_any(hipStream_t s, const DevScene& S, const float4* rays, uint8_t* occ, int n, uint32_t* spill,
-                          int lds_depth, unsigned long long* stats, uint32_t* overflow_ctr) {
+hipError_t launch_api_any(hipStream_t s, const DevScene& S, const float4* rays, uint8_t* occ, int n, int grid,
+                          uint32_t* spill, int lds_depth, unsigned long long* stats, uint32_t* overflow_ctr) {
   const int block = 256;
-  hipLaunchKernelGGL(k_api_any, dim3((n + block - 1) / block), dim3(block),
+  hipLaunchKernelGGL(k_api_any, dim3(grid), dim3(block),
                      static_cast<size_t>(block) * lds_depth * 4, s, S, rays, occ, n, spill, lds_depth, stats,
                      overflow_ctr);
   return hipGetLastError();

@@ -27,10 +27,10 @@ hipError_t launch_advance(hipStream_t s, uint32_t* counters);
 hipError_t launch_average(hipStream_t s, const float4* accum, float* out, int npix, float inv_spp);
 // Ray-batch kernels: rays in the xnh_ray layout (2 float4 per ray:
 // {org.xyz, dir.x} {dir.yz, tmin, tmax}), hits in the xnh_hit layout.
-hipError_t launch_api_closest(hipStream_t s, const DevScene& S, const float4* rays, float* hits, int n,
+hipError_t launch_api_closest(hipStream_t s, const DevScene& S, const float4* rays, float* hits, int n, int grid,
                               uint32_t* spill, int lds_depth, unsigned long long* stats, uint32_t* overflow_ctr);
-hipError_t launch_api_any(hipStream_t s, const DevScene& S, const float4* rays, uint8_t* occ, int n, uint32_t* spill,
-                          int lds_depth, unsigned long long* stats, uint32_t* overflow_ctr);
+hipError_t launch_api_any(hipStream_t s, const DevScene& S, const float4* rays, uint8_t* occ, int n, int grid,
+                          uint32_t* spill, int lds_depth, unsigned long long* stats, uint32_t* overflow_ctr);
 
 hipError_t launch_guide_eval(hipStream_t s, const GuideNet& net, int n, const float* pos, const float* nrm,
                              float* raw);
@@ -83,10 +83,11 @@ hipError_t img_static_scratch(int device, ImgScratch* sc);
 // checked by the caller) -> 2n-1 nodes in the reference's node format and n
 // leaf slots; refit: boxes of an existing tree in that format (structure
 // checked by the caller). parent and flag: nn words of scratch each; err
-// gets a nonzero bit mask if the tree came out malformed. build frees its
-// own scratch and synchronises the stream.
+// gets a nonzero bit mask if the tree came out malformed. build works in
+// `scratch`, of the size build_blas_scratch gives.
+hipError_t build_blas_scratch(hipStream_t s, int n, size_t* bytes);
 hipError_t build_blas_device(hipStream_t s, const float* vx, const float* vy, const float* vz, const int32_t* idx,
-                             int n, xnh_bvh_node* nodes, uint32_t* prims, uint32_t* err);
+                             int n, xnh_bvh_node* nodes, uint32_t* prims, uint32_t* err, char* scratch);
 hipError_t refit_blas_device(hipStream_t s, xnh_bvh_node* nodes, int nn, const uint32_t* prims, int nprims,
                              const float* vx, const float* vy, const float* vz, const int32_t* idx, uint32_t* parent,
                              uint32_t* flag, uint32_t* err);

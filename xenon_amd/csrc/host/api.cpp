@@ -26,6 +26,7 @@
 #include <cstddef>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <string>
 #include <vector>
@@ -118,10 +119,23 @@ struct xnh_ctx {
     ImgScratch sc{};
     std::vector<void*> allocs;
   } out;
+  // Device scratch of the calls that need buffers only while they run (ray
+  // batches, batched jobs, guide batches, BLAS builds): one allocation, grown
+  // as needed and kept for the next call up to kScratchKeep bytes (see
+  // Scratch). Used in stream order, like the queues.
+  char* scratch = nullptr;
+  size_t scratch_cap = 0;
+  int scratch_users = 0;          // calls whose buffers lie in it now
+  std::recursive_mutex scratch_lock;   // held by such a call: others of this context wait their turn
+  char* pinned = nullptr;         // kPinnedBytes of pinned host memory: small tables up, counters down
   xnh_stats stats{};
 };
 
 namespace {
+
+constexpr size_t kScratchKeep = size_t(1) << 30;
+constexpr size_t kPinnedBytes = size_t(1) << 16;
+constexpr size_t kPinnedBatch = kPinnedBytes - 4096;   // ray batches' counters (a render may use what lies below)
 
 // Default samples per pixel per batch: about 2^28 paths in flight (about
 // 75 GB of queues at 292 B per path, a quarter of the device), at most 256
@@ -163,9 +177,27 @@ int fail(xnh_ctx* c, int code, const std::string& msg) {
 // hipMalloc that reports a refusal as XNH_E_ALLOC and clears the runtime's
 // last-error state it leaves, which the next launch check (hipGetLastError)
 // would otherwise report as a failure of that launch.
+void release_scratch(xnh_ctx* c) {
+  if (c->scratch) {
+    hipStreamSynchronize(c->stream);
+    hipFree(c->scratch);
+  }
+  c->scratch = nullptr;
+  c->scratch_cap = 0;
+}
+
 int raw_alloc(xnh_ctx* c, void** p, size_t bytes, const char* what) {
   *p = nullptr;
-  const hipError_t e = hipMalloc(p, bytes);
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess && c && c->scratch_lock.try_lock()) {   // what is kept between calls gives way
+    if (c->scratch && c->scratch_users == 0) {
+      (void)hipGetLastError();
+      *p = nullptr;
+      release_scratch(c);
+      e = hipMalloc(p, bytes);
+    }
+    c->scratch_lock.unlock();
+  }
   if (e == hipSuccess) return XNH_OK;
   (void)hipGetLastError();
   *p = nullptr;
@@ -199,6 +231,47 @@ void free_all(std::vector<void*>& v) {
   for (void* p : v) hipFree(p);
   v.clear();
 }
+
+// Lays out a call's buffers in the context's scratch: `take` the sizes, `get`
+// the memory once, `at` the buffers. Allocating and freeing them in each call
+// cost more than most calls' kernels (hipFree waits for the device, and
+// fresh memory is mapped again): a 1M-ray batch took 12 ms for it, 300,000
+// triangles' BLAS 2 ms.
+class Scratch {
+ public:
+  explicit Scratch(xnh_ctx* c) : c_(c) {
+    c_->scratch_lock.lock();
+    ++c_->scratch_users;
+  }
+  ~Scratch() {
+    if (--c_->scratch_users == 0 && c_->scratch_cap > kScratchKeep) release_scratch(c_);
+    c_->scratch_lock.unlock();
+  }
+  Scratch(const Scratch&) = delete;
+  Scratch& operator=(const Scratch&) = delete;
+  size_t take(size_t bytes) {
+    const size_t at = used_;
+    used_ += (std::max<size_t>(bytes, 1) + 255) & ~size_t(255);
+    return at;
+  }
+  int get() {
+    if (used_ <= c_->scratch_cap) return XNH_OK;
+    release_scratch(c_);   // (every user waits for the stream before it returns)
+    void* p = nullptr;
+    const int rc = raw_alloc(c_, &p, used_, "scratch");
+    if (rc != XNH_OK) return rc;
+    c_->scratch = static_cast<char*>(p);
+    c_->scratch_cap = used_;
+    return XNH_OK;
+  }
+  template <class T>
+  T* at(size_t offset) const {
+    return reinterpret_cast<T*>(c_->scratch + offset);
+  }
+ private:
+  xnh_ctx* c_;
+  size_t used_ = 0;
+};
 
 float4 f4(float x, float y, float z, float w) {
   float4 r;
@@ -606,8 +679,10 @@ int alloc_waves(xnh_ctx* c) {
   if (rc == XNH_OK) rc = dev_alloc(c, c->wave_allocs, &B.sh_c, 2 * qcap);
   if (rc == XNH_OK) rc = dev_alloc(c, c->wave_allocs, &B.l_term, cap);
   if (rc == XNH_OK) rc = dev_alloc(c, c->wave_allocs, &B.l_nee, 2 * cap);
-  if (rc == XNH_OK) rc = dev_alloc(c, c->wave_allocs, &B.counters, static_cast<size_t>(kNumCtr));
-  if (rc == XNH_OK) rc = dev_alloc(c, c->wave_allocs, &B.stats, static_cast<size_t>(kNumStat));
+  // the statistics and right after them the counters, whose first words a
+  // render reads back (and clears) with them
+  if (rc == XNH_OK) rc = dev_alloc(c, c->wave_allocs, &B.stats, static_cast<size_t>(kNumStat + (kNumCtr + 1) / 2));
+  if (rc == XNH_OK) B.counters = reinterpret_cast<uint32_t*>(B.stats + kNumStat);
   if (rc == XNH_OK) {
     const size_t spill = static_cast<size_t>(kMaxStack + 1 - c->lds_depth) * c->grid_trace * c->block;
     rc = dev_alloc(c, c->wave_allocs, &B.spill, spill);
@@ -831,6 +906,27 @@ void attach_guide(xnh_ctx* c) {
   B.guide_depth = g.on ? g.cfg.guide_depth : 0;
 }
 
+// The counters' words that hold a render's outcome, and the statistics with
+// them.
+constexpr int kResultWords = 16;
+constexpr size_t kResultBytes = sizeof(unsigned long long) * kNumStat + sizeof(uint32_t) * kResultWords;
+static_assert(kCnt == kResultWords, "the outcome's words come before the queue counters");
+
+// A render's small tables go up through the pinned memory without waiting
+// (each call has waited for its work before it returns, so the memory is
+// free); larger ones directly. *pin: the bytes staged so far.
+int upload_table(xnh_ctx* c, void* dst, const void* src, size_t bytes, size_t* pin) {
+  if (*pin + bytes <= kPinnedBatch) {
+    std::memcpy(c->pinned + *pin, src, bytes);
+    src = c->pinned + *pin;
+    *pin += (bytes + 63) & ~size_t(63);
+    HIP_OR_FAIL(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream));
+  } else {
+    HIP_OR_FAIL(c, hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
+  }
+  return XNH_OK;
+}
+
 int render_jobs(xnh_ctx* c, const std::vector<JobSpec>& jobs) {
   size_t cap = static_cast<size_t>(c->B.capacity);
   if (cap == 0)
@@ -930,13 +1026,17 @@ int render_jobs(xnh_ctx* c, const std::vector<JobSpec>& jobs) {
   }
   hipStream_t s = c->stream;
   HIP_OR_FAIL(c, hipStreamSynchronize(s));
-  if (!dj.empty()) HIP_OR_FAIL(c, hipMemcpy(c->d_jobs, dj.data(), dj.size() * sizeof(DevJob), hipMemcpyHostToDevice));
-  if (nb) {
-    HIP_OR_FAIL(c, hipMemcpy(c->d_chunks, chunks.data(), chunks.size() * sizeof(DevChunk), hipMemcpyHostToDevice));
-    HIP_OR_FAIL(c, hipMemcpy(c->d_nchunks, counts.data(), counts.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+  size_t pin = 0;
+  if (!dj.empty()) {
+    rc = upload_table(c, c->d_jobs, dj.data(), dj.size() * sizeof(DevJob), &pin);
+    if (rc != XNH_OK) return rc;
   }
-  HIP_OR_FAIL(c, hipMemsetAsync(c->B.stats, 0, sizeof(unsigned long long) * kNumStat, s));
-  HIP_OR_FAIL(c, hipMemsetAsync(c->B.counters, 0, sizeof(uint32_t) * 16, s));   // batch index, overflow
+  if (nb) {
+    rc = upload_table(c, c->d_chunks, chunks.data(), chunks.size() * sizeof(DevChunk), &pin);
+    if (rc == XNH_OK) rc = upload_table(c, c->d_nchunks, counts.data(), counts.size() * sizeof(int32_t), &pin);
+    if (rc != XNH_OK) return rc;
+  }
+  HIP_OR_FAIL(c, hipMemsetAsync(c->B.stats, 0, kResultBytes, s));   // statistics, batch index, overflow
   const size_t nev = c->profiling ? nb * depth * 6 : 0;
   while (c->prof_events.size() < nev) {
     hipEvent_t e;
@@ -963,14 +1063,14 @@ int render_jobs(xnh_ctx* c, const std::vector<JobSpec>& jobs) {
     }
   }
   HIP_OR_FAIL(c, hipEventRecord(c->ev_end, s));
-  unsigned long long st[kNumStat];
-  uint32_t ovf = 0;
-  HIP_OR_FAIL(c, hipMemcpyAsync(st, c->B.stats, sizeof st, hipMemcpyDeviceToHost, s));
-  HIP_OR_FAIL(c, hipMemcpyAsync(&ovf, c->B.counters + kOverflow, sizeof ovf, hipMemcpyDeviceToHost, s));
-  uint32_t dog = 0, segovf = 0;
-  HIP_OR_FAIL(c, hipMemcpyAsync(&dog, c->B.counters + kWatchdog, sizeof dog, hipMemcpyDeviceToHost, s));
-  HIP_OR_FAIL(c, hipMemcpyAsync(&segovf, c->B.counters + kSegOverflow, sizeof segovf, hipMemcpyDeviceToHost, s));
+  // (the tables staged in the pinned memory have been read by then)
+  HIP_OR_FAIL(c, hipMemcpyAsync(c->pinned, c->B.stats, kResultBytes, hipMemcpyDeviceToHost, s));
   HIP_OR_FAIL(c, hipStreamSynchronize(s));
+  unsigned long long st[kNumStat];
+  uint32_t words[kResultWords];
+  std::memcpy(st, c->pinned, sizeof st);
+  std::memcpy(words, c->pinned + sizeof st, sizeof words);
+  const uint32_t ovf = words[kOverflow], dog = words[kWatchdog], segovf = words[kSegOverflow];
   xnh_stats& o = c->stats;
   o = xnh_stats{};
   o.paths = st[kStPaths];
@@ -1055,6 +1155,12 @@ int xnh_create(const xnh_config* cfg, xnh_ctx** out) {
     xnh_destroy(c);
     return XNH_E_HIP;
   }
+  if (hipHostMalloc(reinterpret_cast<void**>(&c->pinned), kPinnedBytes, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    c->pinned = nullptr;
+    xnh_destroy(c);
+    return XNH_E_ALLOC;
+  }
   c->grid_trace = trace_grid(c->block, c->lds_depth);
   const int cus = num_cus();
   if (c->grid_trace <= 0 || cus <= 0) {
@@ -1081,6 +1187,8 @@ void xnh_destroy(xnh_ctx* c) {
   free_all(c->pix_allocs);
   free_all(c->guide.allocs);
   free_all(c->out.allocs);
+  if (c->scratch) hipFree(c->scratch);
+  if (c->pinned) hipHostFree(c->pinned);
   if (c->d_jobs) hipFree(c->d_jobs);
   if (c->d_chunks) hipFree(c->d_chunks);
   if (c->d_nchunks) hipFree(c->d_nchunks);
@@ -1156,59 +1264,49 @@ int xnh_render(xnh_ctx* c, const xnh_camera* cam, int32_t spp_first, int32_t spp
 int xnh_render_jobs(xnh_ctx* c, const xnh_job* jobs, int32_t njobs) {
   if (!c || njobs < 0 || (njobs > 0 && !jobs)) return XNH_E_INVALID;
   std::vector<JobSpec> spec;
-  std::vector<void*> tmp;
-  std::vector<float4*> acc(njobs, nullptr);
+  std::vector<size_t> acc(njobs), rgb(njobs), sum(njobs);
+  Scratch mem(c);
+  size_t acc_end = 0;
   for (int j = 0; j < njobs; ++j) {
     const xnh_job& jb = jobs[j];
     if (jb.width <= 0 || jb.height <= 0 || jb.spp_first < 0 || jb.spp_count < 0 || jb.max_bounces < 0 ||
-        jb.max_bounces > 64 || jb.min_bounces < 0) {
-      free_all(tmp);
+        jb.max_bounces > 64 || jb.min_bounces < 0)
       return fail(c, XNH_E_INVALID, "bad job");
-    }
     const DevScene* S = jb.scene ? &jb.scene->S : (c->has_scene ? &c->own.S : nullptr);
-    if (!S) {
-      free_all(tmp);
-      return fail(c, XNH_E_NO_SCENE, "job without a scene");
-    }
+    if (!S) return fail(c, XNH_E_NO_SCENE, "job without a scene");
     const size_t npix = static_cast<size_t>(jb.width) * jb.height;
-    int rc = dev_alloc(c, tmp, &acc[j], npix);
-    if (rc != XNH_OK) {
-      free_all(tmp);
-      return rc;
-    }
-    if (hipMemsetAsync(acc[j], 0, sizeof(float4) * npix, c->stream) != hipSuccess) {
-      free_all(tmp);
-      return fail(c, XNH_E_HIP, "hipMemsetAsync");
-    }
+    acc[j] = mem.take(sizeof(float4) * npix);
+    acc_end = acc[j] + sizeof(float4) * npix;
     spec.push_back(JobSpec{S, jb.camera, jb.width, jb.height, jb.spp_first, jb.spp_count, jb.max_bounces,
-                           jb.min_bounces, acc[j]});
+                           jb.min_bounces, nullptr});
   }
-  int rc = render_jobs(c, spec);
-  for (int j = 0; j < njobs && rc == XNH_OK; ++j) {
+  // the images, averaged on the device and copied whole
+  for (int j = 0; j < njobs; ++j) {
+    const size_t bytes = 3 * sizeof(float) * static_cast<size_t>(jobs[j].width) * jobs[j].height;
+    if (jobs[j].rgb_out) rgb[j] = mem.take(bytes);
+    if (jobs[j].sum_out) sum[j] = mem.take(bytes);
+  }
+  int rc = mem.get();
+  if (rc != XNH_OK) return rc;
+  for (int j = 0; j < njobs; ++j) spec[j].accum = mem.at<float4>(acc[j]);
+  if (acc_end > 0) HIP_OR_FAIL(c, hipMemsetAsync(mem.at<char>(0), 0, acc_end, c->stream));
+  rc = render_jobs(c, spec);
+  hipError_t e = hipSuccess;
+  for (int j = 0; j < njobs && rc == XNH_OK && e == hipSuccess; ++j) {
     const xnh_job& jb = jobs[j];
-    const size_t npix = static_cast<size_t>(jb.width) * jb.height;
-    if (!jb.rgb_out && !jb.sum_out) continue;
-    std::vector<float4> h(npix);
-    if (hipMemcpy(h.data(), acc[j], sizeof(float4) * npix, hipMemcpyDeviceToHost) != hipSuccess) {
-      rc = fail(c, XNH_E_HIP, "hipMemcpy");
-      break;
-    }
+    const int npix = jb.width * jb.height;
+    const size_t bytes = 3 * sizeof(float) * static_cast<size_t>(npix);
     const float inv = jb.spp_count > 0 ? 1.0f / static_cast<float>(jb.spp_count) : 0.f;
-    for (size_t p = 0; p < npix; ++p) {
-      if (jb.sum_out) {
-        jb.sum_out[3 * p] = h[p].x;
-        jb.sum_out[3 * p + 1] = h[p].y;
-        jb.sum_out[3 * p + 2] = h[p].z;
-      }
-      if (jb.rgb_out) {
-        jb.rgb_out[3 * p] = h[p].x * inv;
-        jb.rgb_out[3 * p + 1] = h[p].y * inv;
-        jb.rgb_out[3 * p + 2] = h[p].z * inv;
-      }
-    }
+    if (jb.rgb_out) e = launch_average(c->stream, spec[j].accum, mem.at<float>(rgb[j]), npix, inv);
+    if (e == hipSuccess && jb.sum_out) e = launch_average(c->stream, spec[j].accum, mem.at<float>(sum[j]), npix, 1.f);
+    if (e == hipSuccess && jb.rgb_out)
+      e = hipMemcpyAsync(jb.rgb_out, mem.at<float>(rgb[j]), bytes, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess && jb.sum_out)
+      e = hipMemcpyAsync(jb.sum_out, mem.at<float>(sum[j]), bytes, hipMemcpyDeviceToHost, c->stream);
   }
-  hipStreamSynchronize(c->stream);
-  free_all(tmp);
+  const hipError_t es = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = es;
+  if (rc == XNH_OK && e != hipSuccess) rc = fail(c, XNH_E_HIP, std::string("jobs: ") + hipGetErrorString(e));
   return rc;
 }
 
@@ -1349,25 +1447,26 @@ int check_mesh_indices(xnh_ctx* c, const xnh_mesh* m) {
   return XNH_OK;
 }
 
-struct DevMesh {   // one mesh's vertices and indices on the device, freed on scope exit
-  std::vector<void*> allocs;
-  float *vx = nullptr, *vy = nullptr, *vz = nullptr;
-  int32_t* idx = nullptr;
-  ~DevMesh() { free_all(allocs); }
+struct DevMesh {   // one mesh's vertices and indices in the call's scratch
+  size_t vx, vy, vz, idx;
+  DevMesh(Scratch& mem, const xnh_mesh* m) {
+    const size_t nv = sizeof(float) * static_cast<size_t>(m->num_vertices);
+    vx = mem.take(nv);
+    vy = mem.take(nv);
+    vz = mem.take(nv);
+    idx = mem.take(3 * sizeof(int32_t) * static_cast<size_t>(m->num_triangles));
+  }
 };
 
-int upload_mesh(xnh_ctx* c, const xnh_mesh* m, DevMesh& d) {
-  const size_t nv = static_cast<size_t>(m->num_vertices), ni = 3 * static_cast<size_t>(m->num_triangles);
-  int rc = dev_alloc(c, d.allocs, &d.vx, nv);
-  if (rc == XNH_OK) rc = dev_alloc(c, d.allocs, &d.vy, nv);
-  if (rc == XNH_OK) rc = dev_alloc(c, d.allocs, &d.vz, nv);
-  if (rc == XNH_OK) rc = dev_alloc(c, d.allocs, &d.idx, ni);
-  if (rc != XNH_OK) return rc;
-  HIP_OR_FAIL(c, hipMemcpyAsync(d.vx, m->vx, sizeof(float) * nv, hipMemcpyHostToDevice, c->stream));
-  HIP_OR_FAIL(c, hipMemcpyAsync(d.vy, m->vy, sizeof(float) * nv, hipMemcpyHostToDevice, c->stream));
-  HIP_OR_FAIL(c, hipMemcpyAsync(d.vz, m->vz, sizeof(float) * nv, hipMemcpyHostToDevice, c->stream));
-  HIP_OR_FAIL(c, hipMemcpyAsync(d.idx, m->indices, sizeof(int32_t) * ni, hipMemcpyHostToDevice, c->stream));
-  return XNH_OK;
+hipError_t upload_mesh(xnh_ctx* c, const xnh_mesh* m, const Scratch& mem, const DevMesh& d) {
+  const size_t nv = sizeof(float) * static_cast<size_t>(m->num_vertices);
+  hipError_t e = hipMemcpyAsync(mem.at<float>(d.vx), m->vx, nv, hipMemcpyHostToDevice, c->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(mem.at<float>(d.vy), m->vy, nv, hipMemcpyHostToDevice, c->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(mem.at<float>(d.vz), m->vz, nv, hipMemcpyHostToDevice, c->stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(mem.at<int32_t>(d.idx), m->indices, 3 * sizeof(int32_t) * static_cast<size_t>(m->num_triangles),
+                       hipMemcpyHostToDevice, c->stream);
+  return e;
 }
 
 }  // namespace
@@ -1395,30 +1494,29 @@ int xnh_build_blas(xnh_ctx* c, const xnh_mesh* m, xnh_bvh_node* nodes_out, uint3
     prims_out[0] = 0;
     return XNH_OK;
   }
-  DevMesh d;
-  rc = upload_mesh(c, m, d);
+  Scratch mem(c);
+  const DevMesh d(mem, m);
+  const size_t o_nodes = mem.take(sizeof(xnh_bvh_node) * (2 * static_cast<size_t>(n) - 1));
+  const size_t o_prims = mem.take(sizeof(uint32_t) * static_cast<size_t>(n)), o_err = mem.take(sizeof(uint32_t));
+  size_t tmp = 0;
+  HIP_OR_FAIL(c, build_blas_scratch(c->stream, n, &tmp));
+  const size_t o_tmp = mem.take(tmp);
+  rc = mem.get();
   if (rc != XNH_OK) return rc;
-  std::vector<void*> own;
-  xnh_bvh_node* nodes = nullptr;
-  uint32_t *prims = nullptr, *err = nullptr;
-  rc = dev_alloc(c, own, &nodes, static_cast<size_t>(2 * n - 1));
-  if (rc == XNH_OK) rc = dev_alloc(c, own, &prims, static_cast<size_t>(n));
-  if (rc == XNH_OK) rc = dev_alloc(c, own, &err, 1);
+  xnh_bvh_node* nodes = mem.at<xnh_bvh_node>(o_nodes);
+  uint32_t *prims = mem.at<uint32_t>(o_prims), *err = mem.at<uint32_t>(o_err);
   uint32_t herr = 0;
-  hipError_t e = hipSuccess;
-  if (rc == XNH_OK) {
-    e = hipMemsetAsync(err, 0, 4, c->stream);
-    if (e == hipSuccess) e = build_blas_device(c->stream, d.vx, d.vy, d.vz, d.idx, n, nodes, prims, err);
-    if (e == hipSuccess) e = hipMemcpyAsync(&herr, err, 4, hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(nodes_out, nodes, sizeof(xnh_bvh_node) * (2 * n - 1), hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(prims_out, prims, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, c->stream);
-    const hipError_t es = hipStreamSynchronize(c->stream);
-    if (e == hipSuccess) e = es;
-  }
-  free_all(own);
-  if (rc != XNH_OK) return rc;
+  hipError_t e = upload_mesh(c, m, mem, d);
+  if (e == hipSuccess) e = hipMemsetAsync(err, 0, 4, c->stream);
+  if (e == hipSuccess)
+    e = build_blas_device(c->stream, mem.at<float>(d.vx), mem.at<float>(d.vy), mem.at<float>(d.vz),
+                          mem.at<int32_t>(d.idx), n, nodes, prims, err, mem.at<char>(o_tmp));
+  if (e == hipSuccess) e = hipMemcpyAsync(&herr, err, 4, hipMemcpyDeviceToHost, c->stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(nodes_out, nodes, sizeof(xnh_bvh_node) * (2 * n - 1), hipMemcpyDeviceToHost, c->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(prims_out, prims, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, c->stream);
+  const hipError_t es = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = es;
   if (e != hipSuccess) return fail(c, XNH_E_HIP, std::string("device BLAS build: ") + hipGetErrorString(e));
   if (herr != 0) return fail(c, XNH_E_HIP, "device BLAS build produced a malformed tree (mask " + std::to_string(herr) + ")");
   return XNH_OK;
@@ -1442,34 +1540,43 @@ int xnh_refit_blas(xnh_ctx* c, const xnh_mesh* m, xnh_bvh_node* nodes_out) {
   }
   for (int k = 0; k < n; ++k)
     if (m->prims[k] >= static_cast<uint32_t>(n)) return fail(c, XNH_E_INVALID, "slot names no triangle");
-  DevMesh d;
-  rc = upload_mesh(c, m, d);
+  Scratch mem(c);
+  const DevMesh d(mem, m);
+  const size_t o_nodes = mem.take(sizeof(xnh_bvh_node) * static_cast<size_t>(nn));
+  const size_t words = sizeof(uint32_t) * static_cast<size_t>(nn);
+  const size_t o_prims = mem.take(sizeof(uint32_t) * static_cast<size_t>(n));
+  const size_t o_parent = mem.take(words), o_flag = mem.take(words), o_err = mem.take(sizeof(uint32_t));
+  rc = mem.get();
   if (rc != XNH_OK) return rc;
-  std::vector<void*> own;
-  xnh_bvh_node* nodes = nullptr;
-  uint32_t *prims = nullptr, *parent = nullptr, *flag = nullptr, *err = nullptr;
-  rc = dev_alloc(c, own, &nodes, static_cast<size_t>(nn));
-  if (rc == XNH_OK) rc = dev_alloc(c, own, &prims, static_cast<size_t>(n));
-  if (rc == XNH_OK) rc = dev_alloc(c, own, &parent, static_cast<size_t>(nn));
-  if (rc == XNH_OK) rc = dev_alloc(c, own, &flag, static_cast<size_t>(nn));
-  if (rc == XNH_OK) rc = dev_alloc(c, own, &err, 1);
+  xnh_bvh_node* nodes = mem.at<xnh_bvh_node>(o_nodes);
+  uint32_t *prims = mem.at<uint32_t>(o_prims), *err = mem.at<uint32_t>(o_err);
   uint32_t herr = 0;
-  hipError_t e = hipSuccess;
-  if (rc == XNH_OK) {
+  hipError_t e = upload_mesh(c, m, mem, d);
+  if (e == hipSuccess)
     e = hipMemcpyAsync(nodes, m->nodes, sizeof(xnh_bvh_node) * nn, hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(prims, m->prims, sizeof(uint32_t) * n, hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(err, 0, 4, c->stream);
-    if (e == hipSuccess) e = refit_blas_device(c->stream, nodes, nn, prims, n, d.vx, d.vy, d.vz, d.idx, parent, flag, err);
-    if (e == hipSuccess) e = hipMemcpyAsync(&herr, err, 4, hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(nodes_out, nodes, sizeof(xnh_bvh_node) * nn, hipMemcpyDeviceToHost, c->stream);
-    const hipError_t es = hipStreamSynchronize(c->stream);
-    if (e == hipSuccess) e = es;
-  }
-  free_all(own);
-  if (rc != XNH_OK) return rc;
+  if (e == hipSuccess) e = hipMemcpyAsync(prims, m->prims, sizeof(uint32_t) * n, hipMemcpyHostToDevice, c->stream);
+  if (e == hipSuccess) e = hipMemsetAsync(err, 0, 4, c->stream);
+  if (e == hipSuccess)
+    e = refit_blas_device(c->stream, nodes, nn, prims, n, mem.at<float>(d.vx), mem.at<float>(d.vy),
+                          mem.at<float>(d.vz), mem.at<int32_t>(d.idx), mem.at<uint32_t>(o_parent),
+                          mem.at<uint32_t>(o_flag), err);
+  if (e == hipSuccess) e = hipMemcpyAsync(&herr, err, 4, hipMemcpyDeviceToHost, c->stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(nodes_out, nodes, sizeof(xnh_bvh_node) * nn, hipMemcpyDeviceToHost, c->stream);
+  const hipError_t es = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = es;
   if (e != hipSuccess) return fail(c, XNH_E_HIP, std::string("device BLAS refit: ") + hipGetErrorString(e));
   if (herr != 0) return fail(c, XNH_E_HIP, "device BLAS refit found a malformed tree (mask " + std::to_string(herr) + ")");
+  return XNH_OK;
+}
+
+int xnh_read_frame(xnh_ctx* c, float* rgb_out) {
+  if (!c || !rgb_out) return XNH_E_INVALID;
+  const float inv = c->spp_total > 0 ? 1.0f / static_cast<float>(c->spp_total) : 0.f;
+  HIP_OR_FAIL(c, launch_img_from_accum(c->stream, c->accum, inv, c->cfg.width, c->cfg.height, c->d_out));
+  HIP_OR_FAIL(c, hipMemcpyAsync(rgb_out, c->d_out, sizeof(float) * 3 * c->cfg.width * c->cfg.height,
+                                hipMemcpyDeviceToHost, c->stream));
+  HIP_OR_FAIL(c, hipStreamSynchronize(c->stream));
   return XNH_OK;
 }
 
@@ -1779,21 +1886,17 @@ int xnh_guide_get_params(xnh_ctx* c, float* grid, float* w) {
 int xnh_guide_eval(xnh_ctx* c, int32_t n, const float* pos, const float* nrm, float* raw) {
   if (!c || !c->guide.on || n < 0 || (n > 0 && (!pos || !nrm || !raw))) return XNH_E_INVALID;
   if (n == 0) return XNH_OK;
-  std::vector<void*> tmp;
-  float *dp, *dn, *dr;
-  int rc = dev_alloc(c, tmp, &dp, size_t(n) * 3);
-  if (rc == XNH_OK) rc = dev_alloc(c, tmp, &dn, size_t(n) * 3);
-  if (rc == XNH_OK) rc = dev_alloc(c, tmp, &dr, size_t(n) * kGOut);
-  hipError_t e = hipSuccess;
-  if (rc == XNH_OK) {
-    e = hipMemcpyAsync(dp, pos, size_t(n) * 12, hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(dn, nrm, size_t(n) * 12, hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = launch_guide_eval(c->stream, c->guide.net, n, dp, dn, dr);
-    if (e == hipSuccess) e = hipMemcpyAsync(raw, dr, size_t(n) * kGOut * 4, hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-  }
-  free_all(tmp);
+  Scratch mem(c);
+  const size_t op = mem.take(size_t(n) * 12), on = mem.take(size_t(n) * 12), orw = mem.take(size_t(n) * kGOut * 4);
+  const int rc = mem.get();
   if (rc != XNH_OK) return rc;
+  float *dp = mem.at<float>(op), *dn = mem.at<float>(on), *dr = mem.at<float>(orw);
+  hipError_t e = hipMemcpyAsync(dp, pos, size_t(n) * 12, hipMemcpyHostToDevice, c->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(dn, nrm, size_t(n) * 12, hipMemcpyHostToDevice, c->stream);
+  if (e == hipSuccess) e = launch_guide_eval(c->stream, c->guide.net, n, dp, dn, dr);
+  if (e == hipSuccess) e = hipMemcpyAsync(raw, dr, size_t(n) * kGOut * 4, hipMemcpyDeviceToHost, c->stream);
+  const hipError_t es = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = es;
   if (e != hipSuccess) return fail(c, XNH_E_HIP, std::string("guide eval: ") + hipGetErrorString(e));
   return XNH_OK;
 }
@@ -1802,27 +1905,23 @@ int xnh_guide_query(xnh_ctx* c, int32_t n, const float* pos, const float* nrm, c
                     float* pdf) {
   if (!c || !c->guide.on || n < 0 || (n > 0 && (!pos || !nrm || !dir || !pdf))) return XNH_E_INVALID;
   if (n == 0) return XNH_OK;
-  std::vector<void*> tmp;
-  float *dp, *dn, *du = nullptr, *dd, *dq;
-  int rc = dev_alloc(c, tmp, &dp, size_t(n) * 3);
-  if (rc == XNH_OK) rc = dev_alloc(c, tmp, &dn, size_t(n) * 3);
-  if (rc == XNH_OK && u) rc = dev_alloc(c, tmp, &du, size_t(n) * 3);
-  if (rc == XNH_OK) rc = dev_alloc(c, tmp, &dd, size_t(n) * 3);
-  if (rc == XNH_OK) rc = dev_alloc(c, tmp, &dq, size_t(n));
-  hipError_t e = hipSuccess;
-  if (rc == XNH_OK) {
-    hipStream_t s = c->stream;
-    e = hipMemcpyAsync(dp, pos, size_t(n) * 12, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(dn, nrm, size_t(n) * 12, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess && u) e = hipMemcpyAsync(du, u, size_t(n) * 12, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess && !u) e = hipMemcpyAsync(dd, dir, size_t(n) * 12, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = launch_guide_query(s, c->guide.net, n, dp, dn, du, dd, dq);
-    if (e == hipSuccess && u) e = hipMemcpyAsync(dir, dd, size_t(n) * 12, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(pdf, dq, size_t(n) * 4, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipStreamSynchronize(s);
-  }
-  free_all(tmp);
+  Scratch mem(c);
+  const size_t op = mem.take(size_t(n) * 12), on = mem.take(size_t(n) * 12), ou = mem.take(u ? size_t(n) * 12 : 0),
+               od = mem.take(size_t(n) * 12), oq = mem.take(size_t(n) * 4);
+  const int rc = mem.get();
   if (rc != XNH_OK) return rc;
+  float *dp = mem.at<float>(op), *dn = mem.at<float>(on), *du = u ? mem.at<float>(ou) : nullptr,
+        *dd = mem.at<float>(od), *dq = mem.at<float>(oq);
+  hipStream_t s = c->stream;
+  hipError_t e = hipMemcpyAsync(dp, pos, size_t(n) * 12, hipMemcpyHostToDevice, s);
+  if (e == hipSuccess) e = hipMemcpyAsync(dn, nrm, size_t(n) * 12, hipMemcpyHostToDevice, s);
+  if (e == hipSuccess && u) e = hipMemcpyAsync(du, u, size_t(n) * 12, hipMemcpyHostToDevice, s);
+  if (e == hipSuccess && !u) e = hipMemcpyAsync(dd, dir, size_t(n) * 12, hipMemcpyHostToDevice, s);
+  if (e == hipSuccess) e = launch_guide_query(s, c->guide.net, n, dp, dn, du, dd, dq);
+  if (e == hipSuccess && u) e = hipMemcpyAsync(dir, dd, size_t(n) * 12, hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipMemcpyAsync(pdf, dq, size_t(n) * 4, hipMemcpyDeviceToHost, s);
+  const hipError_t es = hipStreamSynchronize(s);
+  if (e == hipSuccess) e = es;
   if (e != hipSuccess) return fail(c, XNH_E_HIP, std::string("guide query: ") + hipGetErrorString(e));
   return XNH_OK;
 }
@@ -1862,23 +1961,19 @@ int xnh_guide_train(xnh_ctx* c, int32_t n, const float* pos, const float* nrm, c
   if (!(lsum > 0.0)) return fail(c, XNH_E_INVALID, "training weights sum to zero");
   const float lam_scale = static_cast<float>(double(n) / lsum);
   GuideState& g = c->guide;
-  std::vector<void*> tmp;
-  float *dp, *dn, *dd, *dl;
-  int rc = dev_alloc(c, tmp, &dp, size_t(n) * 3);
-  if (rc == XNH_OK) rc = dev_alloc(c, tmp, &dn, size_t(n) * 3);
-  if (rc == XNH_OK) rc = dev_alloc(c, tmp, &dd, size_t(n) * 3);
-  if (rc == XNH_OK) rc = dev_alloc(c, tmp, &dl, size_t(n));
-  if (rc != XNH_OK) {
-    free_all(tmp);
-    return rc;
-  }
+  Scratch mem(c);
+  const size_t op = mem.take(size_t(n) * 12), on = mem.take(size_t(n) * 12), od = mem.take(size_t(n) * 12),
+               ol = mem.take(size_t(n) * 4);
+  int rc = mem.get();
+  if (rc != XNH_OK) return rc;
+  float *dp = mem.at<float>(op), *dn = mem.at<float>(on), *dd = mem.at<float>(od), *dl = mem.at<float>(ol);
   hipStream_t s = c->stream;
   hipError_t e = hipMemcpyAsync(dp, pos, size_t(n) * 12, hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipMemcpyAsync(dn, nrm, size_t(n) * 12, hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipMemcpyAsync(dd, dir, size_t(n) * 12, hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipMemcpyAsync(dl, lam, size_t(n) * 4, hipMemcpyHostToDevice, s);
   if (e != hipSuccess) {
-    free_all(tmp);
+    hipStreamSynchronize(s);
     return fail(c, XNH_E_HIP, "guide train upload");
   }
   rc = guide_step(c, n, dp, dn, dd, dl, lam_scale, apply != 0);
@@ -1892,7 +1987,7 @@ int xnh_guide_train(xnh_ctx* c, int32_t n, const float* pos, const float* nrm, c
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) rc = fail(c, XNH_E_HIP, std::string("guide train: ") + hipGetErrorString(e));
   }
-  free_all(tmp);
+  if (rc != XNH_OK) hipStreamSynchronize(s);
   if (loss_out) *loss_out = loss / static_cast<float>(n);
   return rc;
 }
@@ -1903,49 +1998,45 @@ static int trace_common(xnh_ctx* c, const xnh_ray* rays, int32_t n, bool any, vo
   c->stats = xnh_stats{};
   if (n == 0) return XNH_OK;
   static_assert(sizeof(xnh_ray) == 2 * sizeof(float4), "the kernels read xnh_ray as two float4");
-  std::vector<float4> hr(2 * static_cast<size_t>(n));
-  std::memcpy(hr.data(), rays, sizeof(xnh_ray) * static_cast<size_t>(n));
-  std::vector<void*> tmp;
-  float4* d_rays = nullptr;
-  void* d_out = nullptr;
-  uint32_t* d_spill = nullptr;
-  unsigned long long* d_stats = nullptr;
-  uint32_t* d_ovf = nullptr;
+  // a grid of at most the traversal kernels' (each lane of it has a spill
+  // column; past it the work-groups take further rays in turn)
   const int block = 256;
-  const size_t threads = static_cast<size_t>((n + block - 1) / block) * block;
-  int rc = dev_upload(c, tmp, &d_rays, hr);
-  if (rc == XNH_OK) {
-    if (any) rc = dev_alloc(c, tmp, reinterpret_cast<uint8_t**>(&d_out), static_cast<size_t>(n));
-    else rc = dev_alloc(c, tmp, reinterpret_cast<float**>(&d_out), static_cast<size_t>(n) * 16);
-  }
-  if (rc == XNH_OK) rc = dev_alloc(c, tmp, &d_spill, static_cast<size_t>(kMaxStack + 1 - c->lds_depth) * threads);
-  if (rc == XNH_OK) rc = dev_alloc(c, tmp, &d_stats, static_cast<size_t>(kNumStat));
-  if (rc == XNH_OK) rc = dev_alloc(c, tmp, &d_ovf, 1);
-  if (rc != XNH_OK) {
-    free_all(tmp);
-    return rc;
-  }
-  hipError_t e = hipMemsetAsync(d_stats, 0, sizeof(unsigned long long) * kNumStat, c->stream);
-  if (e == hipSuccess) e = hipMemsetAsync(d_ovf, 0, sizeof(uint32_t), c->stream);
+  const int most = std::max(1, c->grid_trace * c->block / block);
+  const int grid = std::min((n + block - 1) / block, most);
+  const size_t out_bytes = static_cast<size_t>(n) * (any ? sizeof(uint8_t) : sizeof(xnh_hit));
+  Scratch mem(c);
+  const size_t o_stats = mem.take(sizeof(unsigned long long) * kNumStat + sizeof(uint32_t));
+  const size_t o_rays = mem.take(sizeof(xnh_ray) * static_cast<size_t>(n)), o_out = mem.take(out_bytes);
+  const size_t o_spill =
+      mem.take(sizeof(uint32_t) * static_cast<size_t>(kMaxStack + 1 - c->lds_depth) * static_cast<size_t>(grid) * block);
+  const int rc = mem.get();
+  if (rc != XNH_OK) return rc;
+  unsigned long long* d_stats = mem.at<unsigned long long>(o_stats);
+  uint32_t* d_ovf = reinterpret_cast<uint32_t*>(d_stats + kNumStat);
+  const float4* d_rays = mem.at<float4>(o_rays);
+  const size_t result = sizeof(unsigned long long) * kNumStat + sizeof(uint32_t);
+  hipError_t e = hipMemcpyAsync(mem.at<char>(o_rays), rays, sizeof(xnh_ray) * static_cast<size_t>(n),
+                                hipMemcpyHostToDevice, c->stream);
+  if (e == hipSuccess) e = hipMemsetAsync(d_stats, 0, result, c->stream);
   if (e == hipSuccess) e = hipEventRecord(c->ev_begin, c->stream);
-  if (e == hipSuccess) {
-    e = any ? launch_api_any(c->stream, c->own.S, d_rays, static_cast<uint8_t*>(d_out), n, d_spill, c->lds_depth, d_stats,
-                             d_ovf)
-            : launch_api_closest(c->stream, c->own.S, d_rays, static_cast<float*>(d_out), n, d_spill, c->lds_depth,
-                                 d_stats, d_ovf);
-  }
-  if (e == hipSuccess) e = hipEventRecord(c->ev_end, c->stream);
   if (e == hipSuccess)
-    e = hipMemcpyAsync(out, d_out, any ? static_cast<size_t>(n) : static_cast<size_t>(n) * 64, hipMemcpyDeviceToHost,
-                       c->stream);
+    e = any ? launch_api_any(c->stream, c->own.S, d_rays, mem.at<uint8_t>(o_out), n, grid, mem.at<uint32_t>(o_spill),
+                             c->lds_depth, d_stats, d_ovf)
+            : launch_api_closest(c->stream, c->own.S, d_rays, mem.at<float>(o_out), n, grid, mem.at<uint32_t>(o_spill),
+                                 c->lds_depth, d_stats, d_ovf);
+  if (e == hipSuccess) e = hipEventRecord(c->ev_end, c->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(c->pinned + kPinnedBatch, d_stats, result, hipMemcpyDeviceToHost, c->stream);
+  if (e == hipSuccess) e = hipMemcpyAsync(out, mem.at<char>(o_out), out_bytes, hipMemcpyDeviceToHost, c->stream);
+  const hipError_t es = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) e = es;
   unsigned long long st[kNumStat] = {};
   uint32_t ovf = 0;
-  if (e == hipSuccess) e = hipMemcpyAsync(st, d_stats, sizeof st, hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipMemcpyAsync(&ovf, d_ovf, sizeof ovf, hipMemcpyDeviceToHost, c->stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess) {
+    std::memcpy(st, c->pinned + kPinnedBatch, sizeof st);
+    std::memcpy(&ovf, c->pinned + kPinnedBatch + sizeof st, sizeof ovf);
+  }
   float ms = 0.f;
   if (e == hipSuccess) e = hipEventElapsedTime(&ms, c->ev_begin, c->ev_end);
-  free_all(tmp);
   if (e != hipSuccess) return fail(c, XNH_E_HIP, std::string("trace: ") + hipGetErrorString(e));
   c->stats.closest_rays = st[kStClosest];
   c->stats.shadow_rays = st[kStShadow];

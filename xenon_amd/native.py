@@ -177,6 +177,7 @@ SIGNATURES = {
     "xnh_trace_any": (C.c_int, [_vp, C.POINTER(Ray), C.c_int32, C.POINTER(C.c_uint8)]),
     "xnh_scene_upload": (C.c_int, [_vp, C.POINTER(FlatScene), C.POINTER(_vp)]),
     "xnh_scene_release": (None, [_vp, _vp]),
+    "xnh_read_frame": (C.c_int, [_vp, _fp]),
     "xnh_render_jobs": (C.c_int, [_vp, C.POINTER(Job), C.c_int32]),
     "xnh_scene_new": (_vp, []),
     "xnh_scene_free": (None, [_vp]),

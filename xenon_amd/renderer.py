@@ -254,13 +254,18 @@ class HipRenderer:
         top (rows flipped, render/cpu_tiled.cpp:228-229). With a
         TripleSwapchain the frame goes into its write buffer, which is then
         published (cuda_renderer.cu:501-590)."""
-        img = self.render(camera, self.spp() + 1, 1)
-        frame = img.reshape(self.height, self.width, 3)[::-1]
-        if chain is None:
-            return frame.copy()
-        out = chain.get_write_buffer()
-        np.copyto(out, frame)
-        chain.swap_writer()
+        self.render(camera, self.spp() + 1, 1, want_image=False)
+        # the library averages and flips on the device; the frame is copied once
+        shape = (self.height, self.width, 3)
+        out = np.empty(shape, np.float32) if chain is None else chain.get_write_buffer()
+        if out.shape == shape and out.dtype == np.float32 and out.flags.c_contiguous and out.flags.writeable:
+            self._chk(N.lib().xnh_read_frame(self.h, _fp(out)))
+        else:
+            frame = np.empty(shape, np.float32)
+            self._chk(N.lib().xnh_read_frame(self.h, _fp(frame)))
+            np.copyto(out, frame)
+        if chain is not None:
+            chain.swap_writer()
         return out
 
     def spp(self) -> int:
@@ -299,8 +304,8 @@ class HipRenderer:
         triangle), nodes in NODE_DTYPE."""
         v, keep = self._mesh_view(positions, indices)
         n = v.num_triangles
-        nodes = np.zeros(max(2 * n - 1, 0), NODE_DTYPE)
-        prims = np.zeros(n, np.uint32)
+        nodes = np.empty(max(2 * n - 1, 0), NODE_DTYPE)
+        prims = np.empty(n, np.uint32)
         nn = C.c_int32()
         self._chk(N.lib().xnh_build_blas(self.h, C.byref(v), nodes.ctypes.data_as(C.POINTER(N.BvhNode)),
                                          prims.ctypes.data_as(N._u32p), C.byref(nn)))
@@ -311,7 +316,7 @@ class HipRenderer:
         """The boxes of (nodes, prims) recomputed for new vertex positions
         (xnh_refit_blas); the topology is kept."""
         v, keep = self._mesh_view(positions, indices, np.asarray(nodes, NODE_DTYPE), prims)
-        out = np.zeros(v.num_nodes, NODE_DTYPE)
+        out = np.empty(v.num_nodes, NODE_DTYPE)
         self._chk(N.lib().xnh_refit_blas(self.h, C.byref(v), out.ctypes.data_as(C.POINTER(N.BvhNode))))
         del keep
         return out
@@ -555,7 +560,7 @@ class HipRenderer:
     def trace_closest(self, rays: np.ndarray) -> np.ndarray:
         rays = np.ascontiguousarray(rays, np.float32).reshape(-1, 8)
         n = rays.shape[0]
-        hits = np.zeros(n, HIT_DTYPE)
+        hits = np.empty(n, HIT_DTYPE)   # the library writes every record
         self._chk(N.lib().xnh_trace_closest(self.h, rays.ctypes.data_as(C.POINTER(N.Ray)), n,
                                             hits.ctypes.data_as(C.POINTER(N.Hit))))
         return hits
@@ -563,7 +568,7 @@ class HipRenderer:
     def trace_any(self, rays: np.ndarray) -> np.ndarray:
         rays = np.ascontiguousarray(rays, np.float32).reshape(-1, 8)
         n = rays.shape[0]
-        occ = np.zeros(n, np.uint8)
+        occ = np.empty(n, np.uint8)
         self._chk(N.lib().xnh_trace_any(self.h, rays.ctypes.data_as(C.POINTER(N.Ray)), n,
                                         occ.ctypes.data_as(C.POINTER(C.c_uint8))))
         return occ
