@@ -599,14 +599,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGuide
                          l3 = S.lights[4 * k + 3];
             const float u1 = rng.f();
             const float u2 = rng.f();
-            const float su1 = sqrtf(u1);
+            const float su1 = sqrt_r(u1);
             const float b0 = 1.0f - su1;
             const float b1 = u2 * su1;
             const float b2 = 1.0f - b0 - b1;
             const f3 lp = xyz(l0) * b0 + xyz(l1) * b1 + xyz(l2) * b2;
             const f3 sdv = lp - sf.pos;
             const float d2 = len2(sdv);
-            const float dist = sqrtf(d2);
+            const float dist = sqrt_any(d2);
             if (dist > 1e-6f) {
               const f3 wi = sdv * recip(dist);
               const float cl = smax(0.0f, dot(xyz(l3), -wi));
@@ -614,8 +614,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGuide
               const f3 wo_l = fr.local(-d);
               const f3 wi_l = fr.local(wi);
               if (cl > 1e-6f && wi_l.z > 1e-6f) {
-                const f3 f = nee_f(wo_l, wi_l, m);
-                float bp = nee_pdf(wo_l, wi_l, m);
+                f3 f;
+                float bp;
+                nee_eval(wo_l, wi_l, m, f, bp);
                 if (guided) bp = alpha * stored_pdf(B.mix, B.mix_stride, mi, wi) + (1.f - alpha) * bp;
                 const float lpdf = ((1.0f / l0.w) * pick) * (d2 / cl);
                 const float w = mis_power2(lpdf, bp);
@@ -644,8 +645,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kGuide
               const f3 wo_l = fr.local(-d);
               const f3 wi_l = fr.local(sdir);
               if (wi_l.z > 1e-6f) {
-                const f3 f = nee_f(wo_l, wi_l, m);
-                float bp = nee_pdf(wo_l, wi_l, m);
+                f3 f;
+                float bp;
+                nee_eval(wo_l, wi_l, m, f, bp);
                 if (guided) bp = alpha * stored_pdf(B.mix, B.mix_stride, mi, sdir) + (1.f - alpha) * bp;
                 const float cs = wi_l.z;
                 const float lpdf = 1e8f * spick;
