@@ -209,8 +209,10 @@ struct WaveBuffers {
   float4* sh0;      // shadow ray {o.xyz, d.x}
   float4* sh1;      // {d.y, d.z, tmax, slot*2+k}
   float4* sh_c;     // unoccluded contribution
-  float4* l_term;   // per slot: emission / sky at path end
-  float4* l_nee;    // per slot x 2: area and sun NEE sums
+  // per slot, three floats each: emission / sky at the path's end (written
+  // when it ends), the sums of the area lights' and the suns' NEE (cleared by
+  // k_raygen, and there only for jobs that have such lights)
+  float *l_term, *l_area, *l_sun;
   const DevJob* jobs;
   const DevChunk* chunks;   // [batch][kMaxChunks]
   const int32_t* nchunks;   // chunks per batch
@@ -232,7 +234,8 @@ struct WaveBuffers {
 };
 
 enum Ctr : int {
-  kBatch = 0,                            // batch being rendered (advanced on the device)
+  kBatch = 0,                            // batch being rendered: kNext, as k_raygen found it
+  kNext = 2,                             // batch to render next (k_accumulate sets it)
   kOverflow = 1,                         // lanes whose stack exceeded kMaxStack
   kWatchdog = 3,                         // waves that hit an iteration bound (see dtrace.h)
   kSegOverflow = 4,                      // appends past a queue segment's end (dropped; never expected)

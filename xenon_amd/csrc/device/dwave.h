@@ -502,6 +502,18 @@ __device__ __forceinline__ void flush_counts_block(unsigned long long* stats, co
   }
 }
 
+// Slot `slot` of a per-slot radiance array.
+__device__ __forceinline__ f3 slot_f3(const float* a, uint32_t slot) {
+  const float* p = a + 3 * static_cast<size_t>(slot);
+  return f3{p[0], p[1], p[2]};
+}
+__device__ __forceinline__ void put_slot(float* a, uint32_t slot, f3 v) {
+  float* p = a + 3 * static_cast<size_t>(slot);
+  p[0] = v.x;
+  p[1] = v.y;
+  p[2] = v.z;
+}
+
 // Last chunk c with prefix[c] <= u: the (non-empty) chunk holding item u.
 template <class View>
 __device__ __forceinline__ int find_chunk(const View& v, uint32_t u) {

@@ -378,7 +378,7 @@ __device__ __forceinline__ float record_lambda(const WaveBuffers& B, uint32_t r)
   const uint32_t R = B.rec_cap;
   const float4 a = B.rec[r], b = B.rec[R + r], c = B.rec[2 * R + r], e = B.rec[3 * R + r];
   const uint32_t slot = __float_as_uint(e.w);
-  const float4 t = B.l_term[slot], n0 = B.l_nee[2 * slot], n1 = B.l_nee[2 * slot + 1];
+  const f3 t = slot_f3(B.l_term, slot), n0 = slot_f3(B.l_area, slot), n1 = slot_f3(B.l_sun, slot);
   const float ar = t.x + n0.x + n1.x - e.x, ag = t.y + n0.y + n1.y - e.y, ab = t.z + n0.z + n1.z - e.z;
   const float lr = a.w > 0.f ? ar / a.w : 0.f, lg = b.w > 0.f ? ag / b.w : 0.f, lb = c.w > 0.f ? ab / c.w : 0.f;
   const float l = 0.2126f * lr + 0.7152f * lg + 0.0722f * lb;

@@ -23,7 +23,6 @@ hipError_t launch_trace(hipStream_t s, const WaveBuffers& B, int depth, int what
                         int lds_depth, bool count, bool prims);
 hipError_t launch_shade(hipStream_t s, const WaveBuffers& B, int qi, int depth, int grid);
 hipError_t launch_accumulate(hipStream_t s, const WaveBuffers& B, int max_pixels);
-hipError_t launch_advance(hipStream_t s, uint32_t* counters);
 hipError_t launch_average(hipStream_t s, const float4* accum, float* out, int npix, float inv_spp);
 // Ray-batch kernels: rays in the xnh_ray layout (2 float4 per ray:
 // {org.xyz, dir.x} {dir.yz, tmin, tmax}), hits in the xnh_hit layout.

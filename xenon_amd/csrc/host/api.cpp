@@ -8,7 +8,7 @@
 // uploaded once, and each batch runs
 //
 //   raygen -> camera -> shade(0) -> [trace(d) -> shade(d)] 0 < d < max depth -> trace(last shadow rays)
-//          -> accumulate -> advance
+//          -> accumulate
 //
 // with no host read between kernels: every work count and the batch index
 // live in device memory, so the sequence is captured once as a hipGraph and
@@ -677,8 +677,9 @@ int alloc_waves(xnh_ctx* c) {
   if (rc == XNH_OK) rc = dev_alloc(c, c->wave_allocs, &B.sh0, 2 * qcap);
   if (rc == XNH_OK) rc = dev_alloc(c, c->wave_allocs, &B.sh1, 2 * qcap);
   if (rc == XNH_OK) rc = dev_alloc(c, c->wave_allocs, &B.sh_c, 2 * qcap);
-  if (rc == XNH_OK) rc = dev_alloc(c, c->wave_allocs, &B.l_term, cap);
-  if (rc == XNH_OK) rc = dev_alloc(c, c->wave_allocs, &B.l_nee, 2 * cap);
+  // (a fourth float a slot is spare: the largest batch that fits stays what it was)
+  for (float** l : {&B.l_term, &B.l_area, &B.l_sun})
+    if (rc == XNH_OK) rc = dev_alloc(c, c->wave_allocs, l, 4 * cap);
   // the statistics and right after them the counters, whose first words a
   // render reads back (and clears) with them
   if (rc == XNH_OK) rc = dev_alloc(c, c->wave_allocs, &B.stats, static_cast<size_t>(kNumStat + (kNumCtr + 1) / 2));
@@ -775,7 +776,6 @@ int enqueue_batch(xnh_ctx* c, int depth, size_t* ev) {
     HIP_OR_FAIL(c, mark());
   }
   HIP_OR_FAIL(c, launch_accumulate(s, c->B, cap));
-  HIP_OR_FAIL(c, launch_advance(s, c->B.counters));
   return XNH_OK;
 }
 
