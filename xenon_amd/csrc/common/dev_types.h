@@ -29,11 +29,15 @@
 //   ibox    2 x float4 per instance: the box of its TLAS leaf
 //   inst    4 x float4 per instance: world_to_local columns c0..c3 packed
 //           {c0.xyz, c1.x} {c1.yz, c2.xy} {c2.z, c3.xyz} and
-//           {blas root entry, instance_id, tri_base | flat<<31, light map or -1}
+//           {blas root entry, instance_id, 1 without vertex normals, light map or -1}
 //           (the root's stack entry, see kEntShift; kNoRoot for an empty mesh)
-//   vidx    3 x int per global triangle (global vertex indices)
+//   tsurf   int4 per leaf slot, what shading needs besides: {global indices
+//           of the three vertices, material}, one load that waits for nothing
+//           but the hit. As arrays by triangle (three indices, a material) they
+//           were two requests more, behind the triangle's record: k_shade 42.4
+//           -> 39.8 ms (mesh 1920x1080 at 256 spp). In the triangle's record (64
+//           bytes) they cost the traversal more than they gave shading.
 //   vnrm    float4 per global vertex (xyz normal)
-//   tmat    material id per global triangle
 //   lmap    per instance whose id names area lights: first light index per
 //           mesh triangle, -1 for none
 //   lights  4 x float4 per light: {p0, area} {p1, e.r} {p2, e.g} {n_geo, e.b}
@@ -49,7 +53,6 @@
 namespace xnh {
 
 constexpr int kMaxStack = 128;          // TLAS 64 + BLAS 64, the reference's two stacks
-constexpr uint32_t kFlatBit = 0x80000000u;
 // BLAS stack entries: count << kEntShift | index (see dtrace.h)
 constexpr uint32_t kEntShift = 28;
 constexpr uint32_t kEntIndexMask = (1u << kEntShift) - 1u;
@@ -83,14 +86,13 @@ struct DevScene {
   const float4* bnodes;
   const uint32_t* bigcnt;
   const float4* tris;
+  const int4* tsurf;
   const float4* tnodes;
   const float4* tpairs;
   const float4* ibox;
   const uint32_t* torder;
   const float4* inst;
-  const int32_t* vidx;
   const float4* vnrm;
-  const int32_t* tmat;
   const int32_t* lmap;
   const float4* lights;
   const float4* mats;

@@ -215,7 +215,7 @@ struct InstRec {
   f3 c0, c1, c2, c3;
   uint32_t root;
   int32_t id;
-  uint32_t tri_base;   // with kFlatBit
+  uint32_t flat;       // the mesh has no vertex normals
   int32_t lmap;
 };
 __device__ __forceinline__ InstRec load_inst(const float4* inst, int i) {
@@ -227,7 +227,7 @@ __device__ __forceinline__ InstRec load_inst(const float4* inst, int i) {
   r.c3 = f3{c.y, c.z, c.w};
   r.root = __float_as_uint(m.x);
   r.id = __float_as_int(m.y);
-  r.tri_base = __float_as_uint(m.z);
+  r.flat = __float_as_uint(m.z);
   r.lmap = __float_as_int(m.w);
   return r;
 }

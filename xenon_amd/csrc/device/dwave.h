@@ -273,23 +273,23 @@ __device__ __forceinline__ Surface resolve(const DevScene& S, const HitRef& h, f
     float u, v;
     return resolve_prim(S, h, in, o, d, tmin, u, v);
   }
-  const float4 a = S.tris[3 * h.slot], b = S.tris[3 * h.slot + 1], c = S.tris[3 * h.slot + 2];
+  const float4* rec = S.tris + 3 * static_cast<size_t>(h.slot);
+  const float4 a = rec[0], b = rec[1], c = rec[2];
+  const int4 ts = S.tsurf[h.slot];
   const f3 e1{a.w, b.x, b.y}, e2{b.z, b.w, c.x};
   Surface s;
   s.tri = __float_as_uint(c.y);
-  const uint32_t gtri = (in.tri_base & ~kFlatBit) + s.tri;
   const f3 gl = normalize(cross(e1, e2));
   f3 nl = gl;
-  if (!(in.tri_base & kFlatBit)) {
-    const int i0 = S.vidx[3 * gtri], i1 = S.vidx[3 * gtri + 1], i2 = S.vidx[3 * gtri + 2];
-    const f3 n0 = xyz(S.vnrm[i0]), n1 = xyz(S.vnrm[i1]), n2 = xyz(S.vnrm[i2]);
+  if (!in.flat) {
+    const f3 n0 = xyz(S.vnrm[ts.x]), n1 = xyz(S.vnrm[ts.y]), n2 = xyz(S.vnrm[ts.z]);
     nl = normalize(n0 * (1.f - h.u - h.v) + n1 * h.u + n2 * h.v);
   }
   s.pos = o + h.t * d;
   s.n = normal_out(in, nl);
   s.gn = normal_out(in, gl);
   s.front = dot(s.gn, d) < 0.f;
-  s.mat = S.tmat[gtri];
+  s.mat = ts.w;
   s.inst_id = in.id;
   s.lmap = in.lmap;
   return s;
@@ -311,13 +311,15 @@ __device__ __forceinline__ GeoSurface resolve_geo(const DevScene& S, const HitRe
     const Surface f = resolve_prim(S, h, in, o, d, tmin, u, v);
     return GeoSurface{f.pos, f.gn, f.mat, f.tri, -1};
   }
-  const float4 a = S.tris[3 * h.slot], b = S.tris[3 * h.slot + 1], c = S.tris[3 * h.slot + 2];
+  const float4* rec = S.tris + 3 * static_cast<size_t>(h.slot);
+  const float4 a = rec[0], b = rec[1], c = rec[2];
+  const int4 ts = S.tsurf[h.slot];
   const f3 e1{a.w, b.x, b.y}, e2{b.z, b.w, c.x};
   GeoSurface s;
   s.tri = __float_as_uint(c.y);
   s.pos = o + h.t * d;
   s.gn = normal_out(in, normalize(cross(e1, e2)));
-  s.mat = S.tmat[(in.tri_base & ~kFlatBit) + s.tri];
+  s.mat = ts.w;
   s.lmap = in.lmap;
   return s;
 }

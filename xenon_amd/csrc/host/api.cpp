@@ -312,7 +312,7 @@ int flatten_upload(xnh_ctx* c, const xnh_flat_scene* fs, xnh_gpu_scene* g) {
       fs->num_dir_lights < 0 || fs->num_tlas_nodes < 0)
     return fail(c, XNH_E_INVALID, "negative count in flat scene");
   const int nm = fs->num_meshes;
-  std::vector<uint32_t> node_base(nm), slot_base(nm), tri_base(nm), vert_base(nm);
+  std::vector<uint32_t> node_base(nm), slot_base(nm), vert_base(nm);
   size_t nn = 0, ns = 0, nv = 0;
   for (int m = 0; m < nm; ++m) {
     const xnh_mesh& me = fs->meshes[m];
@@ -322,7 +322,6 @@ int flatten_upload(xnh_ctx* c, const xnh_flat_scene* fs, xnh_gpu_scene* g) {
     if ((nn & 1u) == 0) ++nn;   // odd root: child pairs on 64-byte boundaries
     node_base[m] = static_cast<uint32_t>(nn);
     slot_base[m] = static_cast<uint32_t>(ns);
-    tri_base[m] = static_cast<uint32_t>(ns);
     vert_base[m] = static_cast<uint32_t>(nv);
     nn += static_cast<size_t>(me.num_nodes);
     ns += static_cast<size_t>(me.num_triangles);
@@ -358,8 +357,8 @@ int flatten_upload(xnh_ctx* c, const xnh_flat_scene* fs, xnh_gpu_scene* g) {
     pnodes[2 * j + 1] = f4(n.hi[1], n.hi[2], bits(n.child), bits(n.count));
   }
   std::vector<float4> bnodes(2 * nn), tris(3 * ns), vnrm(nv);
+  std::vector<int4> tsurf(ns);
   std::vector<uint32_t> bigcnt(std::max<size_t>(ns, 1), 0u);   // triangles of a large leaf, at its first slot
-  std::vector<int32_t> vidx(3 * ns), tmat(ns);
   std::vector<bool> flat(nm, false);
   for (int m = 0; m < nm; ++m) {
     const xnh_mesh& me = fs->meshes[m];
@@ -397,12 +396,12 @@ int flatten_upload(xnh_ctx* c, const xnh_flat_scene* fs, xnh_gpu_scene* g) {
       tris[3 * g] = f4(v0[0], v0[1], v0[2], e1[0]);
       tris[3 * g + 1] = f4(e1[1], e1[2], e2[0], e2[1]);
       tris[3 * g + 2] = f4(e2[2], bits(t), 0.f, 0.f);
+      const int vb = static_cast<int32_t>(vert_base[m]);
+      tsurf[g] = make_int4(iv[0] + vb, iv[1] + vb, iv[2] + vb, me.mat_ids[t]);
     }
     for (int t = 0; t < me.num_triangles; ++t) {
-      for (int k = 0; k < 3; ++k) vidx[3 * (tri_base[m] + t) + k] = me.indices[3 * t + k] + static_cast<int32_t>(vert_base[m]);
       const int mid = me.mat_ids[t];
       if (mid < 0 || mid >= fs->num_materials) return fail(c, XNH_E_INVALID, "material id out of range");
-      tmat[tri_base[m] + t] = mid;
     }
     flat[m] = !(me.nx && me.ny && me.nz);
     for (int v = 0; v < me.num_vertices; ++v)
@@ -525,7 +524,7 @@ int flatten_upload(xnh_ctx* c, const xnh_flat_scene* fs, xnh_gpu_scene* g) {
     inst[4 * i] = f4(w[0], w[1], w[2], w[3]);
     inst[4 * i + 1] = f4(w[4], w[5], w[6], w[7]);
     inst[4 * i + 2] = f4(w[8], w[9], w[10], w[11]);
-    inst[4 * i + 3] = f4(bits(root), ibits(in.instance_id), bits(tri_base[in.mesh] | (flat[in.mesh] ? kFlatBit : 0u)),
+    inst[4 * i + 3] = f4(bits(root), ibits(in.instance_id), bits(flat[in.mesh] ? 1u : 0u),
                          ibits(lm));
   }
   // lights: corners in the coordinates of mesh `mesh_id` (cpu_tiled.cpp:93-106)
@@ -587,18 +586,18 @@ int flatten_upload(xnh_ctx* c, const xnh_flat_scene* fs, xnh_gpu_scene* g) {
   DevScene S{};
   float4 *p_bn, *p_tr, *p_tn, *p_tp, *p_ib, *p_in, *p_vn, *p_li, *p_ma, *p_su, *p_pr = nullptr, *p_pn = nullptr;
   uint32_t *p_to, *p_po = nullptr, *p_bc, *p_ik;
-  int32_t *p_vi, *p_tm, *p_lm;
+  int32_t* p_lm;
+  int4* p_ts;
   int rc = dev_upload(c, g->allocs, &p_bn, bnodes);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_bc, bigcnt);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_tr, tris);
+  if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_ts, tsurf);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_tn, tnodes);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_tp, tpairs);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_ib, ibox);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_to, torder);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_in, inst);
-  if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_vi, vidx);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_vn, vnrm);
-  if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_tm, tmat);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_lm, lmap);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_ik, ikind);
   if (rc == XNH_OK) rc = dev_upload(c, g->allocs, &p_li, lights);
@@ -614,15 +613,14 @@ int flatten_upload(xnh_ctx* c, const xnh_flat_scene* fs, xnh_gpu_scene* g) {
   S.bnodes = p_bn;
   S.bigcnt = p_bc;
   S.tris = p_tr;
+  S.tsurf = p_ts;
   S.tnodes = p_tn;
   S.tpairs = p_tp;
   S.ibox = p_ib;
   S.troot = ntn > 0 ? tlas_link(0) : 0u;
   S.torder = p_to;
   S.inst = p_in;
-  S.vidx = p_vi;
   S.vnrm = p_vn;
-  S.tmat = p_tm;
   S.lmap = p_lm;
   S.lights = p_li;
   S.mats = p_ma;
@@ -646,8 +644,8 @@ int flatten_upload(xnh_ctx* c, const xnh_flat_scene* fs, xnh_gpu_scene* g) {
   g->bytes = 0;
   for (const auto* v : {&bnodes, &tris, &tnodes, &tpairs, &ibox, &inst, &vnrm, &lights, &mats, &suns, &prims, &pnodes})
     g->bytes += v->size() * 16;
-  g->bytes += (torder.size() + vidx.size() + tmat.size() + lmap.size() + porder.size() + bigcnt.size() +
-               ikind.size()) * 4;
+  g->bytes += tsurf.size() * 16;
+  g->bytes += (torder.size() + lmap.size() + porder.size() + bigcnt.size() + ikind.size()) * 4;
   return XNH_OK;
 }
 
