@@ -103,6 +103,7 @@ struct DevScene {
   const uint32_t* ikind;    // per instance: the shading class of all its surfaces (kShade*), for sorting
   int32_t num_pnodes;
   int32_t num_tnodes;
+  int32_t tlas_plain;   // 16 or more TLAS nodes, all boxes finite with lo <= hi: min and max order their slab distances
   int32_t num_lights;
   int32_t num_suns;
   uint32_t troot;           // the TLAS root's link

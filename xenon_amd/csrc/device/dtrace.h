@@ -468,8 +468,9 @@ __device__ __forceinline__ bool ent_leaf(uint32_t e) { return e - (1u << kEntShi
 struct SceneTables {
   const float4* bnodes;
   const float4* tris;
-  __device__ __forceinline__ explicit SceneTables(const DevScene& S) : bnodes(S.bnodes), tris(S.tris) {}
-  __device__ __forceinline__ SceneTables() : bnodes(nullptr), tris(nullptr) {}
+  bool plain;   // tlas_plain
+  __device__ __forceinline__ explicit SceneTables(const DevScene& S) : bnodes(S.bnodes), tris(S.tris), plain(S.tlas_plain != 0) {}
+  __device__ __forceinline__ SceneTables() : bnodes(nullptr), tris(nullptr), plain(false) {}
 };
 
 // kPrims: the scene may hold analytic primitives (a variant, because their
@@ -593,7 +594,18 @@ struct Walker {
 
   // Sign-selected slab test of a TLAS box against the world ray
   // (geometry/aabb.h:59-71): near and far planes by direction sign.
-  __device__ __forceinline__ bool tlas_box(float lx, float ly, float lz, float hx, float hy, float hz) const {
+  // `plain` (a wfast ray, a box with lo <= hi): the smaller distance of an axis
+  // is the near one (rounding is monotone), so the hardware's min and max
+  // give the same answer in fewer instructions.
+  __device__ __forceinline__ bool tlas_box(bool plain, float lx, float ly, float lz, float hx, float hy, float hz) const {
+    if (!kCount && plain) {
+      asm volatile("");   // (two branches, not one computation with selects)
+      const float x0 = (lx - o.x) * inv.x, x1 = (hx - o.x) * inv.x;
+      const float y0 = (ly - o.y) * inv.y, y1 = (hy - o.y) * inv.y;
+      const float z0 = (lz - o.z) * inv.z, z1 = (hz - o.z) * inv.z;
+      return fmaxf(fmaxf(fmaxf(fminf(x0, x1), fminf(y0, y1)), fminf(z0, z1)), tmin) <=
+             fminf(fminf(fminf(fmaxf(x0, x1), fmaxf(y0, y1)), fmaxf(z0, z1)), tbest);
+    }
     const bool sx = d.x < 0.f, sy = d.y < 0.f, sz = d.z < 0.f;
     const float txn = ((sx ? hx : lx) - o.x) * inv.x, txf = ((sx ? lx : hx) - o.x) * inv.x;
     const float tyn = ((sy ? hy : ly) - o.y) * inv.y, tyf = ((sy ? ly : hy) - o.y) * inv.y;
@@ -608,12 +620,12 @@ struct Walker {
 
   // An instance: its BLAS walk starts (or the primitives are walked to the
   // end), if its leaf's box is hit at this time (kInstTest).
-  __device__ __forceinline__ void instance_step(const DevScene& S, TravStack& st, TravCount& c) {
+  __device__ __forceinline__ void instance_step(const DevScene& S, TravStack& st, TravCount& c, bool plain) {
     const uint32_t te = st.pop();
     const int ii = static_cast<int>(te & kInstIndexMask);
     const InstRec in = load_inst(S.inst, ii);
     const float4 ba = gld4(S.ibox, 2 * static_cast<size_t>(ii)), bb = gld4(S.ibox, 2 * static_cast<size_t>(ii) + 1);
-    if (te >= kInstTest && !tlas_box(ba.x, ba.y, ba.z, ba.w, bb.x, bb.y)) return;
+    if (te >= kInstTest && !tlas_box(plain, ba.x, ba.y, ba.z, ba.w, bb.x, bb.y)) return;
     if (kCount) ++c.inst_visits;
     lo = in.c0 * o.x + in.c1 * o.y + in.c2 * o.z + in.c3;
     ld = in.c0 * d.x + in.c1 * d.y + in.c2 * d.z;
@@ -649,18 +661,19 @@ struct Walker {
   //     a zero or non-finite component test the node first (wfast false).
   // A step per node hit instead of one per node tested (both children of
   // every node hit), and instances entered in steps of their own: 4096
-  // instances 1920x1080x64 347 -> 219 ms a pass.
-  __device__ __forceinline__ void node_step(const DevScene& S, TravStack& st, TravCount& c) {
+  // instances 1920x1080x64 347 -> 219 ms a pass; with tlas_box's plain form
+  // 211 -> 199.
+  __device__ __forceinline__ void node_step(const DevScene& S, TravStack& st, TravCount& c, bool plain) {
     const uint32_t ni = st.pop();
-    if (!wfast) {
+    if ((kCount || !plain) && !wfast) {
       const float4 na = gld4(S.tnodes, 3 * static_cast<size_t>(ni)), nb = gld4(S.tnodes, 3 * static_cast<size_t>(ni) + 1);
-      if (!tlas_box(na.x, na.y, na.z, na.w, nb.x, nb.y)) return;
+      if (!tlas_box(false, na.x, na.y, na.z, na.w, nb.x, nb.y)) return;
     }
     const float4* rec = S.tpairs + 4 * static_cast<size_t>(ni);
     const float4 a = gld4(rec, 0), b = gld4(rec, 1), q = gld4(rec, 2), k = gld4(rec, 3);
     const uint32_t wl = __float_as_uint(k.z), right = __float_as_uint(k.w);
     const uint32_t ax = (wl >> kTlasAxisShift) & 3u;
-    const bool hl = tlas_box(a.x, a.y, a.z, a.w, b.x, b.y);
+    const bool hl = tlas_box(plain, a.x, a.y, a.z, a.w, b.x, b.y);
     if (ax == kTlasList) {   // a leaf of several instances (or one named twice): walked first to last
       if (hl)
         for (uint32_t n = __float_as_uint(b.z); n-- > 0u;) st.push(kInstTag | gld1(S.torder, right + n));
@@ -670,7 +683,7 @@ struct Walker {
         c.node_tests += 2;
       }
       const uint32_t left = wl & ~(3u << kTlasAxisShift);
-      const bool hr = tlas_box(b.z, b.w, q.x, q.y, q.z, q.w);
+      const bool hr = tlas_box(plain, b.z, b.w, q.x, q.y, q.z, q.w);
       const float oa = comp(o, static_cast<int>(ax)), ia = comp(inv, static_cast<int>(ax));
       const float tl = (k.x - oa) * ia;
       const float tr = (k.y - oa) * ia;
@@ -792,6 +805,26 @@ __device__ __forceinline__ void interior_run(Walker<kAny, kCount, kPrims>& w, co
   } while (ni != 0 && 2 * ni >= nb);
 }
 
+// TLAS steps of the nt lanes that need one, each in this run until it enters a
+// BLAS or ends; each turn takes the kind, node or instance, that more of its
+// lanes need.
+template <bool kAny, bool kCount, bool kPrims>
+__device__ __forceinline__ void tlas_run(Walker<kAny, kCount, kPrims>& w, const DevScene& S, TravStack& st,
+                                         TravCount& c, int nt, bool plain) {
+  bool part = w.e == kEntEnd && !st.empty();
+  int n0 = nt;
+  do {
+    const bool instance = part && Walker<kAny, kCount, kPrims>::is_instance(st.tos);
+    if (2 * lanes_of(instance) <= n0) {
+      if (part && !instance) w.node_step(S, st, c, plain);
+    } else {
+      if (instance) w.instance_step(S, st, c, plain);
+    }
+    part = part && w.e == kEntEnd && !st.empty();
+    n0 = lanes_of(part);
+  } while (n0 != 0 && 2 * n0 >= nt);
+}
+
 // One scheduled run of a wave's walks. Every lane holding a ray names the
 // kind of step it needs next (TLAS entry, leaf, or interior node pair);
 // the kind most lanes need runs, on those lanes only, while the others wait:
@@ -810,10 +843,11 @@ __device__ __forceinline__ void interior_run(Walker<kAny, kCount, kPrims>& w, co
 // 1.3M-triangle mesh 1920x1080x256 240.7 -> 236.5 ms). With primitives, whose
 // long instance steps leave lanes finished for longer, one run at a time
 // (801x449x33 6.38 against 6.50 ms). Every lane of the wave must reach it.
+// `plain`: the scene is tlas_plain and every lane with a ray wfast.
 constexpr int kTurns = 64;
 template <bool kAny, bool kCount, bool kPrims>
 __device__ __forceinline__ void wave_step(Walker<kAny, kCount, kPrims>& w, const DevScene& S, const SceneTables& T,
-                                          TravStack& st, TravCount& c, int rest) {
+                                          TravStack& st, TravCount& c, int rest, bool plain) {
   for (int turn = 0; turn < (kPrims ? 1 : kTurns); ++turn) {
     const int nt = lanes_of(w.e == kEntEnd && !st.empty());
     int ni = lanes_of(ent_interior(w.e)), nl = lanes_of(w.e < kEntEnd) - ni;
@@ -839,20 +873,7 @@ __device__ __forceinline__ void wave_step(Walker<kAny, kCount, kPrims>& w, const
         nl = lanes_of(w.e < kEntEnd) - ni;
       } while (nl != 0 && nl >= ni);
     } else {
-      // in this run until it enters a BLAS or ends; each turn takes the kind,
-      // node or instance, that more of its lanes need
-      bool part = w.e == kEntEnd && !st.empty();
-      int n0;
-      do {
-        const bool instance = Walker<kAny, kCount, kPrims>::is_instance(st.tos);
-        if (lanes_of(part && !instance) >= lanes_of(part && instance)) {
-          if (part && !instance) w.node_step(S, st, c);
-        } else {
-          if (part && instance) w.instance_step(S, st, c);
-        }
-        part = part && w.e == kEntEnd && !st.empty();
-        n0 = lanes_of(part);
-      } while (n0 != 0 && 2 * n0 >= nt);
+      tlas_run(w, S, st, c, nt, plain);
     }
   }
 }
@@ -866,12 +887,13 @@ __device__ __forceinline__ bool walk_scene(const DevScene& S, f3 o, f3 d, float 
   const SceneTables T(S);
   w.begin(S, o, d, tmin, tmax, st, c);
   if (!valid) w.stop(st);
+  const bool plain = T.plain && ballot(!w.wfast) == 0ull;
   for (uint32_t guard = 0; ballot(!w.finished(st)) != 0ull; ++guard) {
     if (guard >= kWaveStepLimit) {
       st.overflow = true;
       break;
     }
-    wave_step(w, S, T, st, c, 64);
+    wave_step(w, S, T, st, c, 64, plain);
   }
   hit = w.hit;
   hit.t = w.found() ? w.tbest : 0.f;

@@ -189,7 +189,7 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const View& v,
   int pci = 0, job = 0;
   SceneTables tables;
   const uint32_t part = 64u >> un.split, pmask = (1u << un.split) - 1u;
-  bool stuck = false;
+  bool stuck = false, plain = false;
   for (uint32_t guard = 0;; ++guard) {
     if (guard >= kWaveStepLimit) {
       stuck = true;
@@ -284,6 +284,7 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const View& v,
           w.begin(S, o, d, tmin, tmax, st, c);
         }
         pnext = min(pend, pnext + static_cast<uint32_t>(__popcll(idle)));
+        plain = tables.plain && ballot(my != kIdle && !w.wfast) == 0ull;
       }
     }
     // (a part of a segment's last unit may hold no entry: a wave without rays
@@ -291,7 +292,7 @@ __device__ __forceinline__ void trace_queue(const WaveBuffers& B, const View& v,
     if ((un.cur >= hi || (un.exhausted && un.cur >= un.end)) && __ballot(my != kIdle) == 0ull) break;
     if (kCount && lane == 0) ++c.round_iters;
     if (kCount && my != kIdle) ++c.round_lanes;
-    wave_step(w, job_scene(B.jobs, job), tables, st, c, kRefill);
+    wave_step(w, job_scene(B.jobs, job), tables, st, c, kRefill, plain);
     if (my != kIdle && w.finished(st)) {
       overflow |= st.overflow;
       finish(my, w);

@@ -631,6 +631,15 @@ int flatten_upload(xnh_ctx* c, const xnh_flat_scene* fs, xnh_gpu_scene* g) {
   S.ikind = p_ik;
   S.num_pnodes = np > 0 ? npn : 0;
   S.num_tnodes = ntn;
+  // (below 16 nodes the plain form has nothing to gain: a 1920x1080x1 frame of
+  // two instances took 5.35 ms with it, 5.29 without; 4096 instances 199 ms
+  // with it, 211 without)
+  S.tlas_plain = ntn >= 16 ? 1 : 0;
+  for (int j = 0; j < ntn; ++j)
+    for (int k = 0; k < 3; ++k) {
+      const xnh_bvh_node& n = fs->tlas_nodes[j];
+      if (!(std::isfinite(n.lo[k]) && std::isfinite(n.hi[k]) && n.lo[k] <= n.hi[k])) S.tlas_plain = 0;
+    }
   S.num_lights = fs->num_lights;
   S.num_suns = fs->num_dir_lights;
   for (int k = 0; k < 3; ++k) {
