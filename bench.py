@@ -485,7 +485,7 @@ def main():
     roofline = {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": read_traffic() if args.config == 1 else None,
-                "kernel": "k_closest (closest-hit traversal)",
+                "kernel": "k_camera, k_trace (closest-hit traversal)",
                 "bytes_per_launch": round(cbytes / launches), "avg_launch_ms": round(tot["closest_ms"] / launches, 4)}
     sbytes = algorithmic_bytes(tot, "shadow")
     # shading: path state (64 B; not for camera paths, which are rebuilt
@@ -515,7 +515,7 @@ def main():
                       "shadow": round(tot["shadow_ms"], 2), "device_total": round(tot["render_ms"], 2)},
         "shadow_roofline": {"achieved": round(sbytes / (tot["shadow_ms"] / 1e3) / 1e9, 2) if tot["shadow_ms"] else None,
                             "frac": round(sbytes / (tot["shadow_ms"] / 1e3) / 1e9 / HBM_PEAK_GBS, 4)
-                            if tot["shadow_ms"] else None, "unit": "GB/s", "kernel": "k_shadow (any-hit traversal)"},
+                            if tot["shadow_ms"] else None, "unit": "GB/s", "kernel": "k_trace (any-hit traversal)"},
         "shade_roofline": {"achieved": round(hbytes / (tot["shade_ms"] / 1e3) / 1e9, 2) if tot["shade_ms"] else None,
                            "frac": round(hbytes / (tot["shade_ms"] / 1e3) / 1e9 / HBM_PEAK_GBS, 4)
                            if tot["shade_ms"] else None, "unit": "GB/s", "kernel": "k_shade (shading)"},

@@ -7,7 +7,7 @@
 // call arguments right to left, so the SECOND draw becomes u1. The kernels
 // draw explicitly in that order.
 //
-// Transcendentals (cos, sin, pow, exp) are the device's and may differ from
+// Transcendentals (cos, sin, pow) are the device's and may differ from
 // glibc by an ulp; everything else rounds as the host does.
 #pragma once
 #include "../common/dev_types.h"

@@ -559,7 +559,7 @@ int flatten_upload(xnh_ctx* c, const xnh_flat_scene* fs, xnh_gpu_scene* g) {
     // the material-only parts of the multiple-scattering compensation
     // (bsdf.h:212-249), in the device's float operation order; the two
     // transcendentals evaluated in double and rounded once, as the device
-    // does for its own (device/dmath.h cos_r etc.)
+    // does for its own (device/dmath.h sincos_r, pow_r)
     const float a = m.alpha;
     const float k1 = 5.0f * static_cast<float>(std::exp(static_cast<double>(-2.69f * a)));
     const float k2 = 1.0f + 22.7f * static_cast<float>(std::pow(static_cast<double>(a), 1.5));
